@@ -557,6 +557,10 @@ typedef struct {
   int c_bf16;           /* 1: c is written as bf16 (rounded once from the fp32 result) */
 } e2v2_gemm_args;
 int e2v2_gemm_s3(const e2v2_gemm_args* args, hipStream_t s);
+/* e2v2_gemm_s3 with every row summed in the same order whatever the number of rows m (e2v2_gemm_s3 takes other
+ * tiles, which split the sum over k, for matrices of few rows): for operands whose row count is a capacity, so
+ * that padding rows change no value. */
+int e2v2_gemm_s3_padded(const e2v2_gemm_args* args, hipStream_t s);
 /* Up to four independent GEMMs (each as e2v2_gemm_s3, with its own shapes, operands and packed weight) in one
  * launch: the groups' tiles share the GPU instead of running one small launch after another; groups are
  * dispatched in the order given (put the longest k first).  Used for the per-degree GEMMs of forward_linear +

@@ -43,6 +43,7 @@
 // column c in slot g ^ ((c / 8) & 1): the rows (columns) that 8 or 16 consecutive
 // lanes read land in distinct bank groups.
 #include "gemm_core.h"
+#include "gemm_ks.h"
 
 namespace e2v2 {
 namespace {
@@ -192,6 +193,135 @@ __device__ __forceinline__ void gemm_tile_r(const e2v2_gemm_args& G, int tile) {
   gemm_store(G, bi, nt, row0, wv, lane, acc);
 }
 
+// Raw A registers of one stage and row tile of the K-split GEMM: the operand, and for a gated call the logits.
+template <bool kAB, bool kGate>
+struct KsRaw {
+  floatx4 x0, x1;
+};
+template <>
+struct KsRaw<true, false> {
+  bf16x8 b;
+};
+template <>
+struct KsRaw<false, true> {
+  floatx4 x0, x1, m0, m1;
+};
+
+// A tile is one row tile of 32 by two column subtiles: 64 rows (two row tiles) were 20-30% slower below 500
+// rows, where the tiles are too few, and within 5% of it above.
+constexpr int kKsR = 1, kKsJ = 2, kKsM = 32 * kKsR, kKsN = 32 * kKsJ;
+__host__ __device__ __forceinline__ int ks_tiles(const e2v2_gemm_args& G) {
+  return G.batch * ((G.m + kKsM - 1) / kKsM) * (G.n / kKsN);
+}
+
+// One 32 x 64 tile of the K-split form (gemm_ks.h); the operands, bounds and epilogue of gemm_tile.
+template <int kP, bool kAB, bool kGate, int kD>
+__device__ __forceinline__ void gemm_tile_ks(const e2v2_gemm_args& G, int tile, float* red, const GateOp& gt) {
+  static_assert(!(kAB && kGate), "the gated operand is fp32");
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5;
+  const int n_mt = (G.m + kKsM - 1) / kKsM, n_ct = G.n / kKsN, n_nt = G.n / kGN;
+  const int ct = tile % n_ct, mt = (tile / n_ct) % n_mt, bi = tile / (n_ct * n_mt);
+  const int row0 = mt * kKsM, nks = G.k / kGK;
+  const int nt = ct / (kGN / kKsN), q0 = (ct % (kGN / kKsN)) * kKsJ;
+  const bool g0 = kGate && bi == 0;                      // batch 0 of a gated call: silu of the logits
+  const int lda = g0 ? (int)gt.ld : (int)G.lda;
+  __amdgpu_buffer_rsrc_t ar;
+  if constexpr (kAB) ar = rows_rsrc_bf(static_cast<const __bf16*>(G.a) + (int64_t)bi * G.a_bs, row0, G.m, lda);
+  else ar = rows_rsrc(g0 ? gt.s : static_cast<const float*>(G.a) + (int64_t)bi * G.a_bs, row0, G.m, lda);
+  const __amdgpu_buffer_rsrc_t sr = kGate ? rows_rsrc(gt.s, row0, G.m, (int)gt.ld) : ar;
+  const __amdgpu_buffer_rsrc_t br = b_rsrc<kP>(G.b, G.widx[bi], n_nt, nt, nks);
+  uint32_t aoff[kKsR], soff[kKsR], boff[kKsJ];
+#pragma unroll
+  for (int i = 0; i < kKsR; ++i) {
+    const int r = 32 * i + (lane & 31);
+    aoff[i] = (uint32_t)(r * lda + 8 * h) * (kAB ? 2u : 4u);
+    soff[i] = kGate ? (uint32_t)(r * (int)gt.ld + G.k * G.widx[bi] + 8 * h) * 4u : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < kKsJ; ++j) boff[j] = ks_b_offset(q0 + j, lane);
+  floatx16 acc[kKsR][kKsJ];
+  ks_zero(acc);
+  using Raw = KsRaw<kAB, kGate>;
+  ks_loop<kP, kKsR, kKsJ, kD, Raw>(
+      br, boff, wv * nks / kKsW, (wv + 1) * nks / kKsW,
+      [&](int ks, int i, Raw& x) {
+        if constexpr (kAB) {
+          x.b = ks_load_b(ar, aoff[i] + (uint32_t)ks * (kGK * 2u));
+        } else {
+          const uint32_t o = (uint32_t)ks * (kGK * 4u);
+          x.x0 = ks_load4(ar, aoff[i] + o);
+          x.x1 = ks_load4(ar, aoff[i] + o + 16u);
+          if constexpr (kGate) {
+            if (!g0) {
+              x.m0 = ks_load4(sr, soff[i] + o);
+              x.m1 = ks_load4(sr, soff[i] + o + 16u);
+            }
+          }
+        }
+      },
+      [&](int, int, const Raw& x, bf16x8 (&a)[kP]) {
+        if constexpr (kAB) {
+          a[0] = x.b;
+        } else {
+          floatx4 x0 = x.x0, x1 = x.x1;
+          if constexpr (kGate) {
+            if (g0) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                x0[e] = silu(x0[e]) * gt.k1;
+                x1[e] = silu(x1[e]) * gt.k1;
+              }
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                x0[e] = sigmoidf_(x.m0[e]) * gt.k2 * x0[e];
+                x1[e] = sigmoidf_(x.m1[e]) * gt.k2 * x1[e];
+              }
+            }
+          }
+          split_pieces<kP>(x0, x1, a);
+        }
+      },
+      acc);
+  constexpr int kN = 16 * kKsR * kKsJ;
+  float part[kN], sum[kN / kKsW];
+  ks_flat(acc, part);
+  ks_reduce<kN, kKsW>(red, part, wv, lane, [](int w, int i) { return w * (kN / kKsW) + i; }, sum);
+  const bool with_bias = G.bias && bi < G.bias_batches;
+  float* cb = static_cast<float*>(G.c) + (G.c_bf16 ? 0 : (int64_t)bi * G.c_bs);
+  __bf16* cbh = static_cast<__bf16*>(G.c) + (G.c_bf16 ? (int64_t)bi * G.c_bs : 0);
+  const float* rb = G.r ? G.r + (int64_t)bi * G.r_bs : nullptr;
+#pragma unroll
+  for (int i = 0; i < kN / kKsW; ++i) {
+    const int q = wv * (kN / kKsW) + i, r = q % 16, j = (q / 16) % kKsJ, it = q / (16 * kKsJ);
+    const int col = ct * kKsN + 32 * j + (lane & 31), row = row0 + 32 * it + acc_row(r, lane);
+    if (row < G.m) {
+      float v = sum[i];
+      if (with_bias) v += G.bias[(int64_t)bi * G.bias_bs + col];
+      if (rb) v += rb[(size_t)row * G.ldr + col];
+      if (G.c_bf16)
+        cbh[(size_t)row * G.ldc + col] = (__bf16)v;
+      else
+        cb[(size_t)row * G.ldc + col] = v;
+    }
+  }
+}
+
+template <int kP, bool kAB, int kD>
+__global__ __launch_bounds__(kKsThreads, 2) void k_gemm_ks(e2v2_gemm_args G) {
+  __shared__ float red[kKsW * 16 * kKsR * kKsJ * 64];
+  const int n_tiles = ks_tiles(G), tile = xcd_row(blockIdx.x, n_tiles);
+  if (tile >= n_tiles) return;
+  gemm_tile_ks<kP, kAB, false, kD>(G, tile, red, GateOp{});
+}
+template <int kP, int kD>
+__global__ __launch_bounds__(kKsThreads, 2) void k_gemm_ks_gate(e2v2_gemm_args G, GateOp gt) {
+  __shared__ float red[kKsW * 16 * kKsR * kKsJ * 64];
+  const int n_tiles = ks_tiles(G), tile = xcd_row(blockIdx.x, n_tiles);
+  if (tile >= n_tiles) return;
+  gemm_tile_ks<kP, false, true, kD>(G, tile, red, gt);
+}
+
 // fp32 A, three pieces
 __global__ __launch_bounds__(kGT, 4) void k_gemm_s3(e2v2_gemm_args G) {
   const int n_tiles = gemm_tiles(G);
@@ -255,6 +385,21 @@ __global__ __launch_bounds__(kGT, 3) void k_gemm_s3_grp_p1(GemmGroups P) {
       const int n_tiles = gemm_tiles(P.g[gi]);
       const int tile = xcd_row(b - P.block0[gi], n_tiles);
       if (tile < n_tiles) gemm_tile<1, kAB, false>(P.g[gi], tile, lds, GateOp{});
+      return;
+    }
+  }
+}
+
+template <int kP, bool kAB, int kD>
+__global__ __launch_bounds__(kKsThreads, 2) void k_gemm_ks_grp(GemmGroups P) {
+  __shared__ float red[kKsW * 16 * kKsR * kKsJ * 64];
+  const int b = blockIdx.x;
+#pragma unroll
+  for (int gi = 0; gi < kGGroups; ++gi) {
+    if (gi < P.n && b >= P.block0[gi] && b < P.block0[gi + 1]) {
+      const int n_tiles = ks_tiles(P.g[gi]);
+      const int tile = xcd_row(b - P.block0[gi], n_tiles);
+      if (tile < n_tiles) gemm_tile_ks<kP, kAB, false, kD>(P.g[gi], tile, red, GateOp{});
       return;
     }
   }
@@ -347,6 +492,85 @@ __global__ __launch_bounds__(kGT, 2) void k_qk_s3_fwd(const float* __restrict__ 
       const int row = row0 + wv * 32 + acc_row(r, lane);
       if (row < n) out[(size_t)row * 3 * hid] = s[j][r];
     }
+  }
+}
+
+// The same for few rows, K split over the wavefronts (gemm_ks.h; c = 256: four stages per wavefront): a
+// workgroup takes 32 rows x 32 pairs (their a- and b-columns) of one degree.  The weight fragments of the
+// wavefront's stages stay in registers over the degree's m-rows, the next m-row's A fragments load while the
+// current one multiplies, and the partial sums of an m-row meet in one of two LDS buffers (one barrier per
+// m-row), where wavefront w finishes rows 8 w .. 8 w + 7 of both column tiles: y, and a b into the pair sums.
+template <int kP, bool kYB>
+__global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_fwd(const float* __restrict__ x, const void* __restrict__ wp,
+                                                             const float* __restrict__ bias, void* __restrict__ y,
+                                                             float* __restrict__ hq, float* __restrict__ hk, int n,
+                                                             int hid) {
+  constexpr int c = 256, nks = c / kGK, kSt = nks / kKsW, kN = 32;
+  __shared__ float red[2][kKsW * kN * 64];
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5;
+  const int n_mt = (n + 31) / 32, n_ps = 2 * hid / 32, tiles = n_mt * n_ps;
+  const int grp = blockIdx.x / xcd_grid(tiles), L = 2 - grp;
+  const int tile = xcd_row(blockIdx.x - grp * xcd_grid(tiles), tiles);
+  if (tile >= tiles) return;
+  const int mt = tile / n_ps, ps = tile % n_ps, row0 = mt * 32, O = 4 * hid;
+  const __amdgpu_buffer_rsrc_t br = b_rsrc<kP>(wp, L, n_ps / 2, ps / 2, nks);
+  const uint32_t boff[2] = {ks_b_offset(ps % 2, lane), ks_b_offset(ps % 2 + 2, lane)};
+  const uint32_t aoff = (uint32_t)((lane & 31) * c + 8 * h + wv * kSt * kGK) * 4u;
+  bf16x8 b[kSt][2][kP];
+#pragma unroll
+  for (int s = 0; s < kSt; ++s)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int p = 0; p < kP; ++p)
+        b[s][j][p] = ks_load_b(br, (uint32_t)(wv * kSt + s) * (b_stage_granules(kP) * 16u) + p * (kGBg * 16u) + boff[j]);
+  floatx4 a[kSt][2];
+  auto load = [&](int m) {
+    const __amdgpu_buffer_rsrc_t ar = rows_rsrc(x + (size_t)m * n * c, row0, n, c);
+#pragma unroll
+    for (int s = 0; s < kSt; ++s) {
+      a[s][0] = ks_load4(ar, aoff + s * (kGK * 4u));
+      a[s][1] = ks_load4(ar, aoff + s * (kGK * 4u) + 16u);
+    }
+  };
+  float sp[4] = {0.f, 0.f, 0.f, 0.f};
+  const int m0 = L * L, m1 = (L + 1) * (L + 1), p0 = 32 * ps + (lane & 31);
+  load(m0);
+  for (int m = m0; m < m1; ++m) {
+    floatx16 acc[1][2];
+    ks_zero(acc);
+    bf16x8 ap[kSt][kP];
+#pragma unroll
+    for (int s = 0; s < kSt; ++s) split_pieces<kP>(a[s][0], a[s][1], ap[s]);
+    if (m + 1 < m1) load(m + 1);
+#pragma unroll
+    for (int s = 0; s < kSt; ++s)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) ks_mfma<kP>(ap[s], b[s][j], acc[0][j]);
+    float part[kN], sum[kN / kKsW];
+    ks_flat(acc, part);
+    // wavefront w finishes registers 4 w .. 4 w + 3 of both column tiles
+    ks_reduce<kN, kKsW>(red[m & 1], part, wv, lane, [](int w, int i) { return 16 * (i / 4) + 4 * w + i % 4; }, sum);
+    float* ym = static_cast<float*>(y) + (kYB ? 0 : (size_t)m * n * O);
+    __bf16* ymb = static_cast<__bf16*>(y) + (kYB ? (size_t)m * n * O : 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int ab = i / 4, row = row0 + acc_row(4 * wv + i % 4, lane);
+      if (m == 0 && bias) sum[i] += bias[128 * (ps / 2) + 64 * ab + 32 * (ps % 2) + (lane & 31)];
+      if (row < n) {
+        const size_t o = (size_t)row * O + pair_pos(p0, ab);
+        if constexpr (kYB) ymb[o] = (__bf16)sum[i];
+        else ym[o] = sum[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sp[i] = fmaf(sum[i], sum[4 + i], sp[i]);
+  }
+  float* out = p0 < hid ? hq + L * hid + p0 : hk + L * hid + (p0 - hid);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = row0 + acc_row(4 * wv + i, lane);
+    if (row < n) out[(size_t)row * 3 * hid] = sp[i];
   }
 }
 
@@ -447,6 +671,92 @@ __global__ __launch_bounds__(kGT, 2) void k_qk_s3_bwd(const void* __restrict__ y
   }
 }
 
+// The same for few rows: a 32 x 64 tile of one m-row, K (the pair columns, then the value projection's) split
+// over the wavefronts (gemm_ks.h).  A lane reads its row's partner values of y and the eight g values itself.
+template <int kP, bool kYB, int kD>
+__global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_bwd(const void* __restrict__ y, const float* __restrict__ ghq,
+                                                          const float* __restrict__ ghk, const void* __restrict__ wp,
+                                                          const float* __restrict__ gv, float* __restrict__ gx, int n,
+                                                          int hid, int c, int cv) {
+  constexpr int kW = kKsW, kN = 16 * kKsJ;
+  __shared__ float red[kW * kN * 64];
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5;
+  const int n_mt = (n + 31) / 32, n_ct = c / (32 * kKsJ), tiles = 9 * n_mt * n_ct;
+  const int tile = xcd_row(blockIdx.x, tiles);
+  if (tile >= tiles) return;
+  const int ct = tile % n_ct, mt = (tile / n_ct) % n_mt, m = tile / (n_ct * n_mt);
+  const int l = m == 0 ? 0 : (m < 4 ? 1 : 2);
+  const int O = 4 * hid, row0 = mt * 32, nk1 = O / kGK, nks_w = nk1 + cv / kGK, r = lane & 31;
+  const __amdgpu_buffer_rsrc_t yr =
+      kYB ? rows_rsrc_bf(static_cast<const __bf16*>(y) + (size_t)m * n * O, row0, n, O)
+          : rows_rsrc(static_cast<const float*>(y) + (size_t)m * n * O, row0, n, O);
+  const __amdgpu_buffer_rsrc_t qr = rows_rsrc(ghq, row0, n, 3 * hid), kr = rows_rsrc(ghk, row0, n, 3 * hid);
+  const __amdgpu_buffer_rsrc_t br = b_rsrc<kP>(wp, l, c / kGN, ct * 32 * kKsJ / kGN, nks_w);
+  const uint32_t yoff = (uint32_t)(r * O + 8 * (1 - h)) * (kYB ? 2u : 4u);      // the partner half of the stage
+  const uint32_t voff = (uint32_t)(r * cv + 8 * h) * 4u, goff = (uint32_t)(r * 3 * hid + l * hid) * 4u;
+  uint32_t boff[kKsJ];
+#pragma unroll
+  for (int j = 0; j < kKsJ; ++j) boff[j] = ks_b_offset((ct * kKsJ + j) % 4, lane);
+  floatx16 acc[1][kKsJ];
+  ks_zero(acc);
+  // pair columns: the first half of the stages are the query's pairs (hid / 8 stages each half), and so is
+  // the first half of the wavefronts
+  struct Raw {
+    floatx4 x0, x1, g0, g1;
+  };
+  const int half = nk1 / 2, own = nk1 / kW, ks0 = wv * own;
+  const __amdgpu_buffer_rsrc_t gr = ks0 < half ? qr : kr;
+  const uint32_t goff2 = goff - (ks0 < half ? 0u : (uint32_t)hid * 4u);
+  ks_loop<kP, 1, kKsJ, kD, Raw>(
+      br, boff, ks0, ks0 + own,
+      [&](int ks, int, Raw& a) {
+        if constexpr (kYB) {
+          a.x0 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 2u));
+        } else {
+          a.x0 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 4u));
+          a.x1 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 4u) + 16u);
+        }
+        a.g0 = ks_load4(gr, goff2 + (uint32_t)ks * 32u);
+        a.g1 = ks_load4(gr, goff2 + (uint32_t)ks * 32u + 16u);
+      },
+      [&](int, int, const Raw& a, bf16x8 (&p)[kP]) {
+        floatx4 x0 = a.x0, x1 = a.x1;
+        if constexpr (kYB) {
+          const bf16x8 yb = __builtin_bit_cast(bf16x8, a.x0);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            x0[u] = (float)yb[u];
+            x1[u] = (float)yb[4 + u];
+          }
+        }
+        split_pieces<kP>(x0 * a.g0, x1 * a.g1, p);
+      },
+      acc);
+  if (gv) {
+    struct RawV {
+      floatx4 x0, x1;
+    };
+    const __amdgpu_buffer_rsrc_t vr = rows_rsrc(gv + (size_t)m * n * cv, row0, n, cv);
+    const int nkv = cv / kGK;
+    ks_loop<kP, 1, kKsJ, kD, RawV>(
+        br, boff, nk1 + wv * nkv / kW, nk1 + (wv + 1) * nkv / kW,
+        [&](int ks, int, RawV& a) {
+          a.x0 = ks_load4(vr, voff + (uint32_t)(ks - nk1) * (kGK * 4u));
+          a.x1 = ks_load4(vr, voff + (uint32_t)(ks - nk1) * (kGK * 4u) + 16u);
+        },
+        [&](int, int, const RawV& a, bf16x8 (&p)[kP]) { split_pieces<kP>(a.x0, a.x1, p); }, acc);
+  }
+  float part[kN], sum[kN / kW];
+  ks_flat(acc, part);
+  ks_reduce<kN, kW>(red, part, wv, lane, [](int w, int i) { return w * (kN / kW) + i; }, sum);
+  float* gm = gx + (size_t)m * n * c;
+#pragma unroll
+  for (int i = 0; i < kN / kW; ++i) {
+    const int q = wv * (kN / kW) + i, row = row0 + acc_row(q % 16, lane);
+    if (row < n) gm[(size_t)row * c + ct * 32 * kKsJ + 32 * (q / 16) + (lane & 31)] = sum[i];
+  }
+}
+
 // Pack: one thread per (weight, column tile, stage, LDS granule): the granule's
 // eight k of its column, split into the three pieces (or rounded to the first alone).
 __global__ __launch_bounds__(256) void k_gemm_pack(const float* __restrict__ w, int64_t ld_n, int64_t ld_k,
@@ -529,15 +839,45 @@ int check_gemm_args(const e2v2_gemm_args& G) {
   return 0;
 }
 int host_tiles(const e2v2_gemm_args& G) { return G.batch * ((G.m + kGM - 1) / kGM) * (G.n / kGN); }
+
+// Which matrices take the K-split tiles (gemm_ks.h): few rows, decided by the rows alone so that a GEMM is
+// summed in the same order whether it runs alone, as a batch member or in a group.  Measured (us per call,
+// 128 x 128 tiles against K-split, operands not in L2):
+//   three pieces, 9 batches, K 256 -> 256:  m 24: 19.0 / 5.9, 648: 24.3 / 11.1, 1500: 26.0 / 19.8,
+//                                           2500: 31.9 / 30.0, 3318: 33.0 / 34.7, 10000: 86.8 / 110
+//   three pieces, 2 batches, K 1536 -> 512: m 24: 61.4 / 14.7, 648: 78.7 / 28.6, 2500: 81.2 / 66.8, 3318: 82.4 / 88.6
+//   one piece, fp32 A, 9 x 256 -> 256:      m 24: 15.2 / 4.8, 1500: 22.1 / 15.5, 2500: 24.0 / 23.6, 3318: 23.5 / 25.9
+//   one piece, bf16 A, 9 x 256 -> 256:      m 24: 14.2 / 4.4, 2500: 20.9 / 15.8, 3318: 21.6 / 18.9, 5000: 23.8 / 26.1
+// Above that the K-split form's fourfold operand traffic per product costs more than the stages it saves.
+constexpr int kKsRows = 2560, kKsRowsBf16 = 3584;
+bool ks_gemm(const e2v2_gemm_args& G) { return G.m <= (G.a_bf16 ? kKsRowsBf16 : kKsRows); }
+// The Q/K projection (three pieces, forward and backward): n 24: 60.2 / 11.8 and 106.6 / 22.8, 648: 79.5 / 57.3 and
+// 122 / 86, 1000: 90.1 / 84.5 and 134 / 132, 1500: 113 / 116 and 136 / 184 (one piece alike: 24: 35.4 / 8.0 and
+// 58.6 / 14.7, 1000: 58.5 / 55.4 and 97.4 / 85.7, 1500: 64.8 / 76.4 and 99.6 / 119).
+constexpr int kKsQkRows = 1024;
+// Ring depths: with three pieces two stages in flight leave four workgroups per CU; one piece takes four.
+constexpr int kKsD3 = 2, kKsD1 = 4;
 }  // namespace
 }  // namespace e2v2
 
-E2V2_API int e2v2_gemm_s3(const e2v2_gemm_args* g, hipStream_t s) {
-  using namespace e2v2;
+namespace e2v2 {
+namespace {
+int launch_gemm(const e2v2_gemm_args* g, bool by_rows, hipStream_t s) {
   E2V2_REQUIRE(g, "gemm_s3: null arguments");
   const e2v2_gemm_args& G = *g;
   if (int rc = check_gemm_args(G)) return rc;
   if (G.m == 0) return 0;
+  if (by_rows && ks_gemm(G)) {
+    const dim3 grid(xcd_grid(ks_tiles(G)));
+    if (G.pieces == 3)
+      hipLaunchKernelGGL((k_gemm_ks<3, false, kKsD3>), grid, dim3(kKsThreads), 0, s, G);
+    else if (G.a_bf16)
+      hipLaunchKernelGGL((k_gemm_ks<1, true, kKsD1>), grid, dim3(kKsThreads), 0, s, G);
+    else
+      hipLaunchKernelGGL((k_gemm_ks<1, false, kKsD1>), grid, dim3(kKsThreads), 0, s, G);
+    E2V2_LAUNCHED("k_gemm_ks");
+    return 0;
+  }
   const dim3 grid(xcd_grid(host_tiles(G)));
   if (G.pieces == 3)
     hipLaunchKernelGGL(k_gemm_s3, grid, dim3(kGT), 0, s, G);
@@ -548,6 +888,11 @@ E2V2_API int e2v2_gemm_s3(const e2v2_gemm_args* g, hipStream_t s) {
   E2V2_LAUNCHED("k_gemm_s3");
   return 0;
 }
+}  // namespace
+}  // namespace e2v2
+
+E2V2_API int e2v2_gemm_s3(const e2v2_gemm_args* g, hipStream_t s) { return e2v2::launch_gemm(g, true, s); }
+E2V2_API int e2v2_gemm_s3_padded(const e2v2_gemm_args* g, hipStream_t s) { return e2v2::launch_gemm(g, false, s); }
 
 E2V2_API int e2v2_gemm_s3_gated(const e2v2_gemm_args* g, const float* s, int64_t ld_s, float k1, float k2,
                                 hipStream_t st) {
@@ -564,6 +909,15 @@ E2V2_API int e2v2_gemm_s3_gated(const e2v2_gemm_args* g, const float* s, int64_t
   E2V2_REQUIRE((uint64_t)(G.m + kGM) * (uint64_t)ld_s * 4u < (1ull << 31), "gemm_s3_gated: logits too large (m=%d)",
                G.m);
   if (G.m == 0) return 0;
+  if (ks_gemm(G)) {
+    const dim3 grid(xcd_grid(ks_tiles(G)));
+    if (G.pieces == 3)
+      hipLaunchKernelGGL((k_gemm_ks_gate<3, kKsD3>), grid, dim3(kKsThreads), 0, st, G, GateOp{s, ld_s, k1, k2});
+    else
+      hipLaunchKernelGGL((k_gemm_ks_gate<1, kKsD1>), grid, dim3(kKsThreads), 0, st, G, GateOp{s, ld_s, k1, k2});
+    E2V2_LAUNCHED("k_gemm_ks_gate");
+    return 0;
+  }
   if (G.pieces == 3)
     hipLaunchKernelGGL((k_gemm_s3_gate<3>), dim3(xcd_grid(host_tiles(G))), dim3(kGT), 0, st, G,
                        GateOp{s, ld_s, k1, k2});
@@ -578,27 +932,40 @@ E2V2_API int e2v2_gemm_s3_grouped(const e2v2_gemm_args* groups, int n_groups, hi
   using namespace e2v2;
   E2V2_REQUIRE(groups && n_groups >= 1 && n_groups <= kGGroups, "gemm_s3_grouped: %d groups (1 .. %d)", n_groups,
                kGGroups);
-  GemmGroups P{};
-  P.block0[0] = 0;
   for (int i = 0; i < n_groups; ++i) {
     if (int rc = check_gemm_args(groups[i])) return rc;
     E2V2_REQUIRE(groups[i].pieces == groups[0].pieces && groups[i].a_bf16 == groups[0].a_bf16,
                  "gemm_s3_grouped: the groups must share the operand pieces and A's storage type");
-    P.g[i] = groups[i];
-    P.block0[i + 1] = P.block0[i] + xcd_grid(host_tiles(groups[i]));
-    E2V2_REQUIRE(P.block0[i + 1] >= P.block0[i], "gemm_s3_grouped: too many tiles");
   }
-  for (int i = n_groups; i < kGGroups; ++i) P.block0[i + 1] = P.block0[n_groups];
-  P.n = n_groups;
-  if (P.block0[n_groups] == 0) return 0;
-  const dim3 grid(P.block0[n_groups]);
-  if (groups[0].pieces == 3)
-    hipLaunchKernelGGL(k_gemm_s3_grp, grid, dim3(kGT), 0, s, P);
-  else if (groups[0].a_bf16)
-    hipLaunchKernelGGL((k_gemm_s3_grp_p1<true>), grid, dim3(kGT), 0, s, P);
-  else
-    hipLaunchKernelGGL((k_gemm_s3_grp_p1<false>), grid, dim3(kGT), 0, s, P);
-  E2V2_LAUNCHED("k_gemm_s3_grp");
+  // the groups of each tiling in the order given: one launch unless both tilings occur
+  for (int ks = 0; ks < 2; ++ks) {
+    GemmGroups P{};
+    P.block0[0] = P.n = 0;
+    for (int i = 0; i < n_groups; ++i) {
+      if (ks_gemm(groups[i]) != (ks == 1)) continue;
+      const int tiles = ks ? ks_tiles(groups[i]) : host_tiles(groups[i]);
+      P.g[P.n] = groups[i];
+      P.block0[P.n + 1] = P.block0[P.n] + xcd_grid(tiles);
+      E2V2_REQUIRE(P.block0[P.n + 1] >= P.block0[P.n], "gemm_s3_grouped: too many tiles");
+      ++P.n;
+    }
+    for (int i = P.n; i < kGGroups; ++i) P.block0[i + 1] = P.block0[P.n];
+    if (P.block0[P.n] == 0) continue;
+    const dim3 grid(P.block0[P.n]);
+    if (ks && P.g[0].pieces == 3)
+      hipLaunchKernelGGL((k_gemm_ks_grp<3, false, kKsD3>), grid, dim3(kKsThreads), 0, s, P);
+    else if (ks && P.g[0].a_bf16)
+      hipLaunchKernelGGL((k_gemm_ks_grp<1, true, kKsD1>), grid, dim3(kKsThreads), 0, s, P);
+    else if (ks)
+      hipLaunchKernelGGL((k_gemm_ks_grp<1, false, kKsD1>), grid, dim3(kKsThreads), 0, s, P);
+    else if (P.g[0].pieces == 3)
+      hipLaunchKernelGGL(k_gemm_s3_grp, grid, dim3(kGT), 0, s, P);
+    else if (P.g[0].a_bf16)
+      hipLaunchKernelGGL((k_gemm_s3_grp_p1<true>), grid, dim3(kGT), 0, s, P);
+    else
+      hipLaunchKernelGGL((k_gemm_s3_grp_p1<false>), grid, dim3(kGT), 0, s, P);
+    E2V2_LAUNCHED("k_gemm_s3_grp");
+  }
   return 0;
 }
 
@@ -618,6 +985,17 @@ E2V2_API int e2v2_qk_proj_fwd_s3(const float* x, const void* wp, const float* bi
   E2V2_REQUIRE(n >= 0 && (uint64_t)(n + kGM) * (uint64_t)c * 4u < (1ull << 31) &&
                    (uint64_t)(n + kGM) * 4u * hid < (1ull << 32), "qk_proj_fwd_s3: n=%d too large", n);
   if (n == 0) return 0;
+  if (n <= kKsQkRows && c == 256) {
+    const dim3 grid(3 * xcd_grid(((n + 31) / 32) * (2 * hid / 32)));
+    if (pieces == 3)
+      hipLaunchKernelGGL((k_qk_ks_fwd<3, false>), grid, dim3(kKsThreads), 0, s, x, wp, bias, y, hq, hk, n, hid);
+    else if (y_bf16)
+      hipLaunchKernelGGL((k_qk_ks_fwd<1, true>), grid, dim3(kKsThreads), 0, s, x, wp, bias, y, hq, hk, n, hid);
+    else
+      hipLaunchKernelGGL((k_qk_ks_fwd<1, false>), grid, dim3(kKsThreads), 0, s, x, wp, bias, y, hq, hk, n, hid);
+    E2V2_LAUNCHED("k_qk_ks_fwd");
+    return 0;
+  }
   const int tiles = ((n + kGM - 1) / kGM) * (2 * hid / 64);
   const dim3 grid(3 * xcd_grid(tiles));
   if (pieces == 3)
@@ -648,6 +1026,17 @@ E2V2_API int e2v2_qk_proj_bwd_s3(const void* y, const float* ghq, const float* g
   E2V2_REQUIRE(n >= 0 && (uint64_t)(n + kGM) * 4u * hid * 4u < (1ull << 31) &&
                    (uint64_t)(n + kGM) * (uint64_t)cv * 4u < (1ull << 31), "qk_proj_bwd_s3: n=%d too large", n);
   if (n == 0) return 0;
+  if (n <= kKsQkRows) {
+    const dim3 grid(xcd_grid(9 * ((n + 31) / 32) * (c / (32 * kKsJ)))), blk(kKsThreads);
+    if (pieces == 3)
+      hipLaunchKernelGGL((k_qk_ks_bwd<3, false, 2>), grid, blk, 0, s, y, ghq, ghk, wp, gv, gx, n, hid, c, cv);
+    else if (y_bf16)
+      hipLaunchKernelGGL((k_qk_ks_bwd<1, true, 2>), grid, blk, 0, s, y, ghq, ghk, wp, gv, gx, n, hid, c, cv);
+    else
+      hipLaunchKernelGGL((k_qk_ks_bwd<1, false, 2>), grid, blk, 0, s, y, ghq, ghk, wp, gv, gx, n, hid, c, cv);
+    E2V2_LAUNCHED("k_qk_ks_bwd");
+    return 0;
+  }
   const int tiles = 9 * ((n + kGM - 1) / kGM) * (c / kGN);
   const dim3 grid(xcd_grid(tiles));
   if (pieces == 3)

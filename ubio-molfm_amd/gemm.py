@@ -144,18 +144,22 @@ def _args(a, pw: PackedWeight, out: torch.Tensor, widx=None, bias=None, bias_bat
 
 def gemm(a, pw: PackedWeight, out: torch.Tensor, widx: Optional[Sequence[int]] = None,
          bias: Optional[torch.Tensor] = None, bias_batches: int = 1, res: Optional[torch.Tensor] = None,
-         gate=None):
+         gate=None, padded_rows: bool = False):
     """out[b] = a[b] W_{widx[b]}^T (+ bias for b < bias_batches) (+ res[b]).
     a [batch, m, k] or [m, k] fp32 (rows may be strided, k contiguous), or a list of
     same-layout [m, k] matrices; out and res [batch, m, n] (res may be out); bias [n]
     (shared) or [batch, n] (one per batch).  gate = (s, k1, k2): Gate_s3's activation
     applied to A as it is read (``e2v2_gemm_s3_gated``): batch 0 takes silu(s[:, :k]) k1,
-    batch b >= 1 takes a[b] * sigmoid(s[:, k widx[b]:k (widx[b] + 1)]) k2."""
+    batch b >= 1 takes a[b] * sigmoid(s[:, k widx[b]:k (widx[b] + 1)]) k2.  padded_rows: the row
+    count is a capacity; every row is summed in the same order whatever m
+    (``e2v2_gemm_s3_padded``)."""
     g, work, keep = _args(a, pw, out, widx, bias, bias_batches, res)   # keep: referenced until the launch
     if g is None:
         return out
     st = _lib.vp(torch.cuda.current_stream(out.device).cuda_stream)
-    entry = "e2v2_gemm_s3" if gate is None else "e2v2_gemm_s3_gated"
+    if padded_rows and gate is not None:
+        raise ValueError("gemm: padded_rows does not combine with a gate")
+    entry = "e2v2_gemm_s3_gated" if gate is not None else "e2v2_gemm_s3_padded" if padded_rows else "e2v2_gemm_s3"
     if gate is not None:
         sg, k1, k2 = gate
         if sg.dtype != torch.float32 or sg.dim() != 2 or sg.stride(1) != 1 or sg.shape[0] != _as3(out).shape[1]:
@@ -166,10 +170,10 @@ def gemm(a, pw: PackedWeight, out: torch.Tensor, widx: Optional[Sequence[int]] =
         top = max(int(g.widx[b]) for b in range(1, nb)) + 1 if nb > 1 else 0
         if pw.k * max(top, 1) > sg.shape[1]:
             raise ValueError(f"gemm: gate logits of {sg.shape[1]} columns, the batches read {pw.k * max(top, 1)}")
-        _lib.call("e2v2_gemm_s3_gated", _lib.C.byref(g), _lib.vp(sg.data_ptr()), _lib.i64(sg.stride(0)),
+        _lib.call(entry, _lib.C.byref(g), _lib.vp(sg.data_ptr()), _lib.i64(sg.stride(0)),
                   _lib.f32(k1), _lib.f32(k2), st)
     else:
-        _lib.call("e2v2_gemm_s3", _lib.C.byref(g), st)
+        _lib.call(entry, _lib.C.byref(g), st)
     del keep
     if _lib._timer is not None:
         _lib._timer.add_work(entry, work)

@@ -763,23 +763,25 @@ class DenseFn(torch.autograd.Function):
 
 class DenseS3Fn(torch.autograd.Function):
     """y = x W^T + b for a constant fp32 weight on the split GEMM (packs of W for
-    the forward and of W^T for the input gradient); input gradient only."""
+    the forward and of W^T for the input gradient); input gradient only.
+    padded_rows: x's rows are the slots of a capacity neighbour list
+    (``gemm.gemm``)."""
 
     @staticmethod
-    def forward(ctx, x, packs, b):
+    def forward(ctx, x, packs, b, padded_rows=False):
         x = x.contiguous()
         pf, pb = packs
         y = x.new_empty(x.shape[0], pf.n)
-        s3gemm.gemm(x, pf, y, bias=b)
-        ctx.pb = pb
+        s3gemm.gemm(x, pf, y, bias=b, padded_rows=padded_rows)
+        ctx.pb, ctx.padded_rows = pb, padded_rows
         return y
 
     @staticmethod
     def backward(ctx, gy):
         gy = gy.contiguous()
         gx = gy.new_empty(gy.shape[0], ctx.pb.n)
-        s3gemm.gemm(gy, ctx.pb, gx)
-        return gx, None, None
+        s3gemm.gemm(gy, ctx.pb, gx, padded_rows=ctx.padded_rows)
+        return gx, None, None, None
 
 
 def dense_packs(lin: nn.Linear, bf16: bool = False):
@@ -794,12 +796,12 @@ def dense_packs(lin: nn.Linear, bf16: bool = False):
                   lambda: (s3gemm.pack(w.detach(), pieces=pc), s3gemm.pack(w.detach(), transpose=True, pieces=pc)))
 
 
-def _linear(x, lin: nn.Linear):
+def _linear(x, lin: nn.Linear, padded_rows: bool = False):
     if x.dim() == 2 and x.dtype == torch.float32:
         packs = dense_packs(lin)
         if packs is not None:
             b = None if lin.bias is None else lin.bias.detach().float().contiguous()
-            return DenseS3Fn.apply(x, packs, b)
+            return DenseS3Fn.apply(x, packs, b, padded_rows)
     return torch.nn.functional.linear(x, lin.weight.detach(), None if lin.bias is None else lin.bias.detach())
 
 
@@ -1500,7 +1502,7 @@ class E2AttentionArbOrder_sparse(nn.Module):
                                          self.fc_m0.bias.detach())
             rad = RadialEvalFn.apply(ctx.dist, nl, ctx.atom_type, tab)
             x0 = ShContractFn.apply(_sh_integral(ctx.dvec), xd, nl).reshape(E, -1)    # [E, 3 Cd]
-            return _linear(x0 * rad, self.fc_m0)
+            return _linear(x0 * rad, self.fc_m0, True)
         rad = RadialEvalFn.apply(ctx.dist, nl, ctx.atom_type, tab)
         # checked once per version of sum_vec (a host readback), not on every evaluation
         if not cached(self, "sum_vec_ok", (self.sum_vec,),
@@ -1508,7 +1510,7 @@ class E2AttentionArbOrder_sparse(nn.Module):
             raise NotImplementedError("QKdotS_alpha: sum_vec must keep its l-block indicator values")
         x0 = ShContractFn.apply(_raw_sh(ctx.dvec), xd, nl).reshape(E, -1)[:, :H]     # [E, H]
         dl = self.direction_linear
-        return _linear(_ln_silu(_linear(x0 * rad[:, :H], dl[0]), dl[1]), dl[3])
+        return _linear(_ln_silu(_linear(x0 * rad[:, :H], dl[0], True), dl[1]), dl[3], True)
 
     def _sum_vec_blocks(self):
         L = self.lmax + 1
