@@ -467,6 +467,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TS) 
   const int n_cl = (A.n_rows + R - 1) / R;
   const int cl = xcd_row(blockIdx.x, n_cl);
   if (cl >= n_cl) return;
+  if (grp < 0) {   // all groups in this launch, one per blockIdx.y, each with its own [E][32] pair
+    grp = blockIdx.y;
+    w_g += (size_t)grp * A.n_edges * kGroupHeads;
+    dqk_g += (size_t)grp * A.n_edges * kGroupHeads;
+  }
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = t >> 6;
   const int c = kGroupC * grp + lane;   // channel position
   const int hc = pos_head(c) - kGroupHeads * grp;                     // its head within the group
@@ -656,9 +661,17 @@ __global__ __launch_bounds__(64) void k_attn_bwd_row_sl(e2v2_attn_args A, const 
   __shared__ float er_hw[6][CH];   // quintic Hermite weights of the fraction in the node interval
   // slice 2 grp on the even XCDs (blockIdx % 8 = 0, 2, 4, 6), 2 grp + 1 on the odd ones; the four XCDs of a
   // slice take contiguous quarters of the rows, each in order, so an XCD's rows stay spatially compact
+  // (grp < 0: all slices in this launch, slice = blockIdx % 8 as in the forward, every group with its own
+  // [E][32] pair)
   const int x = blockIdx.x % kXcd, quarter = (A.n_rows + 3) / 4;
-  const int s = 2 * grp + (x & 1), i = (x >> 1) * quarter + (int)(blockIdx.x / kXcd);
-  if (blockIdx.x / kXcd >= (unsigned)quarter || i >= A.n_rows) return;
+  const bool all = grp < 0;
+  if (all) {
+    grp = x >> 1;
+    w_out += (size_t)grp * A.n_edges * kGroupHeads;
+    dqk_out += (size_t)grp * A.n_edges * kGroupHeads;
+  }
+  const int s = 2 * grp + (x & 1), i = all ? (int)(blockIdx.x / kXcd) : (x >> 1) * quarter + (int)(blockIdx.x / kXcd);
+  if ((!all && blockIdx.x / kXcd >= (unsigned)quarter) || i >= A.n_rows) return;
   const int lane = threadIdx.x, hh = lane & (kSlH - 1), sub = lane >> 4;
   const int h = kSlH * s + hh;
   const int hg = h - kGroupHeads * grp;   // head within the group (w, dqk columns)
@@ -948,35 +961,50 @@ E2V2_API int e2v2_attn_fwd(const e2v2_attn_args* args, void* out, float* mrow, f
   });
 }
 
-// workspace of e2v2_attn_bwd: w [E][32] and dL/dqk [E][32] of one head group, handed from that group's row
-// pass to its column pass, and the slice partials of dL/d dvec, dL/dd [8][E][4]
-static size_t bwd_ws_floats(int64_t n_edges) { return (size_t)n_edges * (2 * kGroupHeads + 4 * kSl); }
+// Up to this many edges the backward runs its four head groups in one row launch and one column launch, each
+// group with its own w / dqk pair: a group of a small system alone leaves most of the GPU idle (row + column
+// passes of a layer: 24 atoms 4 x (17.8 + 26.5) = 177 us, merged 47; 648 atoms, 59 k edges, 4 x (29.2 + 47.5) =
+// 307 us, merged 177).  Above it a group fills the GPU by itself (1,501 atoms, 128 k edges: 3,002 wavefronts of
+// the row pass at two per SIMD) and the pairs of four groups would be the largest per-edge allocation (1.2 KB per
+// edge instead of 384 B).
+constexpr int64_t kMergeEdges = 98304;
+static int bwd_pairs(int64_t n_edges) { return n_edges <= kMergeEdges ? kGroups : 1; }
+// workspace of e2v2_attn_bwd: w [E][32] and dL/dqk [E][32] of one head group (of each, when merged), handed from
+// the row pass to the column pass, and the slice partials of dL/d dvec, dL/dd [8][E][4]
+static size_t bwd_ws_floats(int64_t n_edges) {
+  return (size_t)n_edges * (2 * kGroupHeads * bwd_pairs(n_edges) + 4 * kSl);
+}
 
 E2V2_API size_t e2v2_attn_bwd_workspace(int64_t n_edges) {
   return n_edges > 0 ? bwd_ws_floats(n_edges) * sizeof(float) : 0;
 }
 
-// The four head groups in turn: the row pass of the group's two slices, then its column pass (clusters when
-// given, else one column per workgroup); finally the slice partials are added per edge.
+// The four head groups in turn (or merged): the row pass of the group's two slices, then its column pass (clusters
+// when given, else one column per workgroup); finally the slice partials are added per edge.
 template <typename TS, int kMode>
 static int attn_bwd_launch(const e2v2_attn_args& A, const TS* G, const TS* O, const float* mrow, const float* srow,
                            const int32_t* cnt, float* ddvec, float* ddist, float* dq, float* dk, float* dv,
                            float* ws, hipStream_t s) {
   const int64_t E = A.n_edges;
+  const int np = bwd_pairs(E);
+  const bool all = np == kGroups;
   float* w_g = ws;
-  float* dqk_g = ws + (size_t)E * kGroupHeads;
-  float* part = ws + (size_t)E * 2 * kGroupHeads;
-  for (int g = 0; g < kGroups; ++g) {
-    hipLaunchKernelGGL((k_attn_bwd_row_sl<TS, kMode>), dim3((unsigned)((A.n_rows + 3) / 4) * kXcd), dim3(kWave), 0, s, A, G, O,
-                       mrow, srow, cnt, part, dq, w_g, dqk_g, g);
+  float* dqk_g = ws + (size_t)E * kGroupHeads * np;
+  float* part = ws + (size_t)E * 2 * kGroupHeads * np;
+  const unsigned ny = all ? kGroups : 1;
+  for (int g = 0; g < (all ? 1 : kGroups); ++g) {
+    const int grp = all ? -1 : g;
+    const dim3 rgrid(all ? (unsigned)A.n_rows * kSl : (unsigned)((A.n_rows + 3) / 4) * kXcd);
+    hipLaunchKernelGGL((k_attn_bwd_row_sl<TS, kMode>), rgrid, dim3(kWave), 0, s, A, G, O, mrow, srow, cnt, part, dq,
+                       w_g, dqk_g, grp);
     E2V2_LAUNCHED("k_attn_bwd_row_sl");
     if (A.col_slot_member) {
       const int n_cl = (A.n_rows + 3) / 4;
-      hipLaunchKernelGGL((k_attn_bwd_col_grp<4, TS, true, kMode & kModeZero>), dim3(xcd_grid(n_cl)), dim3(256), 0, s, A, G, w_g, dqk_g,
-                         dv, dk, g);
+      hipLaunchKernelGGL((k_attn_bwd_col_grp<4, TS, true, kMode & kModeZero>), dim3(xcd_grid(n_cl), ny), dim3(256), 0,
+                         s, A, G, w_g, dqk_g, dv, dk, grp);
     } else {
-      hipLaunchKernelGGL((k_attn_bwd_col_grp<1, TS, false, kMode & kModeZero>), dim3(xcd_grid(A.n_rows)), dim3(256), 0, s, A, G, w_g,
-                         dqk_g, dv, dk, g);
+      hipLaunchKernelGGL((k_attn_bwd_col_grp<1, TS, false, kMode & kModeZero>), dim3(xcd_grid(A.n_rows), ny),
+                         dim3(256), 0, s, A, G, w_g, dqk_g, dv, dk, grp);
     }
     E2V2_LAUNCHED("k_attn_bwd_col_grp");
   }

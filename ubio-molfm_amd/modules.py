@@ -410,9 +410,9 @@ class SO2OutFn(torch.autograd.Function):
             K = W.shape[0]
             A = so2[start * N:(start + (2 * l3 + 1) * K) * N].view(-1, K)
             a, b = l3 * l3, (l3 + 1) ** 2
-            if split:
-                problems.append({"a": A, "pw": PF, "out": y[a:b].view(-1, O), "bias": bias if l3 == 0 else None,
-                                 "res": None if res is None else res[a:b].view(-1, O)})
+            if split:      # one batch per order m: N rows each, so that few atoms take the few-row tiles
+                problems.append({"a": A.view(b - a, N, K), "pw": PF, "out": y[a:b], "widx": [0] * (b - a),
+                                 "bias": bias if l3 == 0 else None, "res": None if res is None else res[a:b]})
             elif res is not None:
                 _addmm_into(res[a:b].view(-1, O), A, W, out=y[a:b].view(-1, O))
             else:
@@ -440,7 +440,7 @@ class SO2OutFn(torch.autograd.Function):
             a, b = l3 * l3, (l3 + 1) ** 2
             dst = gso2[start * N:(start + (2 * l3 + 1) * K) * N].view(-1, K)
             if split:
-                problems.append({"a": gy[a:b].view(-1, O), "pw": PB, "out": dst})
+                problems.append({"a": gy[a:b], "pw": PB, "out": dst.view(b - a, N, K), "widx": [0] * (b - a)})
             else:
                 _mm_into(gy[a:b].view(-1, O), WT, out=dst)
         if split:                                # one launch, the most tiles first
