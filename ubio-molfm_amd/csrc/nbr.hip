@@ -5,6 +5,7 @@
 // (src/molfm/models/e2former/module_utils.py:1065-1274,3119-3242) and the
 // CSR metadata of prepare_sparse_qk_edge_index_metadata
 // (src/molfm/models/e2former/triton_dr/triton_sparse_qk_autograd.py:601-652).
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -24,44 +25,81 @@ __global__ void k_fill_f32(float* __restrict__ p, float v, int64_t n) {
   for (; i < n; i += stride) p[i] = v;
 }
 
-// Single-workgroup exclusive scan: out[0..n] with out[n] = total;
-// stats[0] = total, stats[1] = max(in).
-__global__ __launch_bounds__(1024) void k_scan_i32(const int32_t* __restrict__ in, int n,
-                                                   int32_t* __restrict__ out, int32_t* __restrict__ stats) {
-  __shared__ int64_t part[1024];
-  __shared__ int32_t pmax[1024];
-  const int t = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int b = t * per;
-  const int e = min(n, b + per);
-  int64_t s = 0;
+// Exclusive scan: out[0..n] with out[n] = total; stats[0] = total, stats[1] = max(in).  Workgroup b owns the
+// elements [b len, (b + 1) len) and adds up everything before them itself (coalesced, from the L2), so one launch
+// needs neither a workspace nor a wait on other workgroups; the last one sees every element and writes the stats.
+// The re-reading is n / 2 elements per workgroup on average, which bounds the workgroups (kScanBlocks).
+// A single workgroup walking per-thread runs (uncoalesced) took 125 us for 100,000 elements, this takes 10 us.
+constexpr int kScanThreads = 1024, kScanBlocks = 256;
+constexpr int scan_len(int n) {   // elements per workgroup: a multiple of the workgroup's stride
+  const int per = (n + kScanBlocks - 1) / kScanBlocks;
+  return (per + kScanThreads - 1) / kScanThreads * kScanThreads;
+}
+__global__ __launch_bounds__(kScanThreads) void k_scan_i32(const int32_t* __restrict__ in, int n, int len,
+                                                           int32_t* __restrict__ out, int32_t* __restrict__ stats) {
+  constexpr int kW = kScanThreads / 64;
+  __shared__ int64_t wsum[kW];
+  __shared__ int32_t wmax[kW];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const bool last = blockIdx.x == gridDim.x - 1;
+  const int b = blockIdx.x * len, e = min(n, b + len);
+  int64_t base = 0;
   int32_t mx = 0;
-  for (int i = b; i < e; ++i) {
-    s += in[i];
-    mx = max(mx, in[i]);
+#pragma unroll 4
+  for (int i = t; i < b; i += kScanThreads) {
+    const int32_t v = in[i];
+    base += v;
+    mx = max(mx, v);
   }
-  part[t] = s;
-  pmax[t] = mx;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) base += __shfl_xor(base, o, 64);
+  if (lane == 0) wsum[w] = base;
   __syncthreads();
-  // Hillis-Steele inclusive scan over 1024 partials
-  for (int o = 1; o < 1024; o <<= 1) {
-    int64_t v = (t >= o) ? part[t - o] : 0;
-    int32_t m = (t >= o) ? pmax[t - o] : 0;
+  base = 0;
+#pragma unroll
+  for (int u = 0; u < kW; ++u) base += wsum[u];
+  __syncthreads();
+  for (int c = b; c < e; c += kScanThreads) {
+    const int i = c + t;
+    const int32_t v = i < e ? in[i] : 0;
+    mx = max(mx, v);
+    int64_t x = v;                       // inclusive scan over the wavefront
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int64_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[w] = x;
     __syncthreads();
-    part[t] += v;
-    pmax[t] = max(pmax[t], m);
+    int64_t before = base, all = base;
+#pragma unroll
+    for (int u = 0; u < kW; ++u) {
+      before += u < w ? wsum[u] : 0;
+      all += wsum[u];
+    }
+    if (i < e) out[i] = (int32_t)(before + x - v);
+    base = all;
     __syncthreads();
   }
-  int64_t run = part[t] - s;
-  for (int i = b; i < e; ++i) {
-    out[i] = (int32_t)run;
-    run += in[i];
+  if (!last) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
+  if (lane == 0) wmax[w] = mx;
+  __syncthreads();
+  if (t == 0) {
+#pragma unroll
+    for (int u = 0; u < kW; ++u) mx = max(mx, wmax[u]);
+    out[n] = (int32_t)base;
+    stats[0] = (int32_t)base;
+    stats[1] = mx;
   }
-  if (t == 1023) {
-    out[n] = (int32_t)part[1023];
-    stats[0] = (int32_t)part[1023];
-    stats[1] = pmax[1023];
-  }
+}
+static int launch_scan(const int32_t* in, int n, int32_t* out, int32_t* stats, hipStream_t s) {
+  const int len = scan_len(n);
+  const int blocks = n > 0 ? (n + len - 1) / len : 1;
+  hipLaunchKernelGGL(k_scan_i32, dim3(blocks), dim3(kScanThreads), 0, s, in, n, len, out, stats);
+  E2V2_LAUNCHED("k_scan_i32");
+  return 0;
 }
 
 __device__ __forceinline__ int bin_coord(float x, float lo, float h, int dim) {
@@ -138,9 +176,14 @@ __device__ bool image_has_inner(const e2v2_nbr_plan& P, int g, const float* img)
 // rounding of the bin range could add starts beyond q + rc + margin, so it holds
 // no edge.)  emit(ok, j, s, dx, dy, dz, d) is called by every lane of the wave in
 // each round (ok false on lanes without an edge) and may use wave-wide ballots.
+// The bin ranges of 64 shifts are formed at once, one per lane (a large box has 27 shifts of which an atom away
+// from the faces needs one: a walk over them with its six divisions each was most of the count's time), and the
+// nine runs of a shift by nine lanes; the wave then reads them as scalars.  100,000 atoms: count 348 -> 172 us,
+// fill 408 -> 229 us.
 template <class Emit>
-__device__ void visit_edges_wave(const e2v2_nbr_plan& P, int i, Emit&& emit) {
+__device__ void visit_edges_wave(const e2v2_nbr_plan& P, int i_, Emit&& emit) {
   const int lane = threadIdx.x & 63;
+  const int i = __builtin_amdgcn_readfirstlane(i_);
   const int g = P.atom_graph[i];
   const bool periodic = P.graph_periodic[g] != 0;
   const float pi[3] = {P.pos[3 * i], P.pos[3 * i + 1], P.pos[3 * i + 2]};
@@ -149,35 +192,53 @@ __device__ void visit_edges_wave(const e2v2_nbr_plan& P, int i, Emit&& emit) {
   const int d0 = P.grid_dim[3 * g], d1 = P.grid_dim[3 * g + 1], d2 = P.grid_dim[3 * g + 2];
   const int bbase = P.bin_base[g];
   const float r = P.rc + kBinMargin;
-  for (int s = P.graph_shift_ptr[g]; s < P.graph_shift_ptr[g + 1]; ++s) {
-    const float* off = P.shift_off + 3 * s;
-    const float q0 = pi[0] - off[0], q1 = pi[1] - off[1], q2 = pi[2] - off[2];
-    int x0 = (int)floorf((q0 - r - lo0) / h0), x1 = (int)floorf((q0 + r - lo0) / h0);
-    if (x1 < 0 || x0 > d0 - 1) continue;
-    int y0 = (int)floorf((q1 - r - lo1) / h1), y1 = (int)floorf((q1 + r - lo1) / h1);
-    if (y1 < 0 || y0 > d1 - 1) continue;
-    int z0 = (int)floorf((q2 - r - lo2) / h2), z1 = (int)floorf((q2 + r - lo2) / h2);
-    if (z1 < 0 || z0 > d2 - 1) continue;
-    x0 = max(x0, 0); y0 = max(y0, 0); z0 = max(z0, 0);
-    x1 = min(min(x1, d0 - 1), x0 + 2); y1 = min(min(y1, d1 - 1), y0 + 2); z1 = min(min(z1, d2 - 1), z0 + 2);
-    // run r = (a, b) holds bins (x0 + a, y0 + b, z0..z1); pre = inclusive prefix of
+  const int s_end = P.graph_shift_ptr[g + 1];
+  const int ra = lane / 3, rb = lane % 3;             // the run of lanes 0 .. 8
+  for (int sb = P.graph_shift_ptr[g]; sb < s_end; sb += 64) {
+    const int sl = sb + lane;
+    int x0 = 0, x1 = -1, y0 = 0, y1 = -1, z0 = 0, z1 = -1;
+    float o0 = 0.f, o1 = 0.f, o2 = 0.f;
+    bool in = false;
+    if (sl < s_end) {
+      o0 = P.shift_off[3 * sl];
+      o1 = P.shift_off[3 * sl + 1];
+      o2 = P.shift_off[3 * sl + 2];
+      const float q0 = pi[0] - o0, q1 = pi[1] - o1, q2 = pi[2] - o2;
+      x0 = (int)floorf((q0 - r - lo0) / h0), x1 = (int)floorf((q0 + r - lo0) / h0);
+      y0 = (int)floorf((q1 - r - lo1) / h1), y1 = (int)floorf((q1 + r - lo1) / h1);
+      z0 = (int)floorf((q2 - r - lo2) / h2), z1 = (int)floorf((q2 + r - lo2) / h2);
+      in = x1 >= 0 && x0 <= d0 - 1 && y1 >= 0 && y0 <= d1 - 1 && z1 >= 0 && z0 <= d2 - 1;
+      x0 = max(x0, 0); y0 = max(y0, 0); z0 = max(z0, 0);
+      x1 = min(min(x1, d0 - 1), x0 + 2); y1 = min(min(y1, d1 - 1), y0 + 2); z1 = min(min(z1, d2 - 1), z0 + 2);
+    }
+    for (uint64_t todo = __ballot(in); todo; todo &= todo - 1) {
+    const int l = (int)__builtin_ctzll(todo), s = sb + l;
+    auto scalar = [&](int v) { return __builtin_amdgcn_readlane(v, l); };
+    const float off[3] = {__int_as_float(scalar(__float_as_int(o0))), __int_as_float(scalar(__float_as_int(o1))),
+                          __int_as_float(scalar(__float_as_int(o2)))};
+    const int bx = scalar(x0) + ra, by = scalar(y0) + rb, bz0 = scalar(z0), bz1 = scalar(z1);
+    // run (a, b) holds bins (x0 + a, y0 + b, z0..z1); pre = inclusive prefix of
     // run lengths, base = run start - exclusive prefix
+    int st = 0, len = 0;
+    if (lane < 9 && bx <= scalar(x1) && by <= scalar(y1)) {
+      const int bin = bbase + (bx * d1 + by) * d2;
+      st = P.bin_start[bin + bz0];
+      len = P.bin_start[bin + bz1 + 1] - st;
+    }
+    int incl = len;
+#pragma unroll
+    for (int o = 1; o < 9; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    const int bs = st - (incl - len);
     int pre[9], base[9];
-    int total = 0;
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int b = 0; b < 3; ++b) {
-        int st = 0, len = 0;
-        if (x0 + a <= x1 && y0 + b <= y1) {
-          const int bin = bbase + ((x0 + a) * d1 + (y0 + b)) * d2;
-          st = P.bin_start[bin + z0];
-          len = P.bin_start[bin + z1 + 1] - st;
-        }
-        base[3 * a + b] = st - total;
-        total += len;
-        pre[3 * a + b] = total;
-      }
+    for (int q = 0; q < 9; ++q) {
+      pre[q] = __builtin_amdgcn_readlane(incl, q);
+      base[q] = __builtin_amdgcn_readlane(bs, q);
+    }
+    const int total = pre[8];
     for (int c0 = 0; c0 < total; c0 += 64) {
       const int c = c0 + lane;
       bool ok = false;
@@ -204,6 +265,7 @@ __device__ void visit_edges_wave(const e2v2_nbr_plan& P, int i, Emit&& emit) {
         }
       }
       emit(ok, j, s, dx, dy, dz, d);
+    }
     }
   }
 }
@@ -256,6 +318,11 @@ __global__ __launch_bounds__(64 * kNbrWaves) void k_nbr_fill(e2v2_nbr_plan P, co
 // the sorted order as source positions.
 constexpr int kMaxSeg = 4096;
 
+// The comparator of pair q at distance j: elements lo = 2 j (q / j) + q % j and lo + j (every thread takes whole
+// pairs: a walk over the elements leaves half of the threads without one; 100,000 rows of 92 edges: 300 -> 195 us
+// with the copy of the row, columns with 32-bit keys and no payload 289 -> 115 us).
+__device__ __forceinline__ int pair_lo(int q, int j) { return ((q & ~(j - 1)) << 1) | (q & (j - 1)); }
+
 __device__ void segment_sort(const uint64_t* __restrict__ key, int b, int n, uint64_t* sk, int32_t* sv) {
   int p2 = 1;
   while (p2 < n) p2 <<= 1;
@@ -266,17 +333,36 @@ __device__ void segment_sort(const uint64_t* __restrict__ key, int b, int n, uin
   __syncthreads();
   for (int k = 2; k <= p2; k <<= 1) {
     for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int t = threadIdx.x; t < p2; t += blockDim.x) {
-        int x = t ^ j;
-        if (x > t) {
-          bool up = ((t & k) == 0);
-          uint64_t a = sk[t], c = sk[x];
-          int32_t va = sv[t], vc = sv[x];
-          bool gt = (a > c) || (a == c && va > vc);
-          if (gt == up) {
-            sk[t] = c; sk[x] = a;
-            sv[t] = vc; sv[x] = va;
-          }
+      for (int q = threadIdx.x; q < p2 / 2; q += blockDim.x) {
+        const int t = pair_lo(q, j), x = t + j;
+        const bool up = ((t & k) == 0);
+        const uint64_t a = sk[t], c = sk[x];
+        const int32_t va = sv[t], vc = sv[x];
+        const bool gt = (a > c) || (a == c && va > vc);
+        if (gt == up) {
+          sk[t] = c; sk[x] = a;
+          sv[t] = vc; sv[x] = va;
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// The same for distinct 32-bit keys without a payload (edge ids).
+__device__ void segment_sort32(const uint64_t* __restrict__ key, int b, int n, uint32_t* sk) {
+  int p2 = 1;
+  while (p2 < n) p2 <<= 1;
+  for (int t = threadIdx.x; t < p2; t += blockDim.x) sk[t] = (t < n) ? (uint32_t)key[b + t] : ~0u;
+  __syncthreads();
+  for (int k = 2; k <= p2; k <<= 1) {
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int q = threadIdx.x; q < p2 / 2; q += blockDim.x) {
+        const int t = pair_lo(q, j), x = t + j;
+        const uint32_t a = sk[t], c = sk[x];
+        if ((a > c) == ((t & k) == 0)) {
+          sk[t] = c;
+          sk[x] = a;
         }
       }
       __syncthreads();
@@ -324,11 +410,14 @@ __global__ void k_cap_rows(int32_t* __restrict__ row_ptr, int n_rows, int64_t ca
   if (i <= n_rows) row_ptr[i] = (int32_t)min((int64_t)row_ptr[i], cap_edges);
 }
 
-// edge -> row index
-__global__ void k_edge_rows(const int32_t* __restrict__ row_ptr, int n_rows, int32_t* __restrict__ edge_row) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
+// edge -> row index, one wavefront per row (a thread per row wrote 50 us for 100,000 rows of 85 edges)
+constexpr int kRowWaves = 4;
+__global__ __launch_bounds__(64 * kRowWaves) void k_edge_rows(const int32_t* __restrict__ row_ptr, int n_rows,
+                                                              int32_t* __restrict__ edge_row) {
+  const int r = blockIdx.x * kRowWaves + (int)(threadIdx.x >> 6);
   if (r >= n_rows) return;
-  for (int e = row_ptr[r]; e < row_ptr[r + 1]; ++e) edge_row[e] = r;
+  const int e1 = row_ptr[r + 1];
+  for (int e = row_ptr[r] + (int)(threadIdx.x & 63); e < e1; e += 64) edge_row[e] = r;
 }
 
 // e_end (NULL: n_edges) bounds the edges on the device: the query CSR's row_ptr[n_rows],
@@ -380,8 +469,7 @@ __device__ void sort_global(uint64_t* __restrict__ k, int n) {
 __global__ __launch_bounds__(64) void k_sort_cols(const int32_t* __restrict__ key_ptr,
                                                   uint64_t* __restrict__ tkey,
                                                   int32_t* __restrict__ key_eid, int cap) {
-  uint64_t* sk = seg_lds;
-  int32_t* sv = reinterpret_cast<int32_t*>(seg_lds + cap);
+  uint32_t* sk = reinterpret_cast<uint32_t*>(seg_lds);
   const int r = blockIdx.x;
   const int b = key_ptr[r], n = key_ptr[r + 1] - b;
   if (n == 0) return;
@@ -390,7 +478,7 @@ __global__ __launch_bounds__(64) void k_sort_cols(const int32_t* __restrict__ ke
     for (int t = threadIdx.x; t < n; t += blockDim.x) key_eid[b + t] = (int32_t)tkey[b + t];
     return;
   }
-  segment_sort(tkey, b, n, sk, sv);
+  segment_sort32(tkey, b, n, sk);     // edge ids: below 2^31
   for (int t = threadIdx.x; t < n; t += blockDim.x) key_eid[b + t] = (int32_t)sk[t];
 }
 
@@ -407,16 +495,157 @@ __global__ __launch_bounds__(64) void k_sort_cols(const int32_t* __restrict__ ke
 // slot per item in CSR order (correct, without the reuse).
 constexpr int kMaxClusterItems = 4096;
 
-__global__ __launch_bounds__(256) void k_cluster_slots(const int32_t* __restrict__ seg_ptr, int n_seg, int span,
+// A segment whose items ascend by member (a key CSR: edge ids ascend, and with them the rows) lists its
+// (member, occurrence) keys in order, so the slots of a cluster of four such segments are the union of four sorted
+// lists and need no sort: an item owns its slot when no earlier segment holds its key, and the slot's index is the
+// number of owners with a smaller key, the sum over the segments of an owner prefix at the key's lower bound.
+// Clusters with more than kMergeItems items or a segment out of order are left to k_cluster_slots (n_slots = -1).
+// 100,000 atoms of 92 edges: 124 us (+ 12 us for the pass over what is left) against 1,241 us for the sort of every
+// cluster; 24 atoms with many images per pair: below 15 against 98 us.
+constexpr int kMergeItems = 1024, kMergeSpan = 4;
+__global__ __launch_bounds__(256) void k_cluster_merge(const int32_t* __restrict__ seg_ptr, int n_seg,
                                                        const int32_t* __restrict__ member,
                                                        const int32_t* __restrict__ item_eid,
                                                        int32_t* __restrict__ slot_member,
                                                        int32_t* __restrict__ slot_edge,
                                                        int32_t* __restrict__ n_slots) {
+  constexpr int S = kMergeSpan, kPer = kMergeItems / 256;
+  __shared__ uint64_t key[kMergeItems];
+  __shared__ int32_t pre[kMergeItems + 1];
+  __shared__ int32_t wtot[4];
+  __shared__ int unsorted;
+  const int cl = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int s0 = cl * S;
+  int so[S + 1];
+  const int b = seg_ptr[s0];
+#pragma unroll
+  for (int r = 0; r <= S; ++r) so[r] = seg_ptr[min(s0 + r, n_seg)] - b;
+  const int n = so[S];
+  if (n > kMergeItems) {
+    if (t == 0) n_slots[cl] = -1;
+    return;
+  }
+  if (t == 0) unsorted = 0;
+  int eid[kPer], sg[kPer];
+#pragma unroll
+  for (int z = 0; z < kPer; ++z) {
+    const int q = 256 * z + t;
+    eid[z] = sg[z] = 0;
+    if (q < n) {
+      eid[z] = item_eid ? item_eid[b + q] : b + q;
+#pragma unroll
+      for (int r = 1; r < S; ++r) sg[z] += q >= so[r];
+      key[q] = (uint64_t)(uint32_t)member[eid[z]] << 32;
+    }
+  }
+  __syncthreads();
+  // occurrence: rank among the segment's equal members (the high words are not changed meanwhile)
+  const int32_t* hi = reinterpret_cast<const int32_t*>(key);
+  int occ[kPer];
+  bool bad = false;
+#pragma unroll
+  for (int z = 0; z < kPer; ++z) {
+    const int q = 256 * z + t;
+    occ[z] = 0;
+    if (q < n) {
+      const int first = so[0] + (sg[z] > 0 ? so[1] - so[0] : 0) + (sg[z] > 1 ? so[2] - so[1] : 0) +
+                        (sg[z] > 2 ? so[3] - so[2] : 0);
+      const int m = hi[2 * q + 1];
+      if (q > first) bad |= (uint32_t)hi[2 * (q - 1) + 1] > (uint32_t)m;
+      while (q - occ[z] - 1 >= first && hi[2 * (q - occ[z] - 1) + 1] == m) ++occ[z];
+    }
+  }
+  if (bad) unsorted = 1;
+  __syncthreads();
+  if (unsorted) {
+    if (t == 0) n_slots[cl] = -1;
+    return;
+  }
+#pragma unroll
+  for (int z = 0; z < kPer; ++z) {
+    const int q = 256 * z + t;
+    if (q < n) reinterpret_cast<int32_t*>(key)[2 * q] = occ[z];
+  }
+  __syncthreads();
+  // lower bound of the item's key in every segment, and which of them hold it
+  int lb[kPer][S];
+  uint32_t has[kPer];
+  int run = 0;
+#pragma unroll
+  for (int z = 0; z < kPer; ++z) {
+    const int q = 256 * z + t;
+    has[z] = 0;
+    bool own = false;
+    if (q < n) {
+      const uint64_t k = key[q];
+#pragma unroll
+      for (int r = 0; r < S; ++r) {
+        int x = so[r], y = so[r + 1];
+        if (r == sg[z]) {
+          x = y = q;
+        }
+        while (x < y) {
+          const int c = (x + y) >> 1;
+          if (key[c] < k) x = c + 1;
+          else y = c;
+        }
+        lb[z][r] = x;
+        if (x < so[r + 1] && key[x] == k) has[z] |= 1u << r;
+      }
+      own = (has[z] & ((1u << sg[z]) - 1u)) == 0;
+    }
+    // owners before item q: over the chunk's wavefronts, then the chunks in order
+    const uint64_t bal = __ballot(own);
+    if (lane == 0) wtot[w] = __popcll(bal);
+    __syncthreads();
+    int before = run, all = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      before += u < w ? wtot[u] : 0;
+      all += wtot[u];
+    }
+    if (q < n) pre[q] = before + lanes_below(bal);
+    run += all;
+    __syncthreads();
+  }
+  if (t == 0) {
+    pre[n] = run;
+    n_slots[cl] = run;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int z = 0; z < kPer; ++z) {
+    const int q = 256 * z + t;
+    if (q >= n) continue;
+    int64_t sl = b;
+#pragma unroll
+    for (int r = 0; r < S; ++r) sl += pre[lb[z][r]] - pre[so[r]];
+    slot_edge[sl * S + sg[z]] = eid[z];
+    if ((has[z] & ((1u << sg[z]) - 1u)) == 0) {
+      slot_member[sl] = (int32_t)(key[q] >> 32);
+#pragma unroll
+      for (int r = 0; r < S; ++r)
+        if (!(has[z] >> r & 1u)) slot_edge[sl * S + r] = -1;
+    }
+  }
+}
+
+// Any span and order, by a sort of each cluster; with only_left the clusters that k_cluster_merge left.
+constexpr int kSlotBlocks = 2048;
+__global__ __launch_bounds__(256) void k_cluster_slots(const int32_t* __restrict__ seg_ptr, int n_seg, int span,
+                                                       const int32_t* __restrict__ member,
+                                                       const int32_t* __restrict__ item_eid,
+                                                       int32_t* __restrict__ slot_member,
+                                                       int32_t* __restrict__ slot_edge,
+                                                       int32_t* __restrict__ n_slots, bool only_left) {
   __shared__ uint64_t sk[kMaxClusterItems];
   __shared__ int32_t gbase[kMaxClusterItems];
   __shared__ int32_t part[256];
-  const int cl = blockIdx.x, t = threadIdx.x;
+  __shared__ int total;
+  const int t = threadIdx.x, n_cl = (n_seg + span - 1) / span;
+  for (int cl = blockIdx.x; cl < n_cl; cl += gridDim.x) {
+  if (only_left && n_slots[cl] >= 0) continue;   // (uniform over the workgroup)
+  __syncthreads();                               // the previous cluster's LDS reads are done
   const int s0 = cl * span, s1 = min(s0 + span, n_seg);
   const int b = seg_ptr[s0], n = seg_ptr[s1] - b;
   auto eid_of = [&](int p) { return item_eid ? item_eid[p] : p; };
@@ -429,8 +658,9 @@ __global__ __launch_bounds__(256) void k_cluster_slots(const int32_t* __restrict
       slot_member[p] = member[e];
       for (int r = 0; r < span; ++r) slot_edge[(int64_t)p * span + r] = (r == sg) ? e : -1;
     }
+    __syncthreads();                             // every thread has read n_slots[cl]
     if (t == 0) n_slots[cl] = n;
-    return;
+    continue;
   }
   // keys (member, segment, position) sorted ascending
   int p2 = 1;
@@ -483,7 +713,6 @@ __global__ __launch_bounds__(256) void k_cluster_slots(const int32_t* __restrict
   }
   part[t] = local;
   __syncthreads();
-  __shared__ int total;
   if (t == 0) {
     int acc = 0;
     for (int u = 0; u < 256; ++u) {
@@ -523,6 +752,7 @@ __global__ __launch_bounds__(256) void k_cluster_slots(const int32_t* __restrict
     const int pos = (int)(sk[q] & 0xffff);
     const int64_t sl = (int64_t)b + gbase[g] + occ_of(q);
     slot_edge[sl * span + sg] = eid_of(b + pos);
+  }
   }
 }
 
@@ -769,8 +999,7 @@ E2V2_API int e2v2_fill_f32(float* p, float v, int64_t n, hipStream_t s) {
 
 E2V2_API int e2v2_scan_i32(const int32_t* in, int n, int32_t* out, int32_t* stats, hipStream_t s) {
   E2V2_REQUIRE(n >= 0, "scan: negative length %d", n);
-  hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, in, n, out, stats);
-  E2V2_LAUNCHED("k_scan_i32");
+  if (int rc = launch_scan(in, n, out, stats, s)) return rc;
   return 0;
 }
 
@@ -783,8 +1012,7 @@ E2V2_API int e2v2_nbr_bin(const e2v2_nbr_plan* plan, hipStream_t s) {
   hipLaunchKernelGGL(k_bin_assign, dim3(blocks_for(P.n_atoms, 256)), dim3(256), 0, s, P);
   E2V2_LAUNCHED("k_bin_assign");
   // bin_start = exclusive scan of counts; the count buffer becomes the fill cursor
-  hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, P.bin_count, P.n_bins, P.bin_start, P.stats);
-  E2V2_LAUNCHED("k_scan_i32");
+  if (int rc = launch_scan(P.bin_count, P.n_bins, P.bin_start, P.stats, s)) return rc;
   rc = e2v2_fill_i32(P.bin_count, 0, P.n_bins, s);
   if (rc) return rc;
   hipLaunchKernelGGL(k_bin_fill, dim3(blocks_for(P.n_atoms, 256)), dim3(256), 0, s, P, P.bin_count);
@@ -799,8 +1027,7 @@ E2V2_API int e2v2_nbr_count(const e2v2_nbr_plan* plan, int32_t* row_count, int32
                        row_count);
     E2V2_LAUNCHED("k_nbr_count");
   }
-  hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, row_count, P.n_atoms, row_ptr, P.stats);
-  E2V2_LAUNCHED("k_scan_i32");
+  if (int rc = launch_scan(row_count, P.n_atoms, row_ptr, P.stats, s)) return rc;
   return 0;
 }
 
@@ -840,8 +1067,7 @@ E2V2_API int e2v2_nbr_topk(const int32_t* row_ptr, int n_rows, int k, int32_t* c
       hipLaunchKernelGGL(k_topk_count, dim3(blocks_for(n_rows, 256)), dim3(256), 0, s, row_ptr, n_rows, k, cnt);
       E2V2_LAUNCHED("k_topk_count");
     }
-    hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, cnt, n_rows, new_ptr, stats);
-    E2V2_LAUNCHED("k_scan_i32");
+    if (int rc = launch_scan(cnt, n_rows, new_ptr, stats, s)) return rc;
     return 0;
   }
   if (n_rows == 0) return 0;
@@ -867,8 +1093,13 @@ E2V2_API int e2v2_cluster_slots(const int32_t* seg_ptr, int32_t n_seg, const int
   E2V2_REQUIRE(span >= 1 && span <= 16, "cluster_slots: span must be 1..16, got %d", span);
   if (n_seg <= 0) return 0;
   const int n_cl = (n_seg + span - 1) / span;
-  hipLaunchKernelGGL(k_cluster_slots, dim3(n_cl), dim3(256), 0, s, seg_ptr, n_seg, span, member, item_eid,
-                     slot_member, slot_edge, n_slots);
+  if (span == kMergeSpan) {
+    hipLaunchKernelGGL(k_cluster_merge, dim3(n_cl), dim3(256), 0, s, seg_ptr, n_seg, member, item_eid, slot_member,
+                       slot_edge, n_slots);
+    E2V2_LAUNCHED("k_cluster_merge");
+  }
+  hipLaunchKernelGGL(k_cluster_slots, dim3(std::min(n_cl, kSlotBlocks)), dim3(256), 0, s, seg_ptr, n_seg, span, member,
+                     item_eid, slot_member, slot_edge, n_slots, span == kMergeSpan);
   E2V2_LAUNCHED("k_cluster_slots");
   return 0;
 }
@@ -880,7 +1111,8 @@ E2V2_API int e2v2_csr_transpose(const int32_t* row_ptr, const int32_t* col, int 
   // phase 1: fill and sort each column by edge id (any column length)
   if (phase == 0) {
     if (n_rows > 0 && n_edges > 0) {
-      hipLaunchKernelGGL(k_edge_rows, dim3(blocks_for(n_rows, 256)), dim3(256), 0, s, row_ptr, n_rows, edge_row);
+      hipLaunchKernelGGL(k_edge_rows, dim3(blocks_for(n_rows, kRowWaves)), dim3(64 * kRowWaves), 0, s, row_ptr, n_rows,
+                         edge_row);
       E2V2_LAUNCHED("k_edge_rows");
     }
     int rc = e2v2_fill_i32(key_cnt, 0, n_cols, s);
@@ -890,8 +1122,7 @@ E2V2_API int e2v2_csr_transpose(const int32_t* row_ptr, const int32_t* col, int 
                          row_ptr + n_rows, key_cnt);
       E2V2_LAUNCHED("k_col_count");
     }
-    hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, key_cnt, n_cols, key_ptr, stats);
-    E2V2_LAUNCHED("k_scan_i32");
+    if (int rc = launch_scan(key_cnt, n_cols, key_ptr, stats, s)) return rc;
     return 0;
   }
   if (n_edges == 0) return 0;
@@ -945,8 +1176,7 @@ E2V2_API int e2v2_segment_metadata(const int32_t* row_index, const int32_t* othe
                          cnt, stats + 2);
       E2V2_LAUNCHED("k_coo_count");
     }
-    hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, cnt, n_rows, row_ptr, stats);
-    E2V2_LAUNCHED("k_scan_i32");
+    if (int rc = launch_scan(cnt, n_rows, row_ptr, stats, s)) return rc;
     return 0;
   }
   // phase 1: only after phase 0 reported no out-of-range row (stats[2] == 0)
@@ -988,8 +1218,7 @@ E2V2_API int e2v2_pair_count(const e2v2_pair_plan* plan, int32_t* row_count, int
                        row_count);
     E2V2_LAUNCHED("k_pair_count");
   }
-  hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, row_count, P.n_query, row_ptr, stats);
-  E2V2_LAUNCHED("k_scan_i32");
+  if (int rc = launch_scan(row_count, P.n_query, row_ptr, stats, s)) return rc;
   return 0;
 }
 
