@@ -209,6 +209,51 @@ int e2v2_seg_dot(const e2v2_segments* seg, const float* A, const int64_t* a_stri
    (sparse_alpha_sum_edge_index_autograd.py:28-67, 112-126). */
 int e2v2_seg_reduce(const e2v2_segments* seg, const float* W, const int64_t* w_strides, const float* X,
                     const int64_t* x_strides, int H, int D, float* out, const int64_t* out_strides, hipStream_t s);
+/* Fused passes of the training path (forces differentiated once more; second_order.py) over one neighbour list:
+ * the query CSR (row_ptr [n_rows + 1], col [n_edges], edge_row [n_edges]) and its key CSR (key_ptr [n_rows + 1],
+ * key_eid [n_edges]); 256 channels, 128 heads, 9 irreps rows.
+ *
+ * First-order value aggregation (so2_tensor_product.py:341-385 in Cartesian form), S = sum_e sum_k sum_c
+ * w[e, c % 128] u[e, k] sum_r g[k][r][row_e][c] v[r][col_e][c], a term absent when its w (or v2) is NULL:
+ *   e2v2_so2_agg     out[k][r][i][c]: dS/dg of (w1 u1 + w2 u2) v + (w3 u3) v2
+ *   e2v2_so2_agg_dv  dv[r][j][c]: dS/dv of (w1 u1 + w2 u2) with g
+ *   e2v2_so2_agg_dw  dw [E][128]: dS/dw of (u1, v) + (u2, v2); du [E][3]: dS/du of (w1, v) + (w2, v2), with g.
+ * Attention weights alpha = exp(a - max a) p ih / (sum exp(a - max a) p + 1e-3), a = gate qk, per row and head
+ * (e2former.py:327-364): _fwd also writes the row statistics (maximum, sum, number of maxima), _bwd the gradients
+ * for grad = dL/d alpha, _bwd2 the gradients of sum cgate dgate + cih dih + cqk dqk + cp dp with respect to grad,
+ * gate, ih, qk and p (NULL cotangents are zero).  gate and ih rows have their own strides (they may be the halves of
+ * one [E][256] tensor).
+ * e2v2_add_gather2: out[e, :] = (y[e, :] +) a[ia[e], :] + b[ib[e], :]. */
+typedef struct {
+  int32_t n_rows;
+  int64_t n_edges;
+  const int32_t* row_ptr;
+  const int32_t* col;
+  const int32_t* edge_row;
+  const int32_t* key_ptr;
+  const int32_t* key_eid;
+} e2v2_train_edges;
+int e2v2_so2_agg(const e2v2_train_edges* list, const float* w1, const float* u1, const float* w2, const float* u2,
+                 const float* v, const float* w3, const float* u3, const float* v2, float* out, hipStream_t s);
+int e2v2_so2_agg_dv(const e2v2_train_edges* list, const float* w1, const float* u1, const float* w2, const float* u2,
+                    const float* g, float* dv, hipStream_t s);
+int e2v2_so2_agg_dw(const e2v2_train_edges* list, const float* w1, const float* u1, const float* v, const float* w2,
+                    const float* u2, const float* v2, const float* g, float* dw, float* du, hipStream_t s);
+int e2v2_attn_weights_fwd(const e2v2_train_edges* list, const float* gate, int64_t ld_gate, const float* ih,
+                          int64_t ld_ih, const float* qk, const float* p, float* alpha, float* mrow, float* srow,
+                          float* ties, hipStream_t s);
+int e2v2_attn_weights_bwd(const e2v2_train_edges* list, const float* gate, int64_t ld_gate, const float* ih,
+                          int64_t ld_ih, const float* qk, const float* p, const float* mrow, const float* srow,
+                          const float* ties, const float* grad, float* dgate, int64_t ld_dgate, float* dih,
+                          int64_t ld_dih, float* dqk, float* dp, hipStream_t s);
+int e2v2_attn_weights_bwd2(const e2v2_train_edges* list, const float* gate, int64_t ld_gate, const float* ih,
+                           int64_t ld_ih, const float* qk, const float* p, const float* mrow, const float* srow,
+                           const float* ties, const float* grad, const float* cgate, int64_t ld_cgate,
+                           const float* cih, int64_t ld_cih, const float* cqk, const float* cp, float* fgrad,
+                           float* fgate, int64_t ld_fgate, float* fih, int64_t ld_fih, float* fqk, float* fp,
+                           hipStream_t s);
+int e2v2_add_gather2(const float* y, const float* a, const int32_t* ia, const float* b, const int32_t* ib, int64_t n,
+                     int K, float* out, hipStream_t s);
 /* out[e, :K] = in[index[e], :K] (zero rows for an index outside [0, n_in)): _bwd_alpha_sum_edge_index
    (sparse_alpha_sum_edge_index_autograd.py:70-99). */
 int e2v2_gather_rows(const float* in, int64_t n_in, const int32_t* index, int64_t n, int K, float* out,

@@ -24,6 +24,8 @@ EXPORTS = [
     "e2v2_pairdot_fwd", "e2v2_pairdot_bwd", "e2v2_qk_proj_fwd", "e2v2_qk_proj_bwd",
     "e2v2_qk_proj_fwd_bf16", "e2v2_qk_proj_bwd_bf16",
     "e2v2_segment_metadata", "e2v2_pair_count", "e2v2_pair_emit", "e2v2_seg_dot", "e2v2_seg_reduce",
+    "e2v2_so2_agg", "e2v2_so2_agg_dv", "e2v2_so2_agg_dw", "e2v2_attn_weights_fwd", "e2v2_attn_weights_bwd",
+    "e2v2_attn_weights_bwd2", "e2v2_add_gather2",
     "e2v2_gather_rows", "e2v2_outer_reduce", "e2v2_outer_bwd",
     "e2v2_radial_eval", "e2v2_radial_eval_bwd", "e2v2_sh_contract", "e2v2_sh_contract_bwd",
     "e2v2_gemm_s3", "e2v2_gemm_s3_padded", "e2v2_gemm_s3_grouped", "e2v2_gemm_s3_gated", "e2v2_gemm_pack", "e2v2_gemm_packed_bytes", "e2v2_qk_proj_fwd_s3", "e2v2_qk_proj_bwd_s3",
@@ -49,6 +51,11 @@ class PairPlan(C.Structure):
 class Segments(C.Structure):
     _fields_ = [("row_ptr", vp), ("col_index", vp), ("alpha_index", vp), ("n_rows", i32), ("n_cols", i32),
                 ("n_slots", i64), ("n_edges", i64)]
+
+
+class TrainEdges(C.Structure):
+    _fields_ = [("n_rows", i32), ("n_edges", i64), ("row_ptr", vp), ("col", vp), ("edge_row", vp), ("key_ptr", vp),
+                ("key_eid", vp)]
 
 
 class RadialNet(C.Structure):

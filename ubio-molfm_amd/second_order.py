@@ -24,6 +24,7 @@ Every edge operation still runs on the GPU through libe2v2.so; nothing here
 falls back to the CPU."""
 from __future__ import annotations
 
+import ctypes as C
 import math
 from typing import Optional
 
@@ -246,10 +247,12 @@ def run_seq(mods, h: torch.Tensor) -> torch.Tensor:
 
 
 def _cartesian(device) -> torch.Tensor:
-    """The Cartesian coupling table T [20, 9, 3] of the first-order product."""
+    """The Cartesian coupling table of the first-order product as [20, 27]: column 9 k + r couples value row r with
+    component k of the edge vector."""
     key = str(device)
     if key not in _CART:
-        _CART[key] = torch.as_tensor(np.asarray(so3.cartesian_tp_table(), np.float32), device=device)
+        T = np.asarray(so3.cartesian_tp_table(), np.float32).transpose(0, 2, 1).reshape(-1, 27)
+        _CART[key] = torch.as_tensor(np.ascontiguousarray(T), device=device)
     return _CART[key]
 
 
@@ -438,6 +441,7 @@ class TrainEdges:
         off = (nl.dvec[:E] - base.detach()).detach()
         self.dvec = base + off
         self.dist = self.dvec.norm(dim=-1)
+        self._unit = None
         self.Z = ctx.type_z.long()[ctx.atom_type.long()]
         self.offset, self.coeff = ctx.rbf_offset, float(ctx.rbf_coeff)
         self.env_kind, self.env_lo = ctx.env_kind, ctx.env_lo
@@ -446,6 +450,17 @@ class TrainEdges:
         # (query row_ptr, partner rows, edge ids) then the same by key: the 6-tuple of
         # prepare_sparse_qk_edge_index_metadata for an edge list in row order
         self.md = (nl.row_ptr, self.col32, eid, nl.key_ptr, self.row32.index_select(0, key_eid.long()), key_eid)
+
+    def lists(self):
+        """The list as e2v2_train_edges (pointers of this object's tensors, formed for one call)."""
+        t = (self.nl.row_ptr, self.col32, self.row32, self.nl.key_ptr, self.md[5])
+        return C.byref(_lib.TrainEdges(self.N, self.E, *[x.data_ptr() if x.numel() else None for x in t]))
+
+    def unit_vectors(self) -> torch.Tensor:
+        """dvec / max(dist, 1e-6) [E, 3], formed once for all layers."""
+        if self._unit is None:
+            self._unit = self.dvec / self.dist.clamp_min(1e-6).unsqueeze(-1)
+        return self._unit
 
     def rbf(self) -> torch.Tensor:
         """GaussianSmearing (module_utils.py:1853-1869) of the distances."""
@@ -476,6 +491,16 @@ class TrainEdges:
     def gather_k(self, x: torch.Tensor) -> torch.Tensor:
         """x [N, F] -> x[nj] [E, F] (gradient: the sum over each source atom's edges)."""
         return sparse_ops.sparse_gather_edge_index(x, self.col32, self.N, (self.md[3], self.md[5]))
+
+    def add_gathers(self, y: torch.Tensor, xq: torch.Tensor, xk: torch.Tensor) -> torch.Tensor:
+        """y + xq[qi] + xk[nj], y [E, F], xq and xk [N, F]."""
+        if y.dtype == xq.dtype == xk.dtype == torch.float32 and y.shape[1] % 4 == 0 and y.shape[1] <= 1024:
+            return _AddGathersFn.apply(y, xq, xk, self)
+        return y + self.gather_q(xq) + self.gather_k(xk)
+
+    def col_sum(self, x: torch.Tensor) -> torch.Tensor:
+        """x [E, F] -> the sum over each source atom's edges [N, F]."""
+        return sparse_ops.sparse_alpha_sum_edge_index_triton(x, self.col32, self.N, metadata=(self.md[3], self.md[5]))
 
     def qk(self, q: torch.Tensor, k: torch.Tensor) -> torch.Tensor:
         return sparse_ops.sparse_qk_edge_index_triton(q, k, self.row32, self.col32, metadata=self.md)
@@ -513,8 +538,193 @@ class EdgeInput:
         e = self.edges
         ht = self.tgt(e.Z) @ W[:, K:K + ne].t()                  # [N, hidden] per atom
         hs = self.src(e.Z) @ W[:, K + ne:K + 2 * ne].t()
-        h = _EdgeLinearFn.apply(self.rbf, W[:, :K], lin1.bias) + e.gather_q(ht) + e.gather_k(hs)
+        h = e.add_gathers(_EdgeLinearFn.apply(self.rbf, W[:, :K], lin1.bias), ht, hs)
         return run_seq(net[1:], h)
+
+
+class _AddGathersFn(torch.autograd.Function):
+    """y + xq[qi] + xk[nj] in one pass (e2v2_add_gather2); linear, so its gradient (the identity and the two
+    segment sums) and theirs are this function and sums again."""
+
+    @staticmethod
+    def forward(ctx, y, xq, xk, edges):
+        ctx.edges = edges
+        y = None if y is None else y.contiguous()
+        xq, xk = xq.contiguous(), xk.contiguous()
+        out = xq.new_empty(edges.E, xq.shape[1])
+        _lib.call("e2v2_add_gather2", _p(y), _p(xq), _p(edges.row32), _p(xk), _p(edges.col32), _lib.i64(edges.E),
+                  _lib.i32(xq.shape[1]), _p(out), sparse_ops._stream(xq.device))
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        gq, gk = _EdgeSumsFn.apply(g, ctx.edges)
+        return (g if ctx.needs_input_grad[0] else None), gq, gk, None
+
+
+class _EdgeSumsFn(torch.autograd.Function):
+    """(sum over each query row's edges, sum over each source atom's edges) of g [E, F]."""
+
+    @staticmethod
+    def forward(ctx, g, edges):
+        ctx.edges = edges
+        ctx.set_materialize_grads(False)
+        return edges.row_sum(g), edges.col_sum(g)
+
+    @staticmethod
+    def backward(ctx, cq, ck):
+        e = ctx.edges
+        if cq is None or ck is None:
+            return (None if cq is None and ck is None else e.gather_q(cq) if ck is None else e.gather_k(ck)), None
+        return _AddGathersFn.apply(None, cq, ck, e), None
+
+
+class _AttnWeightsFn(torch.autograd.Function):
+    """alpha [E, 128] of the segmented softmax (e2former.py:327-364) from the gate, the QK dot, the inputhead and the
+    envelope, as one kernel (e2v2_attn_weights_fwd); ``eg`` [E, 256] holds gate and inputhead side by side, or
+    (``gate`` given) the inputhead alone.  The maximum's gradient is split over ties, as scatter_reduce's."""
+
+    @staticmethod
+    def forward(ctx, eg, gate, qk, p, edges):
+        eg, qk, p = eg.contiguous(), qk.contiguous(), p.contiguous()
+        gate = None if gate is None else gate.contiguous()
+        N, E, H = edges.N, edges.E, qk.shape[1]
+        alpha = torch.empty_like(qk)
+        m, s, ties = (qk.new_empty(N, H) for _ in range(3))
+        _lib.call("e2v2_attn_weights_fwd", *_aw_args(edges, eg, gate, qk, p), _p(alpha), _p(m), _p(s), _p(ties),
+                  sparse_ops._stream(qk.device))
+        ctx.save_for_backward(eg, gate, qk, p, m, s, ties)
+        ctx.edges = edges
+        return alpha
+
+    @staticmethod
+    def backward(ctx, g):
+        return (*_AttnWeightsGradFn.apply(g, *ctx.saved_tensors, ctx.edges), None)
+
+
+def _aw_pair(eg, gate):
+    """(gate pointer, row stride, inputhead pointer, row stride) of the two forms of ``eg``; eg None: NULLs."""
+    if gate is not None or eg is None or eg.shape[1] == 128:
+        return _p(gate), _lib.i64(128), _p(eg), _lib.i64(128)
+    return _p(eg), _lib.i64(256), _lib.vp(eg.data_ptr() + 512), _lib.i64(256)
+
+
+def _aw_args(edges, eg, gate, qk, p):
+    return (edges.lists(), *_aw_pair(eg, gate), _p(qk), _p(p))
+
+
+class _AttnWeightsGradFn(torch.autograd.Function):
+    """(d eg, d gate, d qk, dp) of _AttnWeightsFn for dL/d alpha (e2v2_attn_weights_bwd); its own gradient is
+    e2v2_attn_weights_bwd2 (the row statistics enter as constants: the kernel differentiates through them)."""
+
+    @staticmethod
+    def forward(ctx, g, eg, gate, qk, p, m, s, ties, edges):
+        g = g.contiguous()
+        deg, dqk, dp = torch.empty_like(eg), torch.empty_like(qk), torch.empty_like(p)
+        dgate = None if gate is None else torch.empty_like(gate)
+        _lib.call("e2v2_attn_weights_bwd", *_aw_args(edges, eg, gate, qk, p), _p(m), _p(s), _p(ties), _p(g),
+                  *_aw_pair(deg, dgate), _p(dqk), _p(dp), sparse_ops._stream(g.device))
+        ctx.save_for_backward(g, eg, gate, qk, p, m, s, ties)
+        ctx.edges = edges
+        ctx.set_materialize_grads(False)
+        return deg, dgate, dqk, dp
+
+    @staticmethod
+    def backward(ctx, ceg, cgate, cqk, cp):
+        g, eg, gate, qk, p, m, s, ties = ctx.saved_tensors
+        if torch.is_grad_enabled():      # a third order was asked for: the composition, differentiable on
+            # (aliases: a gradient by an operand must not run on through g into what g was formed from)
+            args = [None if t is None else t.view_as(t) for t in (g, eg, gate, qk, p)]
+            g, eg, gate, qk, p = args
+            diff = [t is not None and t.requires_grad for t in args]
+            ins = [t for t, r in zip(args[1:], diff[1:]) if r]
+            cots = [c for c, r in zip((ceg, cgate, cqk, cp), diff[1:]) if r]
+            d = torch.autograd.grad(_softmax_weights(eg, gate, qk, p, ctx.edges), ins, g, create_graph=True)
+            pick = [(x, c) for x, c in zip(d, cots) if c is not None]
+            f = iter(torch.autograd.grad([x for x, _ in pick], [t for t, r in zip(args, diff) if r],
+                                         [c for _, c in pick], create_graph=True, allow_unused=True))
+            return (*(next(f) if r else None for r in diff), None, None, None, None)
+        ceg, cgate, cqk, cp = (None if t is None else t.contiguous() for t in (ceg, cgate, cqk, cp))
+        fg, feg, fqk, fp = torch.empty_like(g), torch.empty_like(eg), torch.empty_like(qk), torch.empty_like(p)
+        fgate = None if gate is None else torch.empty_like(gate)
+        _lib.call("e2v2_attn_weights_bwd2", *_aw_args(ctx.edges, eg, gate, qk, p), _p(m), _p(s), _p(ties), _p(g),
+                  *_aw_pair(ceg, cgate), _p(cqk), _p(cp), _p(fg), *_aw_pair(feg, fgate), _p(fqk), _p(fp),
+                  sparse_ops._stream(g.device))
+        return fg, feg, fgate, fqk, fp, None, None, None, None
+
+
+class _So2AggFn(torch.autograd.Function):
+    """a[k, r, i, c] = sum over the edges of row i of w[e, c % 128] u[e, k] v[r, col_e, c] [3, 9, N, 256]: the value
+    aggregation of the first-order product for the three components of the edge vector at once, each value row
+    gathered once (e2v2_so2_agg)."""
+
+    @staticmethod
+    def forward(ctx, w, u, v, edges):
+        w, u, v = w.contiguous(), u.contiguous(), v.contiguous()
+        ctx.save_for_backward(w, u, v)
+        ctx.edges = edges
+        return _so2_agg(edges, v, ((w, u),))
+
+    @staticmethod
+    def backward(ctx, g):
+        return (*_So2AggGradFn.apply(g, *ctx.saved_tensors, ctx.edges), None)
+
+
+def _so2_agg(edges, v, terms, second=(None, None, None)):
+    """e2v2_so2_agg of sum over terms (w u) v + w3 u3 v2, second = (w3, u3, v2)."""
+    (w1, u1), (w2, u2) = (*terms, (None, None))[:2]
+    out = v.new_empty(3, 9, edges.N, 256)
+    _lib.call("e2v2_so2_agg", edges.lists(), _p(w1), _p(u1), _p(w2), _p(u2), _p(v), *map(_p, second), _p(out),
+              sparse_ops._stream(v.device))
+    return out
+
+
+def _so2_dv(edges, g, terms):
+    (w1, u1), (w2, u2) = (*terms, (None, None))[:2]
+    dv = g.new_empty(9, edges.N, 256)
+    _lib.call("e2v2_so2_agg_dv", edges.lists(), _p(w1), _p(u1), _p(w2), _p(u2), _p(g), _p(dv),
+              sparse_ops._stream(g.device))
+    return dv
+
+
+def _so2_dw(edges, g, w1, u1, v, w2=None, u2=None, v2=None):
+    dw, du = g.new_empty(edges.E, 128), g.new_empty(edges.E, 3)
+    _lib.call("e2v2_so2_agg_dw", edges.lists(), _p(w1), _p(u1), _p(v), _p(w2), _p(u2), _p(v2), _p(g), _p(dw),
+              _p(du), sparse_ops._stream(g.device))
+    return dw, du
+
+
+class _So2AggGradFn(torch.autograd.Function):
+    """(dw, du, dv) of _So2AggFn for the output gradient g.  With S = <g, aggregation(w, u, v)>, linear in each
+    operand, the gradient of <qw, dS/dw> + <qu, dS/du> + <qv, dS/dv> is the same forms with one operand replaced by
+    its cotangent, both terms of each in one pass."""
+
+    @staticmethod
+    def forward(ctx, g, w, u, v, edges):
+        g = g.contiguous()
+        ctx.save_for_backward(g, w, u, v)
+        ctx.edges = edges
+        ctx.set_materialize_grads(False)
+        dw, du = _so2_dw(edges, g, w, u, v)
+        return dw, du, _so2_dv(edges, g, ((w, u),))
+
+    @staticmethod
+    def backward(ctx, qw, qu, qv):
+        g, w, u, v = ctx.saved_tensors
+        e = ctx.edges
+        if torch.is_grad_enabled():      # a third order was asked for: the same sums of differentiable forms
+            qw, qu, qv = (torch.zeros_like(t) if q is None else q for q, t in ((qw, w), (qu, u), (qv, v)))
+            parts = [(qw, u, v), (w, qu, v), (w, u, qv)]
+            dg = sum(_So2AggFn.apply(*t, e) for t in parts)
+            (_, du1, dv1), (dw2, _, dv2), (dw3, du3, _) = (_So2AggGradFn.apply(g, *t, e) for t in parts)
+            return dg, dw2 + dw3, du1 + du3, dv1 + dv2, None
+        qw, qu, qv = (None if t is None else t.contiguous() for t in (qw, qu, qv))
+        terms = ([(qw, u)] if qw is not None else []) + ([(w, qu)] if qu is not None else [])
+        t2 = terms or [(None, None)]
+        dg = _so2_agg(e, v, t2, (w, u, qv) if qv is not None else (None, None, None))
+        dv = _so2_dv(e, g, t2) if terms else None
+        dw, du = _so2_dw(e, g, qw, qu, v, w if qv is not None else None, u if qv is not None else None, qv)
+        return dg, dw, du, dv, None
 
 
 class _RowMaxFn(torch.autograd.Function):
@@ -542,14 +752,29 @@ class _RowMaxFn(torch.autograd.Function):
         return edges.gather_q(g / cnt) * tie, None
 
 
-def attention_weights(logit, p, ih, edges: TrainEdges, form: str) -> torch.Tensor:
+def attention_weights(eg, gate, qk, p, edges: TrainEdges, form: str) -> torch.Tensor:
     """alpha [E, H] (e2former.py:327-364): the segmented softmax with the row
     maximum by scatter_reduce(amax) (its gradient split over ties) and the
-    +1e-3 in the denominator, or the softplus / sigmoid forms."""
-    if form == "softplus":
-        return F.softplus(logit) * ih * p.unsqueeze(-1)
-    if form == "sigmoid":
-        return torch.sigmoid(logit) * ih * p.unsqueeze(-1)
+    +1e-3 in the denominator, or the softplus / sigmoid forms.  eg [E, 2 H]: gate
+    and inputhead side by side; with ``gate`` given, eg [E, H] is the inputhead.
+    fp32 on the GPU with 128 heads takes the softmax through _AttnWeightsFn;
+    other inputs the composition."""
+    H = qk.shape[1]
+    if (form == "softmax" and H == 128 and qk.is_cuda and all(t.dtype == torch.float32 for t in (eg, qk, p))
+            and (gate is None or gate.dtype == torch.float32)):
+        return _AttnWeightsFn.apply(eg, gate, qk, p, edges)
+    if form == "softmax":
+        return _softmax_weights(eg, gate, qk, p, edges)
+    gate, ih = eg.split([H, eg.shape[1] - H], dim=1) if gate is None else (gate, eg)
+    act = F.softplus if form == "softplus" else torch.sigmoid
+    return act(gate * qk) * ih * p.unsqueeze(-1)
+
+
+def _softmax_weights(eg, gate, qk, p, edges) -> torch.Tensor:
+    """The softmax form composed of segment ops (any order of gradients)."""
+    H = qk.shape[1]
+    gate, ih = eg.split([H, eg.shape[1] - H], dim=1) if gate is None else (gate, eg)
+    logit = gate * qk
     amax = _RowMaxFn.apply(logit, edges)
     e = torch.exp(logit - edges.gather_q(amax)) * p.unsqueeze(-1)
     s = edges.row_sum(e)
@@ -609,24 +834,20 @@ def attention(ga, x: torch.Tensor, edges: TrainEdges, rbf: torch.Tensor) -> torc
     k = so3_linear2scalar(ga.key_linear, x).reshape(N, H, -1)
     x_edge = edges.edge_input(ga.target_embedding, ga.source_embedding, rbf)
     if ga.tp_type == "QK_alpha":
-        eg = x_edge(ga.fc_easy)
-        gate, ih = eg.split([H, eg.shape[1] - H], dim=1)
+        gate, eg = None, x_edge(ga.fc_easy)
     else:
-        gate, ih = qkdot_gate(ga, x, edges, x_edge)
+        gate, eg = qkdot_gate(ga, x, edges, x_edge)
     qk = edges.qk(q / math.sqrt(q.shape[-1]), k)
-    alpha = attention_weights(gate * qk, edges.envelope(), ih, edges, ga.weight_act)
+    alpha = attention_weights(eg, gate, qk, edges.envelope(), edges, ga.weight_act)
     alpha = ga.alpha_dropout(alpha)
     v = so3_linear(ga.proj_value, x)                                         # [9, N, C]
     C = v.shape[-1]
-    vh = v.permute(1, 0, 2).reshape(N, -1, H)                                # channel c -> head c mod H
     if ga.attn_type == "zero-order":
+        vh = v.permute(1, 0, 2).reshape(N, -1, H)                            # channel c -> head c mod H
         agg = edges.v_agg(vh, alpha).reshape(N, -1, C).permute(1, 0, 2)      # [9, N, C]
         return so3_linear(ga.proj_zero, agg)
-    T = _cartesian(x.device)
-    so2, u = 0, (edges.dvec / edges.dist.clamp_min(1e-6).unsqueeze(-1)).unbind(1)   # alpha / d * dvec_k
-    for kk in range(3):
-        a = edges.v_agg(vh, alpha * u[kk].unsqueeze(-1)).reshape(N, -1, C)    # [N, 9, C]
-        so2 = so2 + torch.einsum("tr,nrc->tnc", T[:, :, kk], a)
+    a = _So2AggFn.apply(alpha, edges.unit_vectors(), v, edges)                # [3, 9, N, C], alpha / d * dvec_k
+    so2 = torch.mm(_cartesian(x.device), a.view(27, N * C)).view(-1, N, C)
     return so3_linear(ga.proj_first, so2_forward_linear(ga.first_order_tp.so2_tp, so2))
 
 
