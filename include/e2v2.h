@@ -641,6 +641,43 @@ int e2v2_qk_proj_fwd_s3(const float* x, const void* wp, const float* bias, void*
                         int hid, int c, int pieces, int y_bf16, hipStream_t s);
 int e2v2_qk_proj_bwd_s3(const void* y, const float* ghq, const float* ghk, const void* wp, const float* gv,
                         float* gx, int n, int hid, int c, int cv, int pieces, int y_bf16, hipStream_t s);
+
+/* ---- whole layers --------------------------------------------------------- */
+/* One attention layer (e2former.py:223-436: Q/K projection and heads, value projection, attention, SO(2) output
+ * linears) and its input gradient as one call each: the launches of the entry points above in the same order, so
+ * the same results, without the host's work per launch.  Packed weights as for those entry points (one piece: the
+ * bf16 mode, q, k, v, y and the SO(2) rows kept as bf16); out_* per output degree, out_cnt its coupling paths (1 for
+ * all degrees of a zero-order layer), out_start its block in the SO(2) rows (elements per node).  q, k, v of args are
+ * set inside.  saved and scratch: n_rows times the bytes per node of e2v2_attn_layer_bytes, 16-byte aligned; saved is
+ * kept from the forward to the backward; workspace as for e2v2_attn_bwd. */
+typedef struct {
+  int32_t pieces, zero_order, hid, c, heads, n_out;
+  const void* qk_fwd; const void* qk_bwd; const float* qk_bias;
+  const void* v_fwd; const float* v_bias;
+  const void* h1_fwd; const void* h1_bwd; const float* h1_bias;
+  const void* h2_fwd; const void* h2_bwd; const float* h2_bias;
+  const float* ln_g[2]; const float* ln_b[2]; float ln_eps[2];
+  const void* out_fwd[3]; const void* out_bwd[3]; int32_t out_cnt[3]; int32_t out_start[3]; const float* out_bias;
+} e2v2_attn_layer;
+int e2v2_attn_layer_bytes(const e2v2_attn_layer* layer, int64_t* saved, int64_t* fwd, int64_t* bwd);
+int e2v2_attn_layer_fwd(const e2v2_attn_layer* layer, const e2v2_attn_args* args, const float* x, void* saved,
+                        void* scratch, float* out, hipStream_t s);
+int e2v2_attn_layer_bwd(const e2v2_attn_layer* layer, const e2v2_attn_args* args, const float* gout, const void* saved,
+                        void* scratch, void* workspace, size_t workspace_bytes, float* gx, float* ddvec, float* ddist,
+                        hipStream_t s);
+/* The feed-forward block (module_utils.py:2755-2797 with Gate_s3's logits folded into the first linear) likewise:
+ * h [9][n][hidden] and sc [n][3 hidden] are kept for the backward, scratch holds 21 n hidden floats; res may be NULL. */
+typedef struct {
+  int32_t pieces, c, hidden;
+  const void* w1_fwd; const void* w1_bwd; const float* b1;
+  const void* gate_fwd; const void* gate_bwd; const float* gate_b;
+  const void* w2_fwd; const void* w2_bwd; const float* b2;
+  float k1, k2;
+} e2v2_ffn_layer;
+int e2v2_ffn_layer_fwd(const e2v2_ffn_layer* layer, int n, const float* x, const float* res, float* h, float* sc,
+                       float* y, hipStream_t s);
+int e2v2_ffn_layer_bwd(const e2v2_ffn_layer* layer, int n, const float* gout, const float* h, const float* sc,
+                       float* scratch, float* gx, hipStream_t s);
 int e2v2_gemm_pack(const float* w, int64_t ld_n, int64_t ld_k, int64_t w_stride, int n_w, int n, int k, int pieces,
                    void* packed, hipStream_t s);
 

@@ -30,6 +30,7 @@ EXPORTS = [
     "e2v2_radial_eval", "e2v2_radial_eval_bwd", "e2v2_sh_contract", "e2v2_sh_contract_bwd",
     "e2v2_gemm_s3", "e2v2_gemm_s3_padded", "e2v2_gemm_s3_grouped", "e2v2_gemm_s3_gated", "e2v2_gemm_pack", "e2v2_gemm_packed_bytes", "e2v2_qk_proj_fwd_s3", "e2v2_qk_proj_bwd_s3",
     "e2v2_qkdot_gate_fwd", "e2v2_qkdot_gate_bwd", "e2v2_qkdot_gate_bwd_workspace",
+    "e2v2_attn_layer_bytes", "e2v2_attn_layer_fwd", "e2v2_attn_layer_bwd", "e2v2_ffn_layer_fwd", "e2v2_ffn_layer_bwd",
 ]
 
 
@@ -99,6 +100,27 @@ class GemmArgs(C.Structure):
                 ("r", vp), ("ldr", i64), ("r_bs", i64), ("bias", vp), ("bias_bs", i64), ("bias_batches", i32),
                 ("m", i32), ("n", i32), ("k", i32), ("batch", i32), ("widx", i32 * 16), ("pieces", i32),
                 ("a_bf16", i32), ("c_bf16", i32)]
+
+
+class AttnLayer(C.Structure):
+    _fields_ = [("pieces", i32), ("zero_order", i32), ("hid", i32), ("c", i32), ("heads", i32), ("n_out", i32),
+                ("qk_fwd", vp), ("qk_bwd", vp), ("qk_bias", vp), ("v_fwd", vp), ("v_bias", vp),
+                ("h1_fwd", vp), ("h1_bwd", vp), ("h1_bias", vp), ("h2_fwd", vp), ("h2_bwd", vp), ("h2_bias", vp),
+                ("ln_g", vp * 2), ("ln_b", vp * 2), ("ln_eps", f32 * 2), ("out_fwd", vp * 3), ("out_bwd", vp * 3),
+                ("out_cnt", i32 * 3), ("out_start", i32 * 3), ("out_bias", vp)]
+
+
+class FfnLayer(C.Structure):
+    _fields_ = [("pieces", i32), ("c", i32), ("hidden", i32), ("w1_fwd", vp), ("w1_bwd", vp), ("b1", vp),
+                ("gate_fwd", vp), ("gate_bwd", vp), ("gate_b", vp), ("w2_fwd", vp), ("w2_bwd", vp), ("b2", vp),
+                ("k1", f32), ("k2", f32)]
+
+
+def stream(device=None):
+    """The current HIP stream of a device (None: the current device) as a call argument."""
+    import torch
+    idx = None if device is None else torch.device(device).index
+    return vp(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx))
 
 
 _lib = None

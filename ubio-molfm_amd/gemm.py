@@ -69,7 +69,7 @@ def pack(w: torch.Tensor, transpose: bool = False, pieces: int = 3) -> PackedWei
     buf = torch.empty(nbytes // 2, dtype=torch.bfloat16, device=w.device)
     _lib.call("e2v2_gemm_pack", _lib.vp(w.data_ptr()), _lib.i64(ld_n), _lib.i64(ld_k), _lib.i64(w.stride(0)),
               _lib.i32(n_w), _lib.i32(n), _lib.i32(k), _lib.i32(pieces), _lib.vp(buf.data_ptr()),
-              _lib.vp(torch.cuda.current_stream(w.device).cuda_stream))
+              _lib.stream(w.device))
     return PackedWeight(buf, n_w, n, k, pieces)
 
 
@@ -156,7 +156,7 @@ def gemm(a, pw: PackedWeight, out: torch.Tensor, widx: Optional[Sequence[int]] =
     g, work, keep = _args(a, pw, out, widx, bias, bias_batches, res)   # keep: referenced until the launch
     if g is None:
         return out
-    st = _lib.vp(torch.cuda.current_stream(out.device).cuda_stream)
+    st = _lib.stream(out.device)
     if padded_rows and gate is not None:
         raise ValueError("gemm: padded_rows does not combine with a gate")
     entry = "e2v2_gemm_s3_gated" if gate is not None else "e2v2_gemm_s3_padded" if padded_rows else "e2v2_gemm_s3"
@@ -202,7 +202,7 @@ def gemm_grouped(problems):
             n += 1
             work += w
     if n:
-        _lib.call("e2v2_gemm_s3_grouped", arr, _lib.i32(n), _lib.vp(torch.cuda.current_stream(dev).cuda_stream))
+        _lib.call("e2v2_gemm_s3_grouped", arr, _lib.i32(n), _lib.stream(dev))
         if _lib._timer is not None:
             _lib._timer.add_work("e2v2_gemm_s3_grouped", work)
     del keep
@@ -277,7 +277,7 @@ def qk_forward(x: torch.Tensor, P: QKPacks, y_bf16: Optional[bool] = None):
     y = x.new_empty(9, n, 4 * P.hid, dtype=torch.bfloat16 if y_bf16 else torch.float32)
     hq = x.new_empty(n, 3 * P.hid)
     hk = x.new_empty(n, 3 * P.hid)
-    st = _lib.vp(torch.cuda.current_stream(x.device).cuda_stream)
+    st = _lib.stream(x.device)
     _lib.call("e2v2_qk_proj_fwd_s3", _lib.vp(x.data_ptr()), _lib.vp(P.fwd.buf.data_ptr()),
               _lib.vp(0 if P.bias is None else P.bias.data_ptr()), _lib.vp(y.data_ptr()), _lib.vp(hq.data_ptr()),
               _lib.vp(hk.data_ptr()), _lib.i32(n), _lib.i32(P.hid), _lib.i32(c), _lib.i32(P.fwd.pieces),
@@ -293,7 +293,7 @@ def qk_backward(y: torch.Tensor, ghq: torch.Tensor, ghk: torch.Tensor, gv: Optio
     y_bf16 = y.dtype == torch.bfloat16
     ghq, ghk = ghq.contiguous(), ghk.contiguous()
     gv = None if gv is None else gv.float().contiguous()
-    st = _lib.vp(torch.cuda.current_stream(y.device).cuda_stream)
+    st = _lib.stream(y.device)
     _lib.call("e2v2_qk_proj_bwd_s3", _lib.vp(y.data_ptr()), _lib.vp(ghq.data_ptr()), _lib.vp(ghk.data_ptr()),
               _lib.vp(P.bwd.buf.data_ptr()), _lib.vp(0 if gv is None else gv.data_ptr()), _lib.vp(gx.data_ptr()),
               _lib.i32(n), _lib.i32(P.hid), _lib.i32(P.c), _lib.i32(P.cv), _lib.i32(P.bwd.pieces),

@@ -13,6 +13,7 @@
 """
 from __future__ import annotations
 
+import contextlib
 import weakref
 from types import SimpleNamespace
 from typing import Dict, Optional
@@ -61,7 +62,7 @@ def spatial_order(pos: torch.Tensor, graph_ptr) -> torch.Tensor:
     key = torch.empty(N, dtype=torch.int64, device=pos.device)
     _lib.call("e2v2_morton_keys", _lib.vp(pos.data_ptr()), None if gid is None else _lib.vp(gid.data_ptr()),
               _lib.vp(lo.data_ptr()), _lib.vp(span.data_ptr()), _lib.i32(N), _lib.vp(key.data_ptr()),
-              _lib.vp(torch.cuda.current_stream(pos.device).cuda_stream))
+              _lib.stream(pos.device))
     return torch.sort(key, stable=True).indices
 
 
@@ -267,6 +268,12 @@ def neighbor_info(nl, perm: Optional[torch.Tensor], pos: torch.Tensor, graph_ptr
             "f_exp_node_pos": exp_pos, "f_outcell_index": out_j}
 
 
+def _backward_here(on: bool = True):
+    """A backward pass on the calling thread (each node on its forward's stream, as on the engine's own threads): the
+    pass is one device's, and handing it to another Python thread and back costs 0.1 to 1 ms."""
+    return torch.autograd.set_multithreading_enabled(False) if on else contextlib.nullcontext()
+
+
 class MLP_energy_head(nn.Module):
     """head.py:330-341."""
 
@@ -284,7 +291,8 @@ class GradientHead(nn.Module):
     (the backbone then runs its twice-differentiable training path)."""
 
     def forward(self, pos, pred_energy):
-        return -torch.autograd.grad(pred_energy, pos, torch.ones_like(pred_energy), create_graph=self.training)[0]
+        with _backward_here(not self.training):
+            return -torch.autograd.grad(pred_energy, pos, torch.ones_like(pred_energy), create_graph=self.training)[0]
 
 
 class MDEnergyForceMultiHead(nn.Module):
@@ -349,7 +357,8 @@ class MolfmAtomic(nn.Module):
         if self.training:   # forces that can be differentiated again (the training path)
             forces = -torch.autograd.grad(energy, pos, torch.ones_like(energy), create_graph=True)[0]
             return energy, forces, nl
-        forces = -torch.autograd.grad(energy, pos, torch.ones_like(energy))[0]
+        with _backward_here():
+            forces = -torch.autograd.grad(energy, pos, torch.ones_like(energy))[0]
         return energy.detach(), forces, nl
 
     def forward(self, batched_data, need_force=True, **unused):

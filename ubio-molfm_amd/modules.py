@@ -11,6 +11,7 @@ selects hipBLASLt's fp32 GEMMs instead of the split ones (a measurement switch).
 """
 from __future__ import annotations
 
+import contextlib
 import math
 import os
 from typing import Optional
@@ -18,13 +19,34 @@ from typing import Optional
 import numpy as np
 import torch
 from torch import nn
-from torch.profiler import record_function
+from torch.profiler import record_function as _record_function
 
 from . import so3
 from . import _lib
 from . import gemm as s3gemm
 from .ops import AttentionFn, DegreeEmbedFn, QKdotGateFn, RadialCache, RadialEvalFn, ShContractFn, \
-    attention_backward, attention_forward
+    _no_double_backward, attention_backward, attention_forward, attn_args, module_params
+
+_NO_RANGE = contextlib.nullcontext()
+
+
+def record_function(name: str):
+    """The profiler range ``name`` while a profiler runs (entering and leaving one costs 10 us of host time
+    with none running)."""
+    return _record_function(name) if torch.autograd._profiler_enabled() else _NO_RANGE
+
+
+# Layers of at most this many nodes are enqueued by one native call each way (e2v2_attn_layer_*, e2v2_ffn_layer_*):
+# an evaluation of four layers takes 2.0 ms instead of 4.6 ms at 24 atoms and 3.2 ms instead of 5.1 ms at 648, with
+# 1.5 and 3.1 ms of kernels.  The GPU, not the host, sets the time from some 1500 nodes on (10,000: 25.8 ms either
+# way), and beyond the limit the launch by launch path frees each intermediate after its last reader.
+LAYER_ROWS = 8192
+
+
+def _layer_call(n: int) -> bool:
+    """Whether a layer of n nodes runs as one native call (never while kernels are timed or a profiler runs: their
+    names and ranges are those of the single launches)."""
+    return 0 < n <= LAYER_ROWS and _lib._timer is None and not torch.autograd._profiler_enabled()
 
 
 def _e3nn_normalize2mom(f) -> float:
@@ -52,7 +74,7 @@ def split_gemm_on() -> bool:
 
 
 def _stream():
-    return _lib.vp(torch.cuda.current_stream().cuda_stream)
+    return _lib.stream()
 
 
 def _dp(t):
@@ -672,6 +694,76 @@ class AttnBlockBF16Fn(torch.autograd.Function):
         return (gx, ddv, dd, dgate) + (None,) * 12
 
 
+class AttnLayer:
+    """The packed weights of one attention layer as e2v2_attn_layer: ``struct`` and what its pointers refer to."""
+    __slots__ = ("struct", "keep", "saved", "fwd", "bwd", "zero")
+
+    def __init__(self, s3, P, Wvop, bv, Wc, out_bias, zero: bool):
+        a = _lib.AttnLayer()
+        vf = Wvop.s3f()
+        a.pieces, a.zero_order, a.hid, a.c, a.heads, a.n_out = s3.fwd.pieces, int(zero), s3.hid, s3.c, 128, P["p2f"].n
+        a.qk_fwd, a.qk_bwd, a.qk_bias = s3.fwd.buf.data_ptr(), s3.bwd.buf.data_ptr(), s3.bias.data_ptr()
+        a.v_fwd, a.v_bias = vf.buf.data_ptr(), bv.data_ptr()
+        a.h1_fwd, a.h1_bwd, a.h1_bias = P["p1f"].buf.data_ptr(), P["p1b"].buf.data_ptr(), P["b1"].data_ptr()
+        a.h2_fwd, a.h2_bwd, a.h2_bias = P["p2f"].buf.data_ptr(), P["p2b"].buf.data_ptr(), P["b2"].data_ptr()
+        for b, (g, be, eps) in enumerate(P["ln"]):
+            a.ln_g[b], a.ln_b[b], a.ln_eps[b] = g.data_ptr(), be.data_ptr(), eps
+        for l, cnt, start, _, _, pf, pb in Wc:
+            a.out_fwd[l], a.out_bwd[l] = pf.buf.data_ptr(), pb.buf.data_ptr()
+            a.out_cnt[l], a.out_start[l] = cnt, start
+        a.out_bias = out_bias.data_ptr()
+        self.struct, self.keep, self.zero = a, (s3, P, vf, bv, [e[5:] for e in Wc], out_bias), zero
+        n = [_lib.i64() for _ in range(3)]
+        _lib.call("e2v2_attn_layer_bytes", _lib.C.byref(a), *(_lib.C.byref(v) for v in n))
+        self.saved, self.fwd, self.bwd = (v.value for v in n)
+
+
+class AttnLayerFn(torch.autograd.Function):
+    """A whole attention layer, x [9, N, 256] -> [9, N, 256], in one native call each way (e2v2_attn_layer_fwd /
+    _bwd): the launches of AttnProjS3Fn, AttentionFn and SO2OutFn (of AttnBlockBF16Fn in the bf16 mode) with the
+    same operands.  What those keep for the backward lies in one buffer [N, bytes].  Inputs with gradients: x,
+    dvec, dist and the external gate."""
+
+    @staticmethod
+    def forward(ctx, x, dvec, dist, ext_gate, layer: AttnLayer, nl, atom_type, table, rc: float, q_div: float, env,
+                weight_act: str):
+        x = x.contiguous()
+        N, dev = x.shape[1], x.device
+        if ext_gate is not None:
+            ext_gate = ext_gate.float().contiguous()
+        args = attn_args(nl, None, None, None, atom_type, table, q_div, rc, layer.struct.pieces == 1, layer.zero, env,
+                         ext_gate, weight_act=weight_act)
+        saved = torch.empty(N, layer.saved, dtype=torch.uint8, device=dev)
+        scratch = torch.empty(N, layer.fwd, dtype=torch.uint8, device=dev)
+        out = torch.empty(9, N, 256, dtype=torch.float32, device=dev)
+        _lib.call("e2v2_attn_layer_fwd", _lib.C.byref(layer.struct), _lib.C.byref(args), _dp(x), _dp(saved),
+                  _dp(scratch), _dp(out), _lib.stream(dev))
+        ctx.save_for_backward(saved, ext_gate)
+        ctx.layer, ctx.nl, ctx.atom_type, ctx.table = layer, nl, atom_type, table
+        ctx.rc, ctx.q_div, ctx.env, ctx.weight_act = rc, q_div, env, weight_act
+        return out
+
+    @staticmethod
+    def backward(ctx, gout):
+        _no_double_backward()
+        saved, ext_gate = ctx.saved_tensors
+        layer, nl = ctx.layer, ctx.nl
+        gout = gout.contiguous()
+        N, E, dev = gout.shape[1], nl.n_edges, gout.device
+        f = dict(dtype=torch.float32, device=dev)
+        dgate = None if ext_gate is None else torch.empty(E, 128, **f)
+        args = attn_args(nl, None, None, None, ctx.atom_type, ctx.table, ctx.q_div, ctx.rc, layer.struct.pieces == 1,
+                         layer.zero, ctx.env, ext_gate, dgate, ctx.weight_act)
+        gx = torch.empty(9, N, 256, **f)
+        ddv, dd = torch.empty(max(E, 1), 3, **f), torch.empty(max(E, 1), **f)
+        scratch = torch.empty(N, layer.bwd, dtype=torch.uint8, device=dev)
+        nb = int(_lib.load().e2v2_attn_bwd_workspace(E))
+        ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
+        _lib.call("e2v2_attn_layer_bwd", _lib.C.byref(layer.struct), _lib.C.byref(args), _dp(gout), _dp(saved),
+                  _dp(scratch), _dp(ws), _lib.C.c_size_t(ws.numel()), _dp(gx), _dp(ddv), _dp(dd), _lib.stream(dev))
+        return (gx, ddv[:E], dd[:E], dgate) + (None,) * 8
+
+
 def head_pair_packs(fq: nn.Sequential, fk: nn.Sequential, owner, bf16: bool = False):
     """Operands of QKHeadsS3Fn for two final_linear stacks (Linear, LayerNorm,
     SiLU, Linear) of the same shapes: each Linear's two weights stacked and packed
@@ -1005,6 +1097,46 @@ class FFNS3Fn(torch.autograd.Function):
         return gx, None, None, None, None, None, None, None, None, (gout if ctx.has_res else None)
 
 
+class FFNLayer:
+    """The packed weights of one feed-forward block as e2v2_ffn_layer: ``struct`` and what its pointers refer to."""
+    __slots__ = ("struct", "keep")
+
+    def __init__(self, W1op, b1, fold: GateFold, W2op, b2):
+        self.keep = (W1op.s3f(), W1op.s3b(), fold.f, fold.bk, W2op.s3f(), W2op.s3b(), b1, fold.b, b2)
+        w1, w1b, f, fb, w2, w2b = (p.buf.data_ptr() for p in self.keep[:6])
+        self.struct = _lib.FfnLayer(W1op.pieces, 256, 256, w1, w1b, b1.data_ptr(), f, fb, fold.b.data_ptr(), w2, w2b,
+                                    b2.data_ptr(), SILU_NORM, SIGMOID_NORM)
+
+
+class FFNLayerFn(torch.autograd.Function):
+    """FFNS3Fn at 256 channels in one native call each way (e2v2_ffn_layer_fwd / _bwd): the same launches with the
+    same operands."""
+
+    @staticmethod
+    def forward(ctx, x, layer: FFNLayer, res=None):
+        x = x.contiguous()
+        res = None if res is None else res.contiguous()
+        N, dev = x.shape[1], x.device
+        f32 = dict(dtype=torch.float32, device=dev)
+        h, sc, y = torch.empty(9, N, 256, **f32), torch.empty(N, 768, **f32), torch.empty(9, N, 256, **f32)
+        _lib.call("e2v2_ffn_layer_fwd", _lib.C.byref(layer.struct), _lib.i32(N), _dp(x),
+                  None if res is None else _dp(res), _dp(h), _dp(sc), _dp(y), _lib.stream(dev))
+        ctx.save_for_backward(sc, h)
+        ctx.layer, ctx.has_res = layer, res is not None
+        return y
+
+    @staticmethod
+    def backward(ctx, gout):
+        sc, h = ctx.saved_tensors
+        gout = gout.contiguous()
+        N, dev = h.shape[1], h.device
+        gx = torch.empty(9, N, 256, dtype=torch.float32, device=dev)
+        scratch = torch.empty(21, N, 256, dtype=torch.float32, device=dev)
+        _lib.call("e2v2_ffn_layer_bwd", _lib.C.byref(ctx.layer.struct), _lib.i32(N), _dp(gout), _dp(h), _dp(sc),
+                  _dp(scratch), _dp(gx), _lib.stream(dev))
+        return gx, None, (gout if ctx.has_res else None)
+
+
 class FeedForwardNetwork_s3(nn.Module):
     """module_utils.py:2755-2797."""
 
@@ -1014,7 +1146,33 @@ class FeedForwardNetwork_s3(nn.Module):
         self.gate = Gate_s3(hidden_channels, lmax=lmax)
         self.slinear_2 = SO3_Linear_e2former(hidden_channels, output_channels, lmax=lmax, bias=True)
 
+    def _layer(self, bf16: bool):
+        """This block as an FFNLayer (cached on its weights), or None where the launch by launch path is the one
+        that applies."""
+        if not (bf16 or split_gemm_on()):
+            return None
+
+        def build():
+            s1, s2, g = self.slinear_1, self.slinear_2, self.gate.gates
+            shapes = [(3, 256, 256)] * 2 + [(768, 256)] + [(256,)] * 2 + [(768,)]
+            ws = (s1.weight, s2.weight, g.weight, s1.bias, s2.bias, g.bias)
+            if ((s1.lmax, s2.lmax, self.gate.lmax) != (2, 2, 2) or not all(
+                    w.shape == sh and w.dtype == torch.float32 and w.is_contiguous() for w, sh in zip(ws, shapes))):
+                return None
+            W1op, W2op = (mrow_weight(m, "weight", m.weight, bf16, 2) for m in (s1, s2))
+            if not (W1op.split_ok() and W2op.split_ok()) or dense_packs(g, bf16) is None:
+                return None
+            return FFNLayer(W1op, s1.bias.detach(), GateFold(g.weight, g.bias, s1.weight[0], s1.bias, W1op.pieces),
+                            W2op, s2.bias.detach())
+        return cached(self, "layer_bf16" if bf16 else "layer", module_params(self), build)
+
     def forward(self, x, res=None, bf16: bool = False, **kw):
+        if (x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.shape[0] == 9 and x.shape[2] == 256
+                and _layer_call(x.shape[1]) and (res is None or (res.shape == x.shape and res.device == x.device
+                                                                 and res.dtype == torch.float32))):
+            layer = self._layer(bf16)
+            if layer is not None:
+                return FFNLayerFn.apply(x, layer, res)
         with record_function("FeedForwardFunction"):
             s1, s2, g = self.slinear_1, self.slinear_2, self.gate.gates
             W1op = mrow_weight(s1, "weight", s1.weight, bf16, s1.lmax)
@@ -1106,9 +1264,9 @@ class SO2_TP_givenl2(nn.Module):
             def build_sliced():
                 P = slice_perm(self.path_norm.device)
                 return [[(t0, nr, Wt[P].contiguous()) for (t0, nr, Wt) in lst] for lst in self.folded_blocks(bf16)]
-            return cached(self, "fold_sl_bf16" if bf16 else "fold_sl", list(self.parameters()), build_sliced)
+            return cached(self, "fold_sl_bf16" if bf16 else "fold_sl", module_params(self), build_sliced)
         if bf16:
-            return cached(self, "fold_bf16", list(self.parameters()),
+            return cached(self, "fold_bf16", module_params(self),
                           lambda: [[(t0, nr, Wt.to(BF16).contiguous()) for (t0, nr, Wt) in lst]
                                    for lst in self.folded_blocks()])
         key = tuple((p.data_ptr(), p._version) for p in self.parameters())
@@ -1461,7 +1619,7 @@ class E2AttentionArbOrder_sparse(nn.Module):
             w = torch.cat([torch.zeros(H, w3.shape[1], device=w3.device), w3[:H]])
             b = torch.cat([torch.zeros(H, device=b3.device), b3[:H]])
             return _profile_with_rows(net, w, b)
-        return cached(self, "attn_profile", list(self.fc_easy.parameters()), build)
+        return cached(self, "attn_profile", module_params(self.fc_easy), build)
 
     def _m0_profiles(self):
         """Nets of the per-edge radial profile of the QKdot gate, 256 channels each:
@@ -1474,7 +1632,7 @@ class E2AttentionArbOrder_sparse(nn.Module):
                 w3, b3 = net[6].weight.detach(), net[6].bias.detach()
                 return [_profile_with_rows(net, w3[256 * m:256 * (m + 1)], b3[256 * m:256 * (m + 1)])
                         for m in range(w3.shape[0] // 256)]
-            return cached(self, "m0_profiles", list(self.rad_func_m0.parameters()), build)
+            return cached(self, "m0_profiles", module_params(self.rad_func_m0), build)
         net = self.fc_easy.net
 
         def build_s():
@@ -1483,7 +1641,7 @@ class E2AttentionArbOrder_sparse(nn.Module):
             w = torch.cat([w3[H:], torch.zeros(256 - H, w3.shape[1], device=w3.device)])
             b = torch.cat([b3[H:], torch.zeros(256 - H, device=b3.device)])
             return [_profile_with_rows(net, w, b)]
-        return cached(self, "m0_profiles", list(self.fc_easy.parameters()), build_s)
+        return cached(self, "m0_profiles", module_params(self.fc_easy), build_s)
 
     def qkdot_gate(self, x: torch.Tensor, ctx: EdgeContext) -> torch.Tensor:
         """The gate [E, H] of the QKdot variants in the edge order of ctx.nl, from
@@ -1546,7 +1704,7 @@ class E2AttentionArbOrder_sparse(nn.Module):
         Cached on the parameters' versions."""
         tp = self.first_order_tp.so2_tp
         pf = self.proj_first
-        params = list(tp.parameters()) + [pf.weight]
+        params = module_params(tp) + [pf.weight]
 
         def build():
             out = []
@@ -1560,6 +1718,40 @@ class E2AttentionArbOrder_sparse(nn.Module):
         key = "so2_out_bf16" if bf16 else ("so2_out_s3" if split_gemm_on() else "so2_out")
         return cached(self, key, params, build)
 
+    def _table(self, ctx: EdgeContext):
+        """The distance table of fc_easy for ctx's atom types (built once per weight version)."""
+        return self._radial.get([self._attn_profile()], self.target_embedding, self.source_embedding,
+                                ctx.rbf_offset, ctx.rbf_coeff, ctx.rc, ctx.type_z, ctx.type_key, layout="attn",
+                                pairs=ctx.pairs)
+
+    def _layer(self, bf16: bool):
+        """This layer as an AttnLayer (cached on every weight it packs), or None where the launch by launch path is
+        the one that applies."""
+        if not (bf16 or split_gemm_on()):
+            return None
+        zero = self.attn_type == "zero-order"
+        m = self._modules
+        params = module_params(m["query_linear"]) + module_params(m["key_linear"]) + module_params(m["proj_value"])
+        for name in ("proj_zero",) if zero else ("proj_first", "first_order_tp"):
+            params += module_params(m[name])
+
+        def build():
+            pv = self.proj_value
+            out = self.proj_zero if zero else self.proj_first
+            s3, P = self.qk_s3_packs(bf16), self.qk_head_packs(bf16)
+            wv, bv = self.value_weights_sliced()
+            Wvop = mrow_weight(pv, "weight_sl", wv, bf16, pv.lmax)
+            Wc = self.zero_out_weights(bf16) if zero else self.so2_out_weights(bf16)
+            ob = out.bias.detach()
+            if (s3 is None or P is None or not Wvop.split_ok() or any(e[5] is None or e[6] is None for e in Wc)
+                    or s3.bias is None or (s3.c, s3.cv, P["p2f"].n, P["p1f"].k) != (256, 256, 1024, 3 * s3.hid)
+                    or P["p1f"].n != s3.hid or [e[0] for e in Wc] != [0, 1, 2]
+                    or any((e[5].k, e[5].n) != (256 * e[1], 256) for e in Wc)
+                    or any(b.dtype != torch.float32 or b.shape != (256,) or not b.is_contiguous() for b in (bv, ob))):
+                return None
+            return AttnLayer(s3, P, Wvop, bv, Wc, ob, zero)
+        return cached(self, "layer_bf16" if bf16 else "layer", params, build)
+
     def forward_fused(self, x: torch.Tensor, ctx: EdgeContext, res: Optional[torch.Tensor] = None):
         """x [9, N, C] (m-major) -> attention(x) (+ res when given), [9, N, C].
         v, the attention rows and their gradients run in the kernels' slice order
@@ -1570,6 +1762,15 @@ class E2AttentionArbOrder_sparse(nn.Module):
         if self.training and self.alpha_dropout.p > 0:
             raise NotImplementedError("attention dropout in training mode is not supported by the HIP path")
         bf16 = ctx.bf16
+        if (res is None and x.is_cuda and x.dtype == torch.float32 and x.shape == (9, ctx.nl.n_atoms, 256)
+                and H == 128 and ctx.dvec.is_cuda and ctx.dist.is_cuda and _layer_call(N)):
+            layer = self._layer(bf16)
+            if layer is not None:
+                table = self._table(ctx)
+                gate = None if self.tp_type == "QK_alpha" else self.qkdot_gate(x, ctx)
+                return AttnLayerFn.apply(x, ctx.dvec, ctx.dist, gate, layer, ctx.nl, ctx.atom_type, table, ctx.rc,
+                                         math.sqrt(self.attn_scalar_head), (ctx.env_kind, ctx.env_lo),
+                                         self.weight_act)
         W, b = self.qk_weights(bf16)
         hid = self.query_linear.weight.shape[1]
         pv = self.proj_value  # its GEMMs run inside QKProjFn (one input gradient)
@@ -1594,9 +1795,7 @@ class E2AttentionArbOrder_sparse(nn.Module):
                 q = self.query_linear.head(hq, bf16).reshape(N, H, -1)
                 k = self.key_linear.head(hk, bf16).reshape(N, H, -1)
         with record_function("rbf function-a"):   # fc_easy as a distance table, built once per weight version
-            table = self._radial.get([self._attn_profile()], self.target_embedding, self.source_embedding,
-                                     ctx.rbf_offset, ctx.rbf_coeff, ctx.rc, ctx.type_z, ctx.type_key, layout="attn",
-                                     pairs=ctx.pairs)
+            table = self._table(ctx)
         zero = self.attn_type == "zero-order"
         with record_function("qk attention"):
             gate = None if self.tp_type == "QK_alpha" else self.qkdot_gate(x, ctx)

@@ -251,7 +251,7 @@ def build_neighbors(pos: torch.Tensor, graph_ptr, cells, pbcs, rc: float, rmin: 
     cells = np.asarray(cells, F32).reshape(-1, 3, 3)
     pbcs = np.asarray(pbcs, bool).reshape(-1, 3)
     N = int(pos.shape[0])
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _lib.stream(dev).value
     i32 = dict(dtype=torch.int32, device=dev)
     plan, keep, shifts_np, sptr = make_plan(pos, graph_ptr, cells, pbcs, rc, rmin, cells_per_direction, grid_box,
                                             src_include=src_include)
@@ -347,7 +347,7 @@ def cluster_slots(seg_ptr: torch.Tensor, n_seg: int, member: torch.Tensor, item_
     ns = torch.empty(max((n_seg + span - 1) // span, 1), **i32)
     _lib.call("e2v2_cluster_slots", _lib.vp(seg_ptr.data_ptr()), _lib.i32(n_seg), _lib.vp(member.data_ptr()),
               _lib.vp(_ptr(item_eid)), _lib.i32(span), _lib.vp(sm.data_ptr()), _lib.vp(se.data_ptr()),
-              _lib.vp(ns.data_ptr()), _lib.vp(torch.cuda.current_stream(dev).cuda_stream))
+              _lib.vp(ns.data_ptr()), _lib.stream(dev))
     return sm, se, ns
 
 
@@ -369,7 +369,7 @@ def count_neighbors_noalloc(pos: torch.Tensor, graph_ptr, cells, pbcs, rc: float
     stats = torch.empty(3, **i32)
     _lib.call("e2v2_nbr_count_noalloc", _lib.C.byref(plan), _lib.vp(row_count.data_ptr()),
               _lib.vp(row_ptr.data_ptr()), _lib.vp(stats.data_ptr()),
-              _lib.vp(torch.cuda.current_stream(pos.device).cuda_stream))
+              _lib.stream(pos.device))
     return row_count[:N], row_ptr, stats
 
 
@@ -430,7 +430,7 @@ def construct_radius_neighbor(node_pos, node_mask, expand_node_pos, expand_node_
         inc = include_mask.to(torch.bool).reshape(B, L2).to(torch.uint8).contiguous()
     plan = _lib.PairPlan(N, B, L2, n_flat, float(max_dist), float(min_dist), 0 if poly == "poly" else 1,
                          _vp(qpos), _vp(qgraph), _vp(spos), _vp(inc), _vp(sbase), _vp(sflat))
-    stream = _lib.vp(torch.cuda.current_stream(dev).cuda_stream)
+    stream = _lib.stream(dev)
     i32 = dict(dtype=torch.int32, device=dev)
     row_count = torch.empty(N, **i32)
     row_ptr = torch.empty(N + 1, **i32)
@@ -502,7 +502,7 @@ def neighbor_list_from_edges(row_ptr: torch.Tensor, src_atom: torch.Tensor, dvec
         if lo < 0 or hi >= N or p0 != 0 or pe != E or bad:
             raise ValueError(f"edge list: source atoms in [{lo}, {hi}] for {N} atoms, row_ptr from {p0} to {pe} "
                              f"for {E} edges, {bad} decreasing steps")
-    stream = _lib.vp(torch.cuda.current_stream(dev).cuda_stream)
+    stream = _lib.stream(dev)
     stats = torch.zeros(3, **i32)
     edge_row = torch.empty(E, **i32)
     key_cnt = torch.empty(max(N, 1), **i32)

@@ -49,7 +49,7 @@ def so2_grouped(rows: torch.Tensor) -> torch.Tensor:
 
 
 def _stream(t: torch.Tensor):
-    return _lib.vp(torch.cuda.current_stream(t.device).cuda_stream)
+    return _lib.stream(t.device)
 
 
 def _p(t: Optional[torch.Tensor]):
@@ -209,8 +209,21 @@ MAX_TYPES = 256
 MAX_PAIRS = 65535
 
 
+def module_params(mod: nn.Module, out=None) -> list:
+    """The parameters of a module tree, read from the modules' own dictionaries
+    (``nn.Module.parameters`` walks the names too, ten times the time)."""
+    out = [] if out is None else out
+    for p in mod._parameters.values():
+        if p is not None:
+            out.append(p)
+    for m in mod._modules.values():
+        if m is not None:
+            module_params(m, out)
+    return out
+
+
 def _version_key(params):
-    return tuple((p.data_ptr(), p._version, p.dtype, str(p.device)) for p in params)
+    return tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in params)
 
 
 class RadialCache:
@@ -224,7 +237,7 @@ class RadialCache:
     def get(self, nets, tgt_emb: nn.Embedding, src_emb: nn.Embedding, rbf_offset: torch.Tensor, rbf_coeff: float,
             rc: float, type_z: torch.Tensor, type_key: tuple, layout: str = "plain", pairs=None):
         """type_key: the host key of the type set (and of ``pairs``, the table's type pairs)."""
-        params = [p for n in nets for p in n.parameters()] + [tgt_emb.weight, src_emb.weight, rbf_offset]
+        params = [p for n in nets for p in module_params(n)] + [tgt_emb.weight, src_emb.weight, rbf_offset]
         key = (_version_key(params), float(rbf_coeff), float(rc), type_key, pairs, layout)
         if key != self.key:
             self.table = None
@@ -335,6 +348,7 @@ WEIGHT_ACTS = {"softmax": 0, "softplus": 1, "sigmoid": 2}
 def attn_args(nl: NeighborList, q, k, v, atom_type, table: RadialTable, q_div: float, rc: float, bf: int,
               zero_order: bool = False, env=(0, 0.0), ext_gate=None, ext_dgate=None, weight_act: str = "softmax"):
     """e2v2_attn_args over the neighbour list (with its column clusters when built).
+    q, k, v None: set by the callee (e2v2_attn_layer_fwd / _bwd).
     zero_order selects the zero-order aggregation; env = (kind, lower end): kind 0
     the polynomial envelope on [0, rc], 1 the smooth bell on [lower end, rc];
     ext_gate [E, 128] fp32 (or None) replaces the table's gate rows, ext_dgate
@@ -347,8 +361,9 @@ def attn_args(nl: NeighborList, q, k, v, atom_type, table: RadialTable, q_div: f
         raise ValueError("the attention needs the table of its fc_easy profile in slice order (layout 'attn')")
     a = _lib.AttnArgs(nl.n_atoms, nl.n_edges, 128, 8, 256, nl.row_ptr.data_ptr(), nl.col.data_ptr(),
                       nl.edge_row.data_ptr(), nl.key_ptr.data_ptr(), nl.key_eid.data_ptr(), nl.dvec.data_ptr(),
-                      nl.dist.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), table.tab.data_ptr(),
-                      atom_type.data_ptr(), table.n_types, table.n_nodes, table.h, float(q_div), float(rc), ENV_A,
+                      nl.dist.data_ptr(), *((None,) * 3 if q is None else (q.data_ptr(), k.data_ptr(), v.data_ptr())),
+                      table.tab.data_ptr(), atom_type.data_ptr(), table.n_types, table.n_nodes, table.h, float(q_div),
+                      float(rc), ENV_A,
                       ENV_B, ENV_C, int(bf))
     a.zero_order = int(bool(zero_order))
     a.env_kind, a.env_lo = int(env[0]), float(env[1])

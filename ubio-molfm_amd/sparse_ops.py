@@ -42,7 +42,7 @@ def _vp(t: Optional[torch.Tensor]):
 
 
 def _stream(dev):
-    return _lib.vp(torch.cuda.current_stream(dev).cuda_stream)
+    return _lib.stream(dev)
 
 
 def _strides(t: torch.Tensor):
