@@ -254,6 +254,21 @@ int e2v2_attn_weights_bwd2(const e2v2_train_edges* list, const float* gate, int6
                            hipStream_t s);
 int e2v2_add_gather2(const float* y, const float* a, const int32_t* ia, const float* b, const int32_t* ib, int64_t n,
                      int K, float* out, hipStream_t s);
+/* The m-contraction of SO3_Linear2Scalar (module_utils.py:2241-2266) on a, b [9][n][hid] and its adjoint:
+ * h[i][l hid + c] = sum_{m in l} a[m][i][c] b[m][i][c]; y[m][i][c] = h[i][l(m) hid + c] b[m][i][c] (hid a multiple
+ * of 4). */
+int e2v2_mdot(const float* a, const float* b, int n, int hid, float* h, hipStream_t s);
+int e2v2_mexpand(const float* h, const float* b, int n, int hid, float* y, hipStream_t s);
+/* e2v2_wgrad: dW[g] [m][k] = sum over the batches bounds[g] .. bounds[g + 1] - 1 and the n rows of a batch of
+ * a[b][r][:m]^T b[b][r][:k], fp32 (m and k multiples of 64; batches and rows may be strided): the weight gradient of
+ * SO3_Linear_e2former (module_utils.py:2010-2052), its 9 m-rows in 3 groups.  part holds
+ * batches * e2v2_wgrad_chunks(n, batches, m, k) * m * k floats.  bounds: groups + 1 host integers from 0 to batches.
+ * e2v2_sum_parts: out[g][:w] = the sum of the rows of part[g] [rows][w] (w a multiple of 4). */
+#define E2V2_MAX_PART_GROUPS 4
+int e2v2_wgrad_chunks(int n, int batches, int m, int k);
+int e2v2_wgrad(const float* a, int64_t lda, int64_t a_bs, const float* b, int64_t ldb, int64_t b_bs, int n, int batches,
+               int m, int k, const int32_t* bounds, int groups, float* part, float* out, hipStream_t s);
+int e2v2_sum_parts(const float* part, int groups, int rows, int w, float* out, hipStream_t s);
 /* out[e, :K] = in[index[e], :K] (zero rows for an index outside [0, n_in)): _bwd_alpha_sum_edge_index
    (sparse_alpha_sum_edge_index_autograd.py:70-99). */
 int e2v2_gather_rows(const float* in, int64_t n_in, const int32_t* index, int64_t n, int K, float* out,

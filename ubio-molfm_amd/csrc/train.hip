@@ -527,6 +527,40 @@ int check_lists(const e2v2_train_edges* L, const char* who) {
   E2V2_REQUIRE(L->n_edges == 0 || (L->col && L->edge_row && L->key_eid), "%s: null edge arrays", who);
   return 0;
 }
+// The m-contraction of SO3_Linear2Scalar (module_utils.py:2241-2266) on separate operands a, b [9][n][hid]:
+// h[i][l hid + c] = the sum over the rows m of degree l of a[m][i][c] b[m][i][c], and its adjoint
+// y[m][i][c] = h[i][l hid + c] b[m][i][c].  Each is the other's derivative, so two passes over the operands serve
+// every order; composed (product, splits, sums, concatenation, expansions) a layer's double backward took some
+// fifty.  Bound by memory: the expansion takes 6.2 us at 1500 nodes
+// of 512 (55 MB, mostly in the Infinity Cache).
+__global__ __launch_bounds__(256) void k_mdot(const float* __restrict__ a, const float* __restrict__ b, int n, int hid,
+                                              float* __restrict__ h) {
+  const int q = hid / 4;
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= (int64_t)n * q) return;
+  const int64_t i = t / q, c = 4 * (t % q), step = (int64_t)n * hid, o = i * hid + c;
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    float4 s = mul4(ld4(a + l * l * step + o), ld4(b + l * l * step + o));
+#pragma unroll
+    for (int m = l * l + 1; m < (l + 1) * (l + 1); ++m) s = fma4(ld4(a + m * step + o), ld4(b + m * step + o), s);
+    st4(h + (i * 3 + l) * hid + c, s);
+  }
+}
+__global__ __launch_bounds__(256) void k_mexpand(const float* __restrict__ h, const float* __restrict__ b, int n,
+                                                 int hid, float* __restrict__ y) {
+  const int q = hid / 4;
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= (int64_t)n * q) return;
+  const int64_t i = t / q, c = 4 * (t % q), step = (int64_t)n * hid, o = i * hid + c;
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    const float4 w = ld4(h + (i * 3 + l) * hid + c);
+#pragma unroll
+    for (int m = l * l; m < (l + 1) * (l + 1); ++m) st4(y + m * step + o, mul4(w, ld4(b + m * step + o)));
+  }
+}
+
 }  // namespace
 }  // namespace e2v2
 
@@ -652,5 +686,28 @@ E2V2_API int e2v2_add_gather2(const float* y, const float* a, const int32_t* ia,
   const int per = 256 / (K / 4) * kAgU;
   hipLaunchKernelGGL(k_add_gather2, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, s, y, a, ia, b, ib, n, K, out);
   E2V2_LAUNCHED("k_add_gather2");
+  return 0;
+}
+
+static int check_mdot(const void* x, const void* y, const void* z, int n, int hid, const char* who) {
+  E2V2_REQUIRE(n > 0 && hid > 0 && hid % 4 == 0 && (int64_t)n * hid < (1LL << 36), "%s: n %d, hid %d", who, n, hid);
+  E2V2_REQUIRE(x && y && z && ((uintptr_t)x | (uintptr_t)y | (uintptr_t)z) % 16 == 0,
+               "%s: operands must be 16-byte aligned", who);
+  return 0;
+}
+
+E2V2_API int e2v2_mdot(const float* a, const float* b, int n, int hid, float* h, hipStream_t s) {
+  if (int rc = check_mdot(a, b, h, n, hid, "mdot")) return rc;
+  const int64_t t = (int64_t)n * (hid / 4);
+  hipLaunchKernelGGL(k_mdot, dim3((uint32_t)((t + 255) / 256)), dim3(256), 0, s, a, b, n, hid, h);
+  E2V2_LAUNCHED("k_mdot");
+  return 0;
+}
+
+E2V2_API int e2v2_mexpand(const float* h, const float* b, int n, int hid, float* y, hipStream_t s) {
+  if (int rc = check_mdot(h, b, y, n, hid, "mexpand")) return rc;
+  const int64_t t = (int64_t)n * (hid / 4);
+  hipLaunchKernelGGL(k_mexpand, dim3((uint32_t)((t + 255) / 256)), dim3(256), 0, s, h, b, n, hid, y);
+  E2V2_LAUNCHED("k_mexpand");
   return 0;
 }

@@ -76,6 +76,15 @@ def _ln_parts(n: int) -> int:
     return max(1, min((n + 3) // 4, 2048))
 
 
+def _sum_parts(part: torch.Tensor) -> torch.Tensor:
+    """part [groups, rows, w] summed over its rows, [groups, w] (e2v2_sum_parts)."""
+    g, rows, w = part.shape
+    out = part.new_empty(g, w)
+    _lib.call("e2v2_sum_parts", _p(part), _lib.i32(g), _lib.i32(rows), _lib.i32(w), _p(out),
+              sparse_ops._stream(part.device))
+    return out
+
+
 class _LNSiLUFn(torch.autograd.Function):
     """silu(LayerNorm(x) * g + b) on rows x [n, w] (a RadialProfile's nn.LayerNorm +
     nn.SiLU, module_utils.py:2151-2178) through e2v2_ln_silu_fwd; its backward is
@@ -111,12 +120,12 @@ class _LNSiLUGradFn(torch.autograd.Function):
         n, w = x.shape
         npart = _ln_parts(n)
         gx = torch.empty_like(x)
-        pg, pb = x.new_empty(npart, w), x.new_empty(npart, w)
-        _lib.call("e2v2_ln_silu_bwd_param", _p(x), _p(g), _p(b), _p(st), _p(gy), _p(gx), _p(pg), _p(pb),
+        part = x.new_empty(2, npart, w)
+        _lib.call("e2v2_ln_silu_bwd_param", _p(x), _p(g), _p(b), _p(st), _p(gy), _p(gx), _p(part[0]), _p(part[1]),
                   _lib.i32(n), _lib.i32(w), _lib.i32(npart), sparse_ops._stream(x.device))
         ctx.save_for_backward(gy, x, g, b, st)
         ctx.set_materialize_grads(False)
-        return gx, pg.sum(0), pb.sum(0)
+        return (gx, *_sum_parts(part).unbind(0))
 
     @staticmethod
     def backward(ctx, qx, qg, qb):
@@ -127,10 +136,10 @@ class _LNSiLUGradFn(torch.autograd.Function):
         qg = None if qg is None else qg.contiguous()
         qb = None if qb is None else qb.contiguous()
         dgy, dx = torch.empty_like(x), torch.empty_like(x)
-        pg, pb = x.new_empty(npart, w), x.new_empty(npart, w)
+        part = x.new_empty(2, npart, w)
         _lib.call("e2v2_ln_silu_bwd2", _p(x), _p(g), _p(b), _p(st), _p(gy), _p(qx), _p(qg), _p(qb), _p(dgy),
-                  _p(dx), _p(pg), _p(pb), _lib.i32(n), _lib.i32(w), _lib.i32(npart), sparse_ops._stream(x.device))
-        return dgy, dx, pg.sum(0), pb.sum(0), None
+                  _p(dx), _p(part[0]), _p(part[1]), _lib.i32(n), _lib.i32(w), _lib.i32(npart), sparse_ops._stream(x.device))
+        return (dgy, dx, *_sum_parts(part).unbind(0), None)
 
 
 _EDGE_ROWS = 16384   # rows from which a Linear takes the split-K weight gradient
@@ -258,22 +267,133 @@ def _cartesian(device) -> torch.Tensor:
 
 # --------------------------------------------------------------------------- per-node layers (m-major [9, N, C])
 
+_DEGREE_ROWS = (0, 1, 4, 9)      # bounds of the m-rows of each degree
+
+
+class _DegreeMmFn(torch.autograd.Function):
+    """y [9, N, O] with y[m] = x[m] W_l(m)^T, W [3, O, K] (``t``: x[m] W_l(m), W [3, K, O]), the bias added to row 0;
+    We is W with its rows expanded to the m-rows.  Gradients of any order: the input gradient is this function with
+    the other orientation, the weight gradient _DegreeWGradFn, skipped when the running backward does not need it."""
+
+    @staticmethod
+    def forward(ctx, x, W, bias, We, t: bool):
+        y = torch.bmm(x, We if t else We.transpose(1, 2))
+        if bias is not None:
+            y[0].add_(bias)
+        ctx.save_for_backward(x, W, We)
+        ctx.t, ctx.has_b = t, bias is not None
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        x, W, We = ctx.saved_tensors
+        nxt = ctx.next_functions
+        gx = _DegreeMmFn.apply(gy, W, None, We, not ctx.t) if ctx.needs_input_grad[0] and _will_run(nxt[0][0]) else None
+        gW = None
+        if ctx.needs_input_grad[1] and _will_run(nxt[1][0]):
+            gW = _DegreeWGradFn.apply(*((x, gy) if ctx.t else (gy, x)))
+        gb = gy[0].sum(0) if ctx.has_b and ctx.needs_input_grad[2] and _will_run(nxt[2][0]) else None
+        return gx, gW, gb, None, None
+
+
+class _DegreeWGradFn(torch.autograd.Function):
+    """dW [3, O, K] = per degree the sum over its m-rows and the nodes of a[m]^T b[m], a [9, N, O], b [9, N, K]
+    (e2v2_wgrad); gradients b Q^T and a Q."""
+
+    @staticmethod
+    def forward(ctx, a, b):
+        a, b = a.contiguous(), b.contiguous()
+        ctx.save_for_backward(a, b)
+        M, n, m = a.shape
+        k = b.shape[2]
+        chunks = int(_lib.load().e2v2_wgrad_chunks(n, M, m, k))
+        part = a.new_empty(M * chunks, m, k)
+        out = a.new_empty(len(_DEGREE_ROWS) - 1, m, k)
+        bounds = (C.c_int32 * len(_DEGREE_ROWS))(*_DEGREE_ROWS)
+        _lib.call("e2v2_wgrad", _p(a), _lib.i64(m), _lib.i64(n * m), _p(b), _lib.i64(k), _lib.i64(n * k), _lib.i32(n),
+                  _lib.i32(M), _lib.i32(m), _lib.i32(k), bounds, _lib.i32(len(_DEGREE_ROWS) - 1), _p(part), _p(out),
+                  sparse_ops._stream(a.device))
+        return out
+
+    @staticmethod
+    def backward(ctx, Q):
+        a, b = ctx.saved_tensors
+        Qe = Q.detach().index_select(0, _expand(2, Q.device))
+        ga = _DegreeMmFn.apply(b, Q, None, Qe, False) if ctx.needs_input_grad[0] else None
+        gb = _DegreeMmFn.apply(a, Q, None, Qe, True) if ctx.needs_input_grad[1] else None
+        return ga, gb
+
+
+def _degree_mm_ok(x: torch.Tensor, W: torch.Tensor) -> bool:
+    """Whether _DegreeMmFn takes x[m] W_l(m)^T: fp32 on the GPU, three degrees, widths of whole 64-column tiles of
+    the weight gradient's kernel and rows within its 32-bit offsets; other inputs run the composition."""
+    return (x.is_cuda and x.dtype == W.dtype == torch.float32 and x.dim() == W.dim() == 3 and x.shape[0] == 9
+            and W.shape[0] == 3 and 0 < x.shape[1] and (x.shape[1] + 64) * max(W.shape[1:]) < 2 ** 29
+            and W.shape[1] % 64 == 0 and W.shape[2] % 64 == 0 and x.shape[2] == W.shape[2]
+            and not torch.is_autocast_enabled())
+
+
+def _degree_mm(x: torch.Tensor, W: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """x[m] W_l(m)^T (+ bias on row 0), x [9, N, K], W [3, O, K]."""
+    e = _expand(math.isqrt(x.shape[0]) - 1, x.device)
+    if _degree_mm_ok(x, W):
+        return _DegreeMmFn.apply(x.contiguous(), W, bias, W.detach().index_select(0, e), False)
+    out = torch.matmul(x, W.index_select(0, e).transpose(1, 2))
+    return out if bias is None else out + _row0(out.shape[0], out) * bias
+
+
 def so3_linear(mod, x: torch.Tensor) -> torch.Tensor:
     """SO3_Linear_e2former (module_utils.py:2010-2052): row m times W_l(m)^T, the
     bias on row 0."""
-    w = mod.weight.index_select(0, _expand(mod.lmax, x.device))          # [9, Cout, Cin]
-    out = torch.matmul(x, w.transpose(1, 2))
-    return out + _row0(out.shape[0], out) * mod.bias.reshape(-1)
+    return _degree_mm(x, mod.weight, mod.bias.reshape(-1))
+
+
+class _MDotFn(torch.autograd.Function):
+    """The m-contraction h [N, 3 hid] of a, b [9, N, hid] (e2v2_mdot); gradients _MExpandFn."""
+
+    @staticmethod
+    def forward(ctx, a, b):
+        a, b = a.contiguous(), b.contiguous()
+        ctx.save_for_backward(a, b)
+        h = a.new_empty(a.shape[1], 3 * a.shape[2])
+        _lib.call("e2v2_mdot", _p(a), _p(b), _lib.i32(a.shape[1]), _lib.i32(a.shape[2]), _p(h),
+                  sparse_ops._stream(a.device))
+        return h
+
+    @staticmethod
+    def backward(ctx, g):
+        a, b = ctx.saved_tensors
+        return (_MExpandFn.apply(g, b) if ctx.needs_input_grad[0] else None,
+                _MExpandFn.apply(g, a) if ctx.needs_input_grad[1] else None)
+
+
+class _MExpandFn(torch.autograd.Function):
+    """y [9, N, hid] with row m = h's degree block of m times b[m] (e2v2_mexpand); gradients _MDotFn and itself."""
+
+    @staticmethod
+    def forward(ctx, h, b):
+        h, b = h.contiguous(), b.contiguous()
+        ctx.save_for_backward(h, b)
+        y = torch.empty_like(b)
+        _lib.call("e2v2_mexpand", _p(h), _p(b), _lib.i32(b.shape[1]), _lib.i32(b.shape[2]), _p(y),
+                  sparse_ops._stream(b.device))
+        return y
+
+    @staticmethod
+    def backward(ctx, g):
+        h, b = ctx.saved_tensors
+        return (_MDotFn.apply(g, b) if ctx.needs_input_grad[0] else None,
+                _MExpandFn.apply(h, g) if ctx.needs_input_grad[1] else None)
 
 
 def so3_linear2scalar(mod, x: torch.Tensor) -> torch.Tensor:
     """SO3_Linear2Scalar_e2former (module_utils.py:2198-2272): two SO(3) linears
     (the bias on the first one's row 0), their m-contraction per degree, then
     final_linear."""
-    e = _expand(mod.lmax, x.device)
-    a = torch.matmul(x, mod.weight.index_select(0, e).transpose(1, 2))
-    a = a + _row0(a.shape[0], a) * mod.bias.reshape(-1)
-    b = torch.matmul(x, mod.weight2.index_select(0, e).transpose(1, 2))
+    a = _degree_mm(x, mod.weight, mod.bias.reshape(-1))
+    b = _degree_mm(x, mod.weight2, None)
+    if a.is_cuda and a.dtype == b.dtype == torch.float32 and a.shape[0] == 9 and a.shape[1] and a.shape[2] % 4 == 0:
+        return run_seq(mod.final_linear, _MDotFn.apply(a, b))
     ab = (a * b).split([2 * l + 1 for l in range(mod.lmax + 1)], dim=0)
     return run_seq(mod.final_linear, torch.cat([p.sum(0) for p in ab], dim=-1))
 
@@ -320,8 +440,8 @@ class _RMSNormGradFn(torch.autograd.Function):
         ctx.save_for_backward(gy, x, w)
         ctx.eps = eps
         ctx.set_materialize_grads(False)
-        p = part.sum(0)
-        return gx, p[:3].contiguous(), p[3].contiguous()
+        p = _sum_parts(part.view(1, npart, -1)).view(part.shape[1:])
+        return gx, p[:3], p[3]
 
     @staticmethod
     def backward(ctx, qx, qw, qb):
@@ -335,7 +455,7 @@ class _RMSNormGradFn(torch.autograd.Function):
         part = x.new_empty(npart, 3, x.shape[2])
         _lib.call("e2v2_rmsnorm_bwd2", _p(x), _p(w), _p(gy), _p(qx), _p(qw), _p(qb), _p(dgy), _p(dx), _p(part),
                   _lib.i32(n), _lib.i32(npart), _lib.f32(ctx.eps), sparse_ops._stream(x.device))
-        return dgy, dx, part.sum(0), None
+        return dgy, dx, _sum_parts(part.view(1, npart, -1)).view(w.shape), None
 
 
 def rms_norm(mod, x: torch.Tensor) -> torch.Tensor:
@@ -441,8 +561,9 @@ class TrainEdges:
         off = (nl.dvec[:E] - base.detach()).detach()
         self.dvec = base + off
         self.dist = self.dvec.norm(dim=-1)
-        self._unit = None
-        self.Z = ctx.type_z.long()[ctx.atom_type.long()]
+        self._unit = self._env = None
+        self.type_z, self.atom_type = ctx.type_z.long(), ctx.atom_type.long()
+        self._hot = None
         self.offset, self.coeff = ctx.rbf_offset, float(ctx.rbf_coeff)
         self.env_kind, self.env_lo = ctx.env_kind, ctx.env_lo
         eid = torch.arange(E, dtype=torch.int32, device=pos.device)
@@ -456,6 +577,15 @@ class TrainEdges:
         t = (self.nl.row_ptr, self.col32, self.row32, self.nl.key_ptr, self.md[5])
         return C.byref(_lib.TrainEdges(self.N, self.E, *[x.data_ptr() if x.numel() else None for x in t]))
 
+    def type_rows(self, dtype) -> torch.Tensor:
+        """[N, T] selecting each atom's type: a product with it expands per-type rows to the atoms, and its
+        transpose sums their gradients (an embedding's gradient walks the atoms of a type one by one: 110 us a
+        profile for 1500 atoms), formed once for all layers."""
+        if self._hot is None or self._hot.dtype != dtype:
+            types = torch.arange(self.type_z.numel(), device=self.type_z.device)
+            self._hot = (self.atom_type[:self.N].view(-1, 1) == types).to(dtype)
+        return self._hot
+
     def unit_vectors(self) -> torch.Tensor:
         """dvec / max(dist, 1e-6) [E, 3], formed once for all layers."""
         if self._unit is None:
@@ -467,6 +597,12 @@ class TrainEdges:
         return torch.exp(self.coeff * (self.dist.view(-1, 1) - self.offset.view(1, -1)).pow(2))
 
     def envelope(self) -> torch.Tensor:
+        """The envelope of every edge [E], formed once for all layers."""
+        if self._env is None:
+            self._env = self._envelope()
+        return self._env
+
+    def _envelope(self) -> torch.Tensor:
         """polynomial(d, rc) (module_utils.py:1946-1954) or, for the long-range
         list of with_cluster "node_bell", smooth_polynomial_bell(d, lo, rc)
         (module_utils.py:1956-1985)."""
@@ -522,8 +658,8 @@ class TrainEdges:
 class EdgeInput:
     """x_edge = [rbf(d), tgt[z_i], src[z_j]] as the input of RadialProfile nets
     (module_utils.py:2151-2178) without the [E, 256 + 2 n_emb] tensor: the first
-    Linear's type blocks act on the embedding rows per atom and are gathered per edge,
-    W x_edge + b = W_rbf rbf + (tgt[Z] W_t^T)[i] + (src[Z] W_s^T)[j] + b (the same sum,
+    Linear's type blocks act on the embedding rows per type and are gathered per edge,
+    W x_edge + b = W_rbf rbf + (tgt W_t^T)[Z_i] + (src W_s^T)[Z_j] + b (the same sum,
     fp32 rounding of another association); the rest of the net follows unchanged, so
     every parameter (the embeddings included) keeps its gradients to any order."""
 
@@ -536,8 +672,9 @@ class EdgeInput:
         K, ne = self.rbf.shape[1], self.tgt.weight.shape[1]
         W = lin1.weight
         e = self.edges
-        ht = self.tgt(e.Z) @ W[:, K:K + ne].t()                  # [N, hidden] per atom
-        hs = self.src(e.Z) @ W[:, K + ne:K + 2 * ne].t()
+        hot = e.type_rows(W.dtype)                               # per type, then per atom [N, hidden]
+        ht = hot @ (self.tgt(e.type_z) @ W[:, K:K + ne].t())
+        hs = hot @ (self.src(e.type_z) @ W[:, K + ne:K + 2 * ne].t())
         h = e.add_gathers(_EdgeLinearFn.apply(self.rbf, W[:, :K], lin1.bias), ht, hs)
         return run_seq(net[1:], h)
 
