@@ -122,6 +122,10 @@ int e2v2_nbr_topk(const int32_t* row_ptr, int n_rows, int k, int32_t* cnt, int32
 #define E2V2_NOALLOC_MAX_BINS (1 << 20)
 int e2v2_nbr_count_noalloc(const e2v2_nbr_plan* plan, int32_t* row_count, int32_t* row_ptr, int32_t* stats_out,
                            hipStream_t s);
+/* Coordinate bounds of pos [n][3]: out[0..2] the minimum, out[3..5] the maximum (NaN if a coordinate is); part holds
+ * E2V2_BOUND_PARTS * 6 floats. */
+#define E2V2_BOUND_PARTS 256
+int e2v2_bounds(const float* pos, int n, float* part, float* out, hipStream_t s);
 /* 30-bit Morton (Z-order) keys of atoms within their graph's bounding box, for the spatial
    ordering of the rows: key[i] = g << 32 | interleave(q) with q = clamp((pos - lo[g]) / span[g]
    * 1023, 0, 1023) truncated; gid [n] the graph of each atom (NULL: one graph), lo/span [B][3].

@@ -58,3 +58,16 @@ def test_cluster_slots_at_the_merge_limit(pkg, cuda, per_segment, shuffled):
         assert ns[c] == len(keys)
         assert [int(x) for x in sm[b:b + len(keys)]] == [k[0] for k in keys]
         assert se[b:b + len(keys)].tolist() == [want[k] for k in keys]
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 256, 257, 65536, 99999])
+def test_coordinate_bounds(pkg, cuda, n):
+    """Exactly the smallest and largest coordinates; NaN where one is, infinities kept."""
+    from ubio_molfm_amd.neighbors import coordinate_bounds
+    pos = (torch.randn(n, 3, generator=torch.Generator().manual_seed(n)) * 50).to(cuda)
+    b = coordinate_bounds(pos)
+    assert torch.equal(b[0], pos.amin(0)) and torch.equal(b[1], pos.amax(0))
+    pos[n // 2, 1], pos[n - 1, 2] = float("nan"), float("-inf")
+    b = coordinate_bounds(pos)
+    assert bool(b[:, 1].isnan().all()) and float(b[0, 2]) == float("-inf")
+    assert torch.equal(b[:, 0], torch.stack([pos[:, 0].amin(), pos[:, 0].amax()]))

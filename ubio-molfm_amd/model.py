@@ -25,14 +25,14 @@ from torch import nn
 from . import _lib
 from . import second_order
 from .modules import E2former, EdgeContext, atom_type_slots, parse_irreps
-from .neighbors import build_neighbors
+from .neighbors import build_neighbors, coordinate_bounds
 from .ops import EdgeGeometryFn
 
 
 def graph_bounds(pos: torch.Tensor, counts: torch.Tensor):
     """Per-graph coordinate minimum and maximum [B, 3] (graphs contiguous)."""
     if counts.shape[0] == 1:
-        return pos.amin(0, keepdim=True), pos.amax(0, keepdim=True)
+        return coordinate_bounds(pos).split(1)
     lo = torch.segment_reduce(pos, "min", lengths=counts, axis=0, unsafe=True)
     hi = torch.segment_reduce(pos, "max", lengths=counts, axis=0, unsafe=True)
     return lo, hi
@@ -51,7 +51,7 @@ def spatial_order(pos: torch.Tensor, graph_ptr) -> torch.Tensor:
     pos = pos.detach().float().contiguous()
     gid = None
     if B == 1:   # no host copies or syncs for a single graph
-        lo, hi = pos.amin(0, keepdim=True), pos.amax(0, keepdim=True)
+        lo, hi = coordinate_bounds(pos).split(1)
     else:
         counts = torch.as_tensor(counts_np, device=pos.device)
         gid = torch.repeat_interleave(torch.arange(B, device=pos.device, dtype=torch.int32), counts,

@@ -169,6 +169,15 @@ def _plan_tables(dev, graph_ptr, cells, pbcs, rc, cells_per_direction, bb):
     return out
 
 
+def coordinate_bounds(pos: torch.Tensor) -> torch.Tensor:
+    """Minimum (row 0) and maximum (row 1) of the coordinates of one graph, [2, 3] (NaN where a coordinate is)."""
+    pos = pos.detach().float().contiguous()
+    out = torch.empty(2, 3, dtype=torch.float32, device=pos.device)
+    part = torch.empty(256, 6, dtype=torch.float32, device=pos.device)
+    _lib.call("e2v2_bounds", _vp(pos), _lib.i32(pos.shape[0]), _vp(part), _vp(out), _lib.stream(pos.device))
+    return out
+
+
 def make_plan(pos: torch.Tensor, graph_ptr, cells, pbcs, rc: float, rmin: float = 1e-4,
               cells_per_direction: int = 4, grid_box=None, workspace: bool = True,
               src_include: Optional[torch.Tensor] = None):
@@ -191,12 +200,12 @@ def make_plan(pos: torch.Tensor, graph_ptr, cells, pbcs, rc: float, rmin: float 
         bb = np.asarray(grid_box, F32).reshape(2, B, 3)
     elif N:
         if B == 1:
-            lo, hi = pos.amin(0, keepdim=True), pos.amax(0, keepdim=True)
+            bb = coordinate_bounds(pos).cpu().numpy().reshape(2, 1, 3)
         else:
             counts = torch.as_tensor(np.diff(graph_ptr), device=dev)
             lo = torch.segment_reduce(pos, "min", lengths=counts, axis=0, unsafe=True)
             hi = torch.segment_reduce(pos, "max", lengths=counts, axis=0, unsafe=True)
-        bb = torch.stack([lo, hi]).cpu().numpy()
+            bb = torch.stack([lo, hi]).cpu().numpy()
     else:
         bb = np.zeros((2, B, 3), F32)
     tabs = _plan_tables(dev, graph_ptr, cells, pbcs, rc, cells_per_direction, bb)
