@@ -391,6 +391,11 @@ int e2v2_sh_contract(const float* Y, const float* xn, const int32_t* row_ptr, in
 /* Its backward for the gradient g [E][3][C]: dY [E][9], dxn [9][n_rows][C] (per-row sums, no atomics). */
 int e2v2_sh_contract_bwd(const float* Y, const float* xn, const int32_t* row_ptr, int32_t n_rows, int32_t C,
                          const float* g, float* dY, float* dxn, hipStream_t s);
+/* Spherical harmonics l <= 2 of the vectors v [n][3], Y [n][9]: the raw polynomials (unit 0, e3nn's
+   _spherical_harmonics of v itself) or e3nn's normalize=True, "integral" ones (unit 1); and dL/dv [n][3] from
+   g = dL/dY. */
+int e2v2_edge_sh(const float* v, int64_t n, int unit, float* Y, hipStream_t s);
+int e2v2_edge_sh_bwd(const float* v, const float* g, int64_t n, int unit, float* gv, hipStream_t s);
 
 /* ---- attention --------------------------------------------------------- */
 /* Channel order of v, out, grad_out, dv and of the fc_easy table rows ("slice order"): position p of a

@@ -29,7 +29,7 @@ EXPORTS = [
     "e2v2_mdot", "e2v2_mexpand", "e2v2_wgrad_chunks", "e2v2_wgrad", "e2v2_sum_parts",
     "e2v2_gather_rows", "e2v2_outer_reduce", "e2v2_outer_bwd",
     "e2v2_radial_eval", "e2v2_radial_eval_bwd", "e2v2_sh_contract", "e2v2_sh_contract_bwd",
-    "e2v2_bounds",
+    "e2v2_bounds", "e2v2_edge_sh", "e2v2_edge_sh_bwd",
     "e2v2_gemm_s3", "e2v2_gemm_s3_padded", "e2v2_gemm_s3_grouped", "e2v2_gemm_s3_gated", "e2v2_gemm_pack", "e2v2_gemm_packed_bytes", "e2v2_qk_proj_fwd_s3", "e2v2_qk_proj_bwd_s3",
     "e2v2_qkdot_gate_fwd", "e2v2_qkdot_gate_bwd", "e2v2_qkdot_gate_bwd_workspace",
     "e2v2_attn_layer_bytes", "e2v2_attn_layer_fwd", "e2v2_attn_layer_bwd", "e2v2_ffn_layer_fwd", "e2v2_ffn_layer_bwd",

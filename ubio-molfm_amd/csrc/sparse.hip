@@ -985,6 +985,77 @@ E2V2_API int e2v2_outer_bwd(const float* grad, int n_rows, const float* sh, cons
   return 0;
 }
 
+// Raw real spherical-harmonic polynomials l <= 2 of each vector v [n][3] (y the polar axis), or with `unit` those of
+// v / |v| times sqrt(2 l + 1) / sqrt(4 pi), and the vectors' gradient.  As tensor operations these were some ninety
+// launches of 3 us per evaluation (each a pass over [n] columns of [n][9]); a vector per thread is two launches.
+constexpr float kS3 = 1.7320508075688772f;
+__device__ __constant__ const float kShInt[3] = {0.28209479177387814f, 0.4886025119029199f, 0.6307831305050401f};
+
+__global__ __launch_bounds__(256) void k_edge_sh(const float* __restrict__ v, int64_t n, int unit, float* __restrict__ Y) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  float x = v[3 * e], y = v[3 * e + 1], z = v[3 * e + 2];
+  float c0 = 1.f, c1 = 1.f, c2 = 1.f;
+  if (unit) {
+    const float d = sqrtf(x * x + y * y + z * z);
+    x /= d; y /= d; z /= d;
+    c0 = kShInt[0]; c1 = kShInt[1]; c2 = kShInt[2];
+  }
+  float* o = Y + 9 * e;
+  o[0] = c0;
+  o[1] = c1 * x;
+  o[2] = c1 * y;
+  o[3] = c1 * z;
+  o[4] = c2 * (kS3 * x * z);
+  o[5] = c2 * (kS3 * x * y);
+  o[6] = c2 * (y * y - 0.5f * (x * x + z * z));
+  o[7] = c2 * (kS3 * y * z);
+  o[8] = c2 * (0.5f * kS3 * (z * z - x * x));
+}
+
+__global__ __launch_bounds__(256) void k_edge_sh_bwd(const float* __restrict__ v, const float* __restrict__ g, int64_t n,
+                                                     int unit, float* __restrict__ gv) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  float x = v[3 * e], y = v[3 * e + 1], z = v[3 * e + 2], d = 1.f, c1 = 1.f, c2 = 1.f;
+  if (unit) {
+    d = sqrtf(x * x + y * y + z * z);
+    x /= d; y /= d; z /= d;
+    c1 = kShInt[1]; c2 = kShInt[2];
+  }
+  const float* G = g + 9 * e;
+  const float g4 = c2 * G[4], g5 = c2 * G[5], g6 = c2 * G[6], g7 = c2 * G[7], g8 = c2 * G[8];
+  float a = c1 * G[1] + kS3 * (z * g4 + y * g5) - x * g6 - kS3 * x * g8;
+  float b = c1 * G[2] + kS3 * (x * g5 + z * g7) + 2.f * y * g6;
+  float c = c1 * G[3] + kS3 * (x * g4 + y * g7) - z * g6 + kS3 * z * g8;
+  if (unit) {
+    const float r = a * x + b * y + c * z;
+    a = (a - r * x) / d;
+    b = (b - r * y) / d;
+    c = (c - r * z) / d;
+  }
+  gv[3 * e] = a;
+  gv[3 * e + 1] = b;
+  gv[3 * e + 2] = c;
+}
+
+E2V2_API int e2v2_edge_sh(const float* v, int64_t n, int unit, float* Y, hipStream_t s) {
+  E2V2_REQUIRE(n >= 0 && n < (1LL << 38) && (n == 0 || (v && Y)), "edge_sh: n %lld, null pointer", (long long)n);
+  if (n == 0) return 0;
+  hipLaunchKernelGGL(k_edge_sh, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, v, n, unit, Y);
+  E2V2_LAUNCHED("k_edge_sh");
+  return 0;
+}
+
+E2V2_API int e2v2_edge_sh_bwd(const float* v, const float* g, int64_t n, int unit, float* gv, hipStream_t s) {
+  E2V2_REQUIRE(n >= 0 && n < (1LL << 38) && (n == 0 || (v && g && gv)), "edge_sh_bwd: n %lld, null pointer",
+               (long long)n);
+  if (n == 0) return 0;
+  hipLaunchKernelGGL(k_edge_sh_bwd, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, v, g, n, unit, gv);
+  E2V2_LAUNCHED("k_edge_sh_bwd");
+  return 0;
+}
+
 E2V2_API int e2v2_sh_contract(const float* Y, const float* xn, const int32_t* row_ptr, int32_t n_rows, int32_t C,
                               float* x0, hipStream_t s) {
   E2V2_REQUIRE(n_rows >= 0 && C >= 1 && C <= 64 * kShPer && (n_rows == 0 || (Y && xn && row_ptr && x0)),

@@ -24,7 +24,7 @@ from torch.profiler import record_function as _record_function
 from . import so3
 from . import _lib
 from . import gemm as s3gemm
-from .ops import AttentionFn, DegreeEmbedFn, QKdotGateFn, RadialCache, RadialEvalFn, ShContractFn, \
+from .ops import AttentionFn, DegreeEmbedFn, EdgeShFn, QKdotGateFn, RadialCache, RadialEvalFn, ShContractFn, \
     _no_double_backward, attention_backward, attention_forward, attn_args, module_params
 
 _NO_RANGE = contextlib.nullcontext()
@@ -1656,17 +1656,17 @@ class E2AttentionArbOrder_sparse(nn.Module):
             packs = dense_packs(self.fc_m0, ctx.bf16)
             if packs is not None and xd.shape[2] == 256 and H == 128 and tab.nc == 768:
                 # the 768-wide edge operand is formed inside the gate GEMM (no per-edge channel tensor)
-                return QKdotGateFn.apply(ctx.dist, _sh_integral(ctx.dvec), xd, nl, ctx.atom_type, tab, packs,
+                return QKdotGateFn.apply(ctx.dist, EdgeShFn.apply(ctx.dvec, True), xd, nl, ctx.atom_type, tab, packs,
                                          self.fc_m0.bias.detach())
             rad = RadialEvalFn.apply(ctx.dist, nl, ctx.atom_type, tab)
-            x0 = ShContractFn.apply(_sh_integral(ctx.dvec), xd, nl).reshape(E, -1)    # [E, 3 Cd]
+            x0 = ShContractFn.apply(EdgeShFn.apply(ctx.dvec, True), xd, nl).reshape(E, -1)    # [E, 3 Cd]
             return _linear(x0 * rad, self.fc_m0, True)
         rad = RadialEvalFn.apply(ctx.dist, nl, ctx.atom_type, tab)
         # checked once per version of sum_vec (a host readback), not on every evaluation
         if not cached(self, "sum_vec_ok", (self.sum_vec,),
                       lambda: torch.equal(self.sum_vec.detach().cpu(), self._sum_vec_blocks())):
             raise NotImplementedError("QKdotS_alpha: sum_vec must keep its l-block indicator values")
-        x0 = ShContractFn.apply(_raw_sh(ctx.dvec), xd, nl).reshape(E, -1)[:, :H]     # [E, H]
+        x0 = ShContractFn.apply(EdgeShFn.apply(ctx.dvec, False), xd, nl).reshape(E, -1)[:, :H]     # [E, H]
         dl = self.direction_linear
         return _linear(_ln_silu(_linear(x0 * rad[:, :H], dl[0], True), dl[1]), dl[3], True)
 

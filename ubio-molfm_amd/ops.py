@@ -577,6 +577,30 @@ def _qkdot_args(nl: NeighborList, atom_type, table: RadialTable, dist, Y, xd, pi
                           int(pieces))
 
 
+class EdgeShFn(torch.autograd.Function):
+    """Spherical harmonics l <= 2 of edge vectors v [E, 3], [E, 9] (e2v2_edge_sh): the raw polynomials of v, or with
+    ``unit`` e3nn's normalised ones."""
+
+    @staticmethod
+    def forward(ctx, v, unit: bool):
+        _need_cuda(v)
+        v = v.float().contiguous()
+        Y = torch.empty(v.shape[0], 9, dtype=torch.float32, device=v.device)
+        _lib.call("e2v2_edge_sh", _p(v), _lib.i64(v.shape[0]), _lib.i32(int(unit)), _p(Y), _stream(v))
+        ctx.save_for_backward(v)
+        ctx.unit = unit
+        return Y
+
+    @staticmethod
+    def backward(ctx, g):
+        _no_double_backward()
+        (v,) = ctx.saved_tensors
+        g = g.float().contiguous()
+        gv = torch.empty_like(v)
+        _lib.call("e2v2_edge_sh_bwd", _p(v), _p(g), _lib.i64(v.shape[0]), _lib.i32(int(ctx.unit)), _p(gv), _stream(v))
+        return gv, None
+
+
 class ShContractFn(torch.autograd.Function):
     """x0 [E, 3, C] with x0[e, l] = sum_{m in l} Y[e, m] xn[m, row(e)] (e2v2_sh_contract):
     the per-edge x_0_extra of the QKdot gates (e2former.py:271-276, 288-296).  Y
