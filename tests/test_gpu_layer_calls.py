@@ -1,6 +1,9 @@
 """Attention layers and feed-forward blocks enqueued by one native call each way against the same layers launched
 one kernel at a time from Python: the launches are the same, so energies, forces and node features are bitwise
 equal, for every attention type, gate and weight form, in both compute modes."""
+import copy
+import pickle
+
 import numpy as np
 import pytest
 import torch
@@ -73,3 +76,14 @@ def test_layer_saved_state_survives_a_saved_tensor_hook(pkg, cuda):
     with torch.autograd.graph.save_on_cpu():
         y = ffn(x)
     assert torch.equal(a, torch.autograd.grad(y, x, g)[0])
+
+
+def test_layer_copies_and_pickles_with_its_module(pkg, cuda):
+    m = _model(cuda, {})
+    ffn = next(x for x in m.modules() if type(x).__name__ == "FeedForwardNetwork_s3")
+    x = torch.randn(9, 5, 256, device=cuda)
+    y = ffn(x)
+    twin, back = copy.deepcopy(ffn), pickle.loads(pickle.dumps(ffn))
+    with torch.no_grad():
+        twin.slinear_2.weight.mul_(2.0)
+    assert torch.equal(ffn(x), y) and torch.equal(back(x), y) and not torch.equal(twin(x), y)

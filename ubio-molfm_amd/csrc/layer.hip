@@ -42,7 +42,7 @@ void with_bias(e2v2_gemm_args& G, const float* bias, int batches, int64_t bs = 0
   G.bias_bs = bs;
 }
 
-// The saved and scratch arrays of an attention layer, each a multiple of 16 bytes per node, one after another.
+// The saved and scratch arrays of an attention layer, one after another (multiples of 16 bytes per node).
 struct Layout {
   int64_t n, at = 0;
   char* base;
@@ -63,13 +63,13 @@ Saved saved_of(const e2v2_attn_layer& W, int64_t n, void* base) {
   Saved S;
   S.y = L.take((int64_t)9 * 4 * W.hid * es);
   S.h1 = L.take((int64_t)2 * W.hid * 4);
-  S.st = L.take(16);
   S.qk = L.take((int64_t)2 * W.n_out * es);
   S.v = L.take((int64_t)9 * W.c * es);
   S.so2 = L.take((int64_t)so2_rows(W) * W.c * es);
   S.mrow = L.take(W.heads * 4);
   S.srow = L.take(W.heads * 4);
   S.cnt = L.take(W.heads * 4);
+  S.st = L.take(16);                 // last: all before it stay on 128-byte lines, whose rows the gathers read
   S.per_node = n ? L.at / n : 0;
   return S;
 }

@@ -698,6 +698,9 @@ class AttnLayer:
     """The packed weights of one attention layer as e2v2_attn_layer: ``struct`` and what its pointers refer to."""
     __slots__ = ("struct", "keep", "saved", "fwd", "bwd", "zero")
 
+    def __reduce__(self):
+        return type(None), ()      # a copied or pickled module packs its own weights
+
     def __init__(self, s3, P, Wvop, bv, Wc, out_bias, zero: bool):
         a = _lib.AttnLayer()
         vf = Wvop.s3f()
@@ -1100,6 +1103,9 @@ class FFNS3Fn(torch.autograd.Function):
 class FFNLayer:
     """The packed weights of one feed-forward block as e2v2_ffn_layer: ``struct`` and what its pointers refer to."""
     __slots__ = ("struct", "keep")
+
+    def __reduce__(self):
+        return type(None), ()      # a copied or pickled module packs its own weights
 
     def __init__(self, W1op, b1, fold: GateFold, W2op, b2):
         self.keep = (W1op.s3f(), W1op.s3b(), fold.f, fold.bk, W2op.s3f(), W2op.s3b(), b1, fold.b, b2)
