@@ -212,60 +212,60 @@ __device__ void visit_edges_wave(const e2v2_nbr_plan& P, int i_, Emit&& emit) {
       x1 = min(min(x1, d0 - 1), x0 + 2); y1 = min(min(y1, d1 - 1), y0 + 2); z1 = min(min(z1, d2 - 1), z0 + 2);
     }
     for (uint64_t todo = __ballot(in); todo; todo &= todo - 1) {
-    const int l = (int)__builtin_ctzll(todo), s = sb + l;
-    auto scalar = [&](int v) { return __builtin_amdgcn_readlane(v, l); };
-    const float off[3] = {__int_as_float(scalar(__float_as_int(o0))), __int_as_float(scalar(__float_as_int(o1))),
-                          __int_as_float(scalar(__float_as_int(o2)))};
-    const int bx = scalar(x0) + ra, by = scalar(y0) + rb, bz0 = scalar(z0), bz1 = scalar(z1);
-    // run (a, b) holds bins (x0 + a, y0 + b, z0..z1); pre = inclusive prefix of
-    // run lengths, base = run start - exclusive prefix
-    int st = 0, len = 0;
-    if (lane < 9 && bx <= scalar(x1) && by <= scalar(y1)) {
-      const int bin = bbase + (bx * d1 + by) * d2;
-      st = P.bin_start[bin + bz0];
-      len = P.bin_start[bin + bz1 + 1] - st;
-    }
-    int incl = len;
-#pragma unroll
-    for (int o = 1; o < 9; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    const int bs = st - (incl - len);
-    int pre[9], base[9];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-      pre[q] = __builtin_amdgcn_readlane(incl, q);
-      base[q] = __builtin_amdgcn_readlane(bs, q);
-    }
-    const int total = pre[8];
-    for (int c0 = 0; c0 < total; c0 += 64) {
-      const int c = c0 + lane;
-      bool ok = false;
-      int j = 0;
-      float dx = 0.f, dy = 0.f, dz = 0.f, d = 0.f;
-      if (c < total) {
-        int t = 0;
-#pragma unroll
-        for (int q = 8; q >= 0; --q)
-          if (c < pre[q]) t = base[q] + c;
-        j = P.bin_atoms[t];
-        exact_edge(pi, P.pos + 3 * j, off, dx, dy, dz);
-        d = exact_dist(dx, dy, dz);
-        ok = d >= P.rmin && d <= P.rc && (P.src_include == nullptr || P.src_include[j] != 0);
-        if (ok && periodic && !(d < P.rc)) {
-          float img[3];
-          {
-#pragma clang fp contract(off)
-            img[0] = P.pos[3 * j] + off[0];
-            img[1] = P.pos[3 * j + 1] + off[1];
-            img[2] = P.pos[3 * j + 2] + off[2];
-          }
-          ok = image_has_inner(P, g, img);
-        }
+      const int l = (int)__builtin_ctzll(todo), s = sb + l;
+      auto scalar = [&](int v) { return __builtin_amdgcn_readlane(v, l); };
+      const float off[3] = {__int_as_float(scalar(__float_as_int(o0))), __int_as_float(scalar(__float_as_int(o1))),
+                            __int_as_float(scalar(__float_as_int(o2)))};
+      const int bx = scalar(x0) + ra, by = scalar(y0) + rb, bz0 = scalar(z0), bz1 = scalar(z1);
+      // run (a, b) holds bins (x0 + a, y0 + b, z0..z1); pre = inclusive prefix of
+      // run lengths, base = run start - exclusive prefix
+      int st = 0, len = 0;
+      if (lane < 9 && bx <= scalar(x1) && by <= scalar(y1)) {
+        const int bin = bbase + (bx * d1 + by) * d2;
+        st = P.bin_start[bin + bz0];
+        len = P.bin_start[bin + bz1 + 1] - st;
       }
-      emit(ok, j, s, dx, dy, dz, d);
-    }
+      int incl = len;
+#pragma unroll
+      for (int o = 1; o < 9; o <<= 1) {
+        const int v = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += v;
+      }
+      const int bs = st - (incl - len);
+      int pre[9], base[9];
+#pragma unroll
+      for (int q = 0; q < 9; ++q) {
+        pre[q] = __builtin_amdgcn_readlane(incl, q);
+        base[q] = __builtin_amdgcn_readlane(bs, q);
+      }
+      const int total = pre[8];
+      for (int c0 = 0; c0 < total; c0 += 64) {
+        const int c = c0 + lane;
+        bool ok = false;
+        int j = 0;
+        float dx = 0.f, dy = 0.f, dz = 0.f, d = 0.f;
+        if (c < total) {
+          int t = 0;
+#pragma unroll
+          for (int q = 8; q >= 0; --q)
+            if (c < pre[q]) t = base[q] + c;
+          j = P.bin_atoms[t];
+          exact_edge(pi, P.pos + 3 * j, off, dx, dy, dz);
+          d = exact_dist(dx, dy, dz);
+          ok = d >= P.rmin && d <= P.rc && (P.src_include == nullptr || P.src_include[j] != 0);
+          if (ok && periodic && !(d < P.rc)) {
+            float img[3];
+            {
+#pragma clang fp contract(off)
+              img[0] = P.pos[3 * j] + off[0];
+              img[1] = P.pos[3 * j + 1] + off[1];
+              img[2] = P.pos[3 * j + 2] + off[2];
+            }
+            ok = image_has_inner(P, g, img);
+          }
+        }
+        emit(ok, j, s, dx, dy, dz, d);
+      }
     }
   }
 }
@@ -644,115 +644,115 @@ __global__ __launch_bounds__(256) void k_cluster_slots(const int32_t* __restrict
   __shared__ int total;
   const int t = threadIdx.x, n_cl = (n_seg + span - 1) / span;
   for (int cl = blockIdx.x; cl < n_cl; cl += gridDim.x) {
-  if (only_left && n_slots[cl] >= 0) continue;   // (uniform over the workgroup)
-  __syncthreads();                               // the previous cluster's LDS reads are done
-  const int s0 = cl * span, s1 = min(s0 + span, n_seg);
-  const int b = seg_ptr[s0], n = seg_ptr[s1] - b;
-  auto eid_of = [&](int p) { return item_eid ? item_eid[p] : p; };
-  if (n > kMaxClusterItems) {
-    for (int q = t; q < n; q += 256) {
-      const int p = b + q;
-      int sg = 0;
-      while (sg + 1 < s1 - s0 && seg_ptr[s0 + sg + 1] <= p) ++sg;
-      const int e = eid_of(p);
-      slot_member[p] = member[e];
-      for (int r = 0; r < span; ++r) slot_edge[(int64_t)p * span + r] = (r == sg) ? e : -1;
+    if (only_left && n_slots[cl] >= 0) continue;   // (uniform over the workgroup)
+    __syncthreads();                               // the previous cluster's LDS reads are done
+    const int s0 = cl * span, s1 = min(s0 + span, n_seg);
+    const int b = seg_ptr[s0], n = seg_ptr[s1] - b;
+    auto eid_of = [&](int p) { return item_eid ? item_eid[p] : p; };
+    if (n > kMaxClusterItems) {
+      for (int q = t; q < n; q += 256) {
+        const int p = b + q;
+        int sg = 0;
+        while (sg + 1 < s1 - s0 && seg_ptr[s0 + sg + 1] <= p) ++sg;
+        const int e = eid_of(p);
+        slot_member[p] = member[e];
+        for (int r = 0; r < span; ++r) slot_edge[(int64_t)p * span + r] = (r == sg) ? e : -1;
+      }
+      __syncthreads();                             // every thread has read n_slots[cl]
+      if (t == 0) n_slots[cl] = n;
+      continue;
     }
-    __syncthreads();                             // every thread has read n_slots[cl]
-    if (t == 0) n_slots[cl] = n;
-    continue;
-  }
-  // keys (member, segment, position) sorted ascending
-  int p2 = 1;
-  while (p2 < n) p2 <<= 1;
-  for (int q = t; q < p2; q += 256) {
-    uint64_t k = ~0ull;
-    if (q < n) {
-      const int p = b + q;
-      int sg = 0;
-      while (sg + 1 < s1 - s0 && seg_ptr[s0 + sg + 1] <= p) ++sg;
-      k = ((uint64_t)(uint32_t)member[eid_of(p)] << 32) | ((uint64_t)sg << 16) | (uint64_t)q;
+    // keys (member, segment, position) sorted ascending
+    int p2 = 1;
+    while (p2 < n) p2 <<= 1;
+    for (int q = t; q < p2; q += 256) {
+      uint64_t k = ~0ull;
+      if (q < n) {
+        const int p = b + q;
+        int sg = 0;
+        while (sg + 1 < s1 - s0 && seg_ptr[s0 + sg + 1] <= p) ++sg;
+        k = ((uint64_t)(uint32_t)member[eid_of(p)] << 32) | ((uint64_t)sg << 16) | (uint64_t)q;
+      }
+      sk[q] = k;
     }
-    sk[q] = k;
-  }
-  __syncthreads();
-  for (int k = 2; k <= p2; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int q = t; q < p2; q += 256) {
-        const int x = q ^ j;
-        if (x > q) {
-          const uint64_t a = sk[q], c = sk[x];
-          if ((a > c) == ((q & k) == 0)) {
-            sk[q] = c;
-            sk[x] = a;
+    __syncthreads();
+    for (int k = 2; k <= p2; k <<= 1) {
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int q = t; q < p2; q += 256) {
+          const int x = q ^ j;
+          if (x > q) {
+            const uint64_t a = sk[q], c = sk[x];
+            if ((a > c) == ((q & k) == 0)) {
+              sk[q] = c;
+              sk[x] = a;
+            }
           }
         }
-      }
-      __syncthreads();
-    }
-  }
-  // per item: occurrence = rank among equal (member, segment); per member group: slot count
-  // = 1 + max occurrence, written at the group's first item
-  auto occ_of = [&](int q) {
-    int o = 0;
-    while (q - o - 1 >= 0 && (sk[q - o - 1] >> 16) == (sk[q] >> 16)) ++o;
-    return o;
-  };
-  constexpr int kPer = kMaxClusterItems / 256;
-  int local = 0;
-  for (int z = 0; z < kPer; ++z) {
-    const int q = t * kPer + z;
-    int cnt = 0;
-    if (q < n && (q == 0 || (sk[q - 1] >> 32) != (sk[q] >> 32))) {
-      int mx = 0;
-      for (int u = q; u < n && (sk[u] >> 32) == (sk[q] >> 32); ++u) mx = max(mx, occ_of(u));
-      cnt = mx + 1;
-    }
-    gbase[q] = cnt;
-    local += cnt;
-  }
-  part[t] = local;
-  __syncthreads();
-  if (t == 0) {
-    int acc = 0;
-    for (int u = 0; u < 256; ++u) {
-      const int v = part[u];
-      part[u] = acc;
-      acc += v;
-    }
-    total = acc;
-    n_slots[cl] = acc;
-  }
-  __syncthreads();
-  int run = part[t];
-  for (int z = 0; z < kPer; ++z) {
-    const int q = t * kPer + z;
-    const int v = gbase[q];
-    gbase[q] = run;
-    run += v;
-  }
-  __syncthreads();
-  // group heads initialise their slots, then every item writes its edge
-  for (int q = t; q < n; q += 256) {
-    if (q == 0 || (sk[q - 1] >> 32) != (sk[q] >> 32)) {
-      // exclusive scan: the item after a group head carries the head's base + count
-      const int cnt = ((q + 1 < n) ? gbase[q + 1] : total) - gbase[q];
-      for (int o = 0; o < cnt; ++o) {
-        const int64_t sl = (int64_t)b + gbase[q] + o;
-        slot_member[sl] = (int32_t)(sk[q] >> 32);
-        for (int r = 0; r < span; ++r) slot_edge[sl * span + r] = -1;
+        __syncthreads();
       }
     }
-  }
-  __syncthreads();
-  for (int q = t; q < n; q += 256) {
-    int g = q;
-    while (g > 0 && (sk[g - 1] >> 32) == (sk[q] >> 32)) --g;
-    const int sg = (int)((sk[q] >> 16) & 0xffff);
-    const int pos = (int)(sk[q] & 0xffff);
-    const int64_t sl = (int64_t)b + gbase[g] + occ_of(q);
-    slot_edge[sl * span + sg] = eid_of(b + pos);
-  }
+    // per item: occurrence = rank among equal (member, segment); per member group: slot count
+    // = 1 + max occurrence, written at the group's first item
+    auto occ_of = [&](int q) {
+      int o = 0;
+      while (q - o - 1 >= 0 && (sk[q - o - 1] >> 16) == (sk[q] >> 16)) ++o;
+      return o;
+    };
+    constexpr int kPer = kMaxClusterItems / 256;
+    int local = 0;
+    for (int z = 0; z < kPer; ++z) {
+      const int q = t * kPer + z;
+      int cnt = 0;
+      if (q < n && (q == 0 || (sk[q - 1] >> 32) != (sk[q] >> 32))) {
+        int mx = 0;
+        for (int u = q; u < n && (sk[u] >> 32) == (sk[q] >> 32); ++u) mx = max(mx, occ_of(u));
+        cnt = mx + 1;
+      }
+      gbase[q] = cnt;
+      local += cnt;
+    }
+    part[t] = local;
+    __syncthreads();
+    if (t == 0) {
+      int acc = 0;
+      for (int u = 0; u < 256; ++u) {
+        const int v = part[u];
+        part[u] = acc;
+        acc += v;
+      }
+      total = acc;
+      n_slots[cl] = acc;
+    }
+    __syncthreads();
+    int run = part[t];
+    for (int z = 0; z < kPer; ++z) {
+      const int q = t * kPer + z;
+      const int v = gbase[q];
+      gbase[q] = run;
+      run += v;
+    }
+    __syncthreads();
+    // group heads initialise their slots, then every item writes its edge
+    for (int q = t; q < n; q += 256) {
+      if (q == 0 || (sk[q - 1] >> 32) != (sk[q] >> 32)) {
+        // exclusive scan: the item after a group head carries the head's base + count
+        const int cnt = ((q + 1 < n) ? gbase[q + 1] : total) - gbase[q];
+        for (int o = 0; o < cnt; ++o) {
+          const int64_t sl = (int64_t)b + gbase[q] + o;
+          slot_member[sl] = (int32_t)(sk[q] >> 32);
+          for (int r = 0; r < span; ++r) slot_edge[sl * span + r] = -1;
+        }
+      }
+    }
+    __syncthreads();
+    for (int q = t; q < n; q += 256) {
+      int g = q;
+      while (g > 0 && (sk[g - 1] >> 32) == (sk[q] >> 32)) --g;
+      const int sg = (int)((sk[q] >> 16) & 0xffff);
+      const int pos = (int)(sk[q] & 0xffff);
+      const int64_t sl = (int64_t)b + gbase[g] + occ_of(q);
+      slot_edge[sl * span + sg] = eid_of(b + pos);
+    }
   }
 }
 
