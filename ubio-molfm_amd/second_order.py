@@ -10,14 +10,16 @@ The fused attention and degree kernels give first-order input gradients only.
 In training mode (``module.train()``) the backbone instead composes each layer
 from the op-level HIP functions of ``sparse_ops`` -- the segment QK dot, the
 alpha sum, the value aggregation and the degree outer product, each with
-second- and higher-order gradients -- and PyTorch ops for the per-node and
-per-edge dense parts, as the reference composes them
+second- and higher-order gradients --, fused passes that are closed under
+differentiation (csrc/train.hip, csrc/wgrad.hip, the second-order norms of
+csrc/node.hip) and PyTorch ops for the other per-node and per-edge dense parts,
+as the reference composes them
 (e2former.py:223-436, 623-753, 958-1145 with ``use_triton``), so gradients of
 the forces reach every parameter and the positions.  The first-order SO(2)
 product runs in its Cartesian form (the sum over the 9 value rows and the three
 components of the edge vector with the coupling table of ``so3``; the identity
-with the node-frame product is pinned in the tests), as three value
-aggregations with weights w * dvec[:, k].  The radial profiles are evaluated per
+with the node-frame product is pinned in the tests), the three components in
+one pass over the value rows (_So2AggFn).  The radial profiles are evaluated per
 edge (no distance tables: their parameters receive gradients).  fp32 only.
 
 Every edge operation still runs on the GPU through libe2v2.so; nothing here
