@@ -119,9 +119,15 @@ class FfnLayer(C.Structure):
 
 
 def stream(device=None):
-    """The current HIP stream of a device (None: the current device) as a call argument."""
+    """The current HIP stream of a device (None: the current device) as a call argument.  ValueError for a device
+    without streams: an operand in host memory is refused here, before its pointer reaches a kernel."""
     import torch
-    idx = None if device is None else torch.device(device).index
+    idx = None
+    if device is not None:
+        device = torch.device(device)
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        idx = device.index
     return vp(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx))
 
 

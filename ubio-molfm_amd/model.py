@@ -32,7 +32,7 @@ from .ops import EdgeGeometryFn
 def graph_bounds(pos: torch.Tensor, counts: torch.Tensor):
     """Per-graph coordinate minimum and maximum [B, 3] (graphs contiguous)."""
     if counts.shape[0] == 1:
-        return coordinate_bounds(pos).split(1)
+        return pos.amin(0, keepdim=True), pos.amax(0, keepdim=True)
     lo = torch.segment_reduce(pos, "min", lengths=counts, axis=0, unsafe=True)
     hi = torch.segment_reduce(pos, "max", lengths=counts, axis=0, unsafe=True)
     return lo, hi

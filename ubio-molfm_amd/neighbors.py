@@ -199,8 +199,10 @@ def make_plan(pos: torch.Tensor, graph_ptr, cells, pbcs, rc: float, rmin: float 
     if grid_box is not None:
         bb = np.asarray(grid_box, F32).reshape(2, B, 3)
     elif N:
-        if B == 1:
+        if B == 1 and pos.is_cuda and pos.dtype == torch.float32:
             bb = coordinate_bounds(pos).cpu().numpy().reshape(2, 1, 3)
+        elif B == 1:
+            bb = torch.stack([pos.amin(0, keepdim=True), pos.amax(0, keepdim=True)]).cpu().numpy()
         else:
             counts = torch.as_tensor(np.diff(graph_ptr), device=dev)
             lo = torch.segment_reduce(pos, "min", lengths=counts, axis=0, unsafe=True)
