@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from ubio_molfm_amd import _lib, gemm, model, neighbors
+from ubio_molfm_amd import _lib, model, neighbors
 
 
 @pytest.mark.parametrize("device", ["cpu", torch.device("cpu"), "meta"])
@@ -19,16 +19,11 @@ def test_stream_of_a_device_without_streams(device):
     lambda p: neighbors.coordinate_bounds(p),
     lambda p: neighbors.cluster_slots(torch.tensor([0, 1], dtype=torch.int32), 1, torch.zeros(1, dtype=torch.int32),
                                       None, 4),
-    lambda p: gemm.pack(torch.zeros(128, 128)),
-], ids=["order_one_graph", "order_two_graphs", "bounds", "cluster_slots", "pack"])
+], ids=["order_one_graph", "order_two_graphs", "bounds", "cluster_slots"])
 def test_host_operands_are_refused(call, monkeypatch):
-    real = _lib.call
-    host_only = {"e2v2_gemm_packed_bytes"}
-
-    def guarded(name, *args):
-        assert name in host_only, f"{name} was called with host pointers"
-        return real(name, *args)
-    monkeypatch.setattr(_lib, "call", guarded)
+    def launched(name, *args):
+        raise AssertionError(f"{name} was called with host pointers")
+    monkeypatch.setattr(_lib, "call", launched)
     with pytest.raises(ValueError, match="Expected a cuda device"):
         call(torch.rand(5, 3))
 
