@@ -118,6 +118,29 @@ def test_attention_weights(pkg, cuda, n, separate):
                  [torch.cat([gate, ih], 1), qk, p], g, cuda)
 
 
+@pytest.mark.parametrize("value", [float("-inf"), float("inf"), float("nan")])
+@pytest.mark.parametrize("where", ["first", "last", "one_group", "all"])
+def test_attention_weights_of_logits_that_are_not_finite(pkg, cuda, value, where):
+    """Rows holding infinite or NaN logits: NaN where the composition has NaN, its values elsewhere (also on the
+    other edges of such a row, and of a wavefront's share of the row that holds nothing else)."""
+    from ubio_molfm_amd import second_order as so
+    e, row, _, g = _edges(12, 3, cuda)
+    e.qi = row.to(cuda)
+    eg, qk = torch.randn(e.E, 2 * H, generator=g), torch.randn(e.E, H, generator=g)
+    p = torch.rand(e.E, generator=g)
+    for r, heads in ((1, slice(0, 5)), (2, slice(64, 128)), (4, slice(0, 128))):
+        ids = torch.nonzero(row == r).flatten()
+        ids = {"first": ids[:1], "last": ids[-1:], "one_group": ids[3::8], "all": ids}[where]
+        for x in ids.tolist():
+            eg[x, :H][heads], qk[x, heads] = value, 1.0
+    eg, qk, p = (t.to(cuda) for t in (eg, qk, p))
+    got, want = so._AttnWeightsFn.apply(eg, None, qk, p, e), so._softmax_weights(eg, None, qk, p, e)
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(got), nan)
+    got, want = got[~nan].double(), want[~nan].double()
+    assert float((got - want).norm()) <= TOL * float(want.norm())
+
+
 @pytest.mark.parametrize("n,F", [(1, 4), (61, 128), (61, 100), (5, 1024)])
 def test_sum_with_gathered_rows(pkg, cuda, n, F):
     from ubio_molfm_amd import second_order as so

@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256) void k_aw_fwd(const int32_t* __restrict__ row_
         m[z] = a;
         cn[z] = 1.f;
       } else {
-        s[z] += expf(a - m[z]) * p;
+        s[z] += (a == m[z] ? 1.f : expf(a - m[z])) * p;     // (a = m = -inf: worth 0 once a larger one comes)
         cn[z] += a == m[z] ? 1.f : 0.f;
       }
     }
@@ -317,9 +317,10 @@ __global__ __launch_bounds__(256) void k_aw_fwd(const int32_t* __restrict__ row_
 #pragma unroll
     for (int u = 0; u < kAwGroups; ++u) {
       const float mu = at(rm[u][q], z);
-      if (mu > -INFINITY) S[z] += at(rs[u][q], z) * expf(mu - M[z]);
+      S[z] += at(rs[u][q], z) * (mu > -INFINITY ? expf(mu - M[z]) : 0.f);   // (a group of NaN alone: its sum is NaN)
       if (mu == M[z]) Cn[z] += at(rc[u][q], z);
     }
+    if (M[z] == INFINITY) S[z] = NAN;         // inf - inf on the edge that attains it
     rho[z] = 1.f / (S[z] + kAwEps);
   }
   if (g == 0) {
