@@ -111,3 +111,95 @@ def test_qk_projection_few_rows(pkg, cuda, n, hid, with_v):
     if with_v:
         ref = ref + gv.double() @ Wv.double()[L_OF_M]
     assert float((gx.double() - ref).norm() / ref.norm()) < 4e-6
+
+
+def _same_rows(few, many, at, m):
+    assert torch.equal(few, many[..., at:at + m, :])
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 128, 16), (33, 256, 144), (700, 512, 256), (2500, 256, 512)])
+@pytest.mark.parametrize("form", ["fp32 A", "bf16 A", "gated"])
+def test_one_piece_rows_do_not_depend_on_the_call(pkg, cuda, m, n, k, form):
+    """bf16 mode: a row's result is bitwise the same among few rows as among many, alone and in a group (a sum in
+    another order would be rounded to another bf16 further on)."""
+    from ubio_molfm_amd import gemm
+    g = torch.Generator().manual_seed(m + n)
+    batch, many, at = 3, 6000, 3211
+    a = torch.randn(batch, many, k, generator=g).to(cuda)
+    w = (torch.randn(2, n, k, generator=g) / math.sqrt(k)).to(cuda)
+    bias, res = torch.randn(n, generator=g).to(cuda), torch.randn(batch, many, n, generator=g).to(cuda)
+    pw, widx = gemm.pack(w, pieces=1), [0, 1, 0]
+    logits = torch.randn(many, 2 * k, generator=g).to(cuda)
+    if form == "bf16 A":
+        a = a.bfloat16()
+
+    def run(rows, dtype, grouped=False):
+        x, r = a[:, rows].contiguous(), res[:, rows].contiguous()
+        out = torch.empty(batch, x.shape[1], n, device=cuda, dtype=dtype)
+        if grouped:
+            gemm.gemm_grouped([dict(a=x, pw=pw, out=out, widx=widx, bias=bias, res=r),
+                               dict(a=a[0], pw=pw, out=torch.empty(many, n, device=cuda), widx=[1])])
+        else:
+            gate = (logits[rows].contiguous(), 1.5, 0.75) if form == "gated" else None
+            gemm.gemm(x, pw, out, widx, bias=bias, bias_batches=1, res=r, gate=gate)
+        return out
+    some = slice(at, at + m)
+    for dtype in (torch.float32, torch.bfloat16):
+        _same_rows(run(some, dtype), run(slice(None), dtype), at, m)
+    if form != "gated":
+        assert torch.equal(run(some, torch.float32, True), run(slice(None), torch.float32, True)[:, some])
+
+
+@pytest.mark.parametrize("n,hid", [(1, 512), (33, 64), (300, 192), (1024, 512)])
+@pytest.mark.parametrize("y_bf16", [True, False])
+def test_one_piece_qk_projection_does_not_depend_on_the_call(pkg, cuda, n, hid, y_bf16):
+    from ubio_molfm_amd import gemm
+    torch.manual_seed(n + hid)
+    C, Cv, many, at = 256, 256, 2100, 1007
+    W, b = torch.randn(3, 4 * hid, C, device=cuda) / 16, torch.randn(4 * hid, device=cuda)
+    P = gemm.pack_qk(W, b, torch.randn(3, Cv, C, device=cuda) / 16, pieces=1)
+    x = torch.randn(9, many, C, device=cuda)
+    ghq, ghk = torch.randn(many, 3 * hid, device=cuda), torch.randn(many, 3 * hid, device=cuda)
+    gv = torch.randn(9, many, Cv, device=cuda)
+    some = slice(at, at + n)
+    out = []
+    for rows in (slice(None), some):
+        hq, hk, y = gemm.qk_forward(x[:, rows].contiguous(), P, y_bf16=y_bf16)
+        out.append([hq, hk, y])
+        for v in (gv[:, rows].contiguous(), None):
+            out[-1].append(gemm.qk_backward(y, ghq[rows].contiguous(), ghk[rows].contiguous(), v, P))
+    for all_rows, few in zip(*out):
+        _same_rows(few, all_rows, at, n)
+
+
+def test_bf16_layers_do_not_depend_on_the_batch(pkg, cuda):
+    """Degree embedding, attention layer and feed-forward block of the bf16 mode: a molecule among copies of itself
+    has bitwise the features and gradients that it has alone."""
+    import numpy as np
+    from ubio_molfm_amd import modules, neighbors, ops
+    from ubio_molfm_amd.model import MolfmAtomic, default_args
+    torch.manual_seed(2)
+    m = MolfmAtomic(default_args(num_layers=1)).to(cuda).eval().requires_grad_(False)
+    dec, rng, n = m.decoder.decoder, np.random.default_rng(4), 33
+    one = torch.as_tensor(rng.random((n, 3)) * 6.0, dtype=torch.float32)
+    Z1 = torch.as_tensor(rng.choice([1, 6, 8], n))
+    x1, g1 = torch.randn(9, n, 256), torch.randn(9, n, 256)
+    out = []
+    for copies in (1, 130):
+        ptr = np.arange(copies + 1) * n
+        pos = one.repeat(copies, 1).to(cuda)
+        Z = Z1.repeat(copies).to(cuda)
+        nl = neighbors.build_neighbors(pos, ptr, np.zeros((copies, 3, 3)), np.zeros((copies, 3), bool), 6.0)
+        type_z, type_key, slot = modules.atom_type_slots(Z, ptr)
+        pos.requires_grad_(True)
+        x, g = (t.repeat(1, copies, 1).to(cuda) for t in (x1, g1))
+        x.requires_grad_(True)
+        dvec, dist = ops.EdgeGeometryFn.apply(pos, nl)
+        ctx = modules.EdgeContext(nl, dvec, dist, slot, type_z, type_key, dec.rbf, 6.0, True)
+        d = dec.edge_deg_embed_dense(ctx)
+        y = dec.blocks[0].ga(x, ctx)
+        z = dec.blocks[0].ffn(y, bf16=True)
+        grads = torch.autograd.grad([d, y, z], [x, pos], [g, g, g])
+        out.append([t[..., :n, :] for t in (d.detach(), y.detach(), z.detach(), *grads)])
+    for alone, among in zip(*out):
+        assert torch.equal(alone, among)

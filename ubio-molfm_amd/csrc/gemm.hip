@@ -207,22 +207,31 @@ struct KsRaw<false, true> {
   floatx4 x0, x1, m0, m1;
 };
 
-// A tile is one row tile of 32 by two column subtiles: 64 rows (two row tiles) were 20-30% slower below 500
-// rows, where the tiles are too few, and within 5% of it above.
-constexpr int kKsR = 1, kKsJ = 2, kKsM = 32 * kKsR, kKsN = 32 * kKsJ;
+// A few-row tile is one row tile of 32 (64 rows were 20-30% slower below 500 rows, where the tiles are too few, and
+// within 5% of it above).  Three pieces: by two column subtiles, K split over the wavefronts.  One piece (the bf16
+// mode): by the 128 columns of a packed tile, a column subtile per wavefront that sums the whole K in the order of
+// kloop.  There a split sum is not an option: its last bit is the next bf16 rounding's whole step (four layers carry
+// it to 2e-3 of the forces), so a molecule's result would change with the rows that share its call.
+constexpr int kKsJ = 2, kKsM = 32;
+// Ring depths: with three pieces two stages in flight leave four workgroups per CU; one piece takes four.
+constexpr int kKsD3 = 2, kKsD1 = 4;
+__host__ __device__ constexpr int ks_cols(int pieces) { return pieces == 3 ? 32 * kKsJ : kGN; }
+__host__ __device__ constexpr int ks_red(int pieces) { return pieces == 3 ? kKsW * 16 * kKsJ * 64 : 1; }   // LDS floats
 __host__ __device__ __forceinline__ int ks_tiles(const e2v2_gemm_args& G) {
-  return G.batch * ((G.m + kKsM - 1) / kKsM) * (G.n / kKsN);
+  return G.batch * ((G.m + kKsM - 1) / kKsM) * (G.n / ks_cols(G.pieces));
 }
 
-// One 32 x 64 tile of the K-split form (gemm_ks.h); the operands, bounds and epilogue of gemm_tile.
+// One few-row tile (gemm_ks.h); the operands, bounds and epilogue of gemm_tile.
 template <int kP, bool kAB, bool kGate, int kD>
 __device__ __forceinline__ void gemm_tile_ks(const e2v2_gemm_args& G, int tile, float* red, const GateOp& gt) {
   static_assert(!(kAB && kGate), "the gated operand is fp32");
+  constexpr bool kSplit = kP == 3;
+  constexpr int kJ = kSplit ? kKsJ : 1, kCols = ks_cols(kP);
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5;
-  const int n_mt = (G.m + kKsM - 1) / kKsM, n_ct = G.n / kKsN, n_nt = G.n / kGN;
+  const int n_mt = (G.m + kKsM - 1) / kKsM, n_ct = G.n / kCols, n_nt = G.n / kGN;
   const int ct = tile % n_ct, mt = (tile / n_ct) % n_mt, bi = tile / (n_ct * n_mt);
   const int row0 = mt * kKsM, nks = G.k / kGK;
-  const int nt = ct / (kGN / kKsN), q0 = (ct % (kGN / kKsN)) * kKsJ;
+  const int nt = ct / (kGN / kCols), q0 = kSplit ? (ct % (kGN / kCols)) * kJ : wv;
   const bool g0 = kGate && bi == 0;                      // batch 0 of a gated call: silu of the logits
   const int lda = g0 ? (int)gt.ld : (int)G.lda;
   __amdgpu_buffer_rsrc_t ar;
@@ -230,31 +239,28 @@ __device__ __forceinline__ void gemm_tile_ks(const e2v2_gemm_args& G, int tile, 
   else ar = rows_rsrc(g0 ? gt.s : static_cast<const float*>(G.a) + (int64_t)bi * G.a_bs, row0, G.m, lda);
   const __amdgpu_buffer_rsrc_t sr = kGate ? rows_rsrc(gt.s, row0, G.m, (int)gt.ld) : ar;
   const __amdgpu_buffer_rsrc_t br = b_rsrc<kP>(G.b, G.widx[bi], n_nt, nt, nks);
-  uint32_t aoff[kKsR], soff[kKsR], boff[kKsJ];
+  const int rl = lane & 31;
+  const uint32_t aoff = (uint32_t)(rl * lda + 8 * h) * (kAB ? 2u : 4u);
+  const uint32_t soff = kGate ? (uint32_t)(rl * (int)gt.ld + G.k * G.widx[bi] + 8 * h) * 4u : 0u;
+  uint32_t boff[kJ];
 #pragma unroll
-  for (int i = 0; i < kKsR; ++i) {
-    const int r = 32 * i + (lane & 31);
-    aoff[i] = (uint32_t)(r * lda + 8 * h) * (kAB ? 2u : 4u);
-    soff[i] = kGate ? (uint32_t)(r * (int)gt.ld + G.k * G.widx[bi] + 8 * h) * 4u : 0u;
-  }
-#pragma unroll
-  for (int j = 0; j < kKsJ; ++j) boff[j] = ks_b_offset(q0 + j, lane);
-  floatx16 acc[kKsR][kKsJ];
+  for (int j = 0; j < kJ; ++j) boff[j] = ks_b_offset(q0 + j, lane);
+  floatx16 acc[1][kJ];
   ks_zero(acc);
   using Raw = KsRaw<kAB, kGate>;
-  ks_loop<kP, kKsR, kKsJ, kD, Raw>(
-      br, boff, wv * nks / kKsW, (wv + 1) * nks / kKsW,
-      [&](int ks, int i, Raw& x) {
+  ks_loop<kP, 1, kJ, kD, Raw>(
+      br, boff, kSplit ? wv * nks / kKsW : 0, kSplit ? (wv + 1) * nks / kKsW : nks,
+      [&](int ks, int, Raw& x) {
         if constexpr (kAB) {
-          x.b = ks_load_b(ar, aoff[i] + (uint32_t)ks * (kGK * 2u));
+          x.b = ks_load_b(ar, aoff + (uint32_t)ks * (kGK * 2u));
         } else {
           const uint32_t o = (uint32_t)ks * (kGK * 4u);
-          x.x0 = ks_load4(ar, aoff[i] + o);
-          x.x1 = ks_load4(ar, aoff[i] + o + 16u);
+          x.x0 = ks_load4(ar, aoff + o);
+          x.x1 = ks_load4(ar, aoff + o + 16u);
           if constexpr (kGate) {
             if (!g0) {
-              x.m0 = ks_load4(sr, soff[i] + o);
-              x.m1 = ks_load4(sr, soff[i] + o + 16u);
+              x.m0 = ks_load4(sr, soff + o);
+              x.m1 = ks_load4(sr, soff + o + 16u);
             }
           }
         }
@@ -283,21 +289,28 @@ __device__ __forceinline__ void gemm_tile_ks(const e2v2_gemm_args& G, int tile, 
         }
       },
       acc);
-  constexpr int kN = 16 * kKsR * kKsJ;
-  float part[kN], sum[kN / kKsW];
+  // the registers this wavefront finishes (of the tile's, numbered over the column subtiles) and their sums
+  constexpr int kN = 16 * kJ, kS = kSplit ? kN / kKsW : kN;
+  float part[kN], sum[kS];
   ks_flat(acc, part);
-  ks_reduce<kN, kKsW>(red, part, wv, lane, [](int w, int i) { return w * (kN / kKsW) + i; }, sum);
+  if constexpr (kSplit) {
+    ks_reduce<kN, kKsW>(red, part, wv, lane, [](int w, int i) { return w * kS + i; }, sum);
+  } else {
+#pragma unroll
+    for (int i = 0; i < kS; ++i) sum[i] = part[i];
+  }
   const bool with_bias = G.bias && bi < G.bias_batches;
   float* cb = static_cast<float*>(G.c) + (G.c_bf16 ? 0 : (int64_t)bi * G.c_bs);
   __bf16* cbh = static_cast<__bf16*>(G.c) + (G.c_bf16 ? (int64_t)bi * G.c_bs : 0);
   const float* rb = G.r ? G.r + (int64_t)bi * G.r_bs : nullptr;
+  const int col = ct * kCols + 32 * (wv * kS / 16) + rl;   // they are of one column subtile
+  const float bv = with_bias ? G.bias[(int64_t)bi * G.bias_bs + col] : 0.f;
 #pragma unroll
-  for (int i = 0; i < kN / kKsW; ++i) {
-    const int q = wv * (kN / kKsW) + i, r = q % 16, j = (q / 16) % kKsJ, it = q / (16 * kKsJ);
-    const int col = ct * kKsN + 32 * j + (lane & 31), row = row0 + 32 * it + acc_row(r, lane);
+  for (int i = 0; i < kS; ++i) {
+    const int row = row0 + acc_row((wv * kS + i) % 16, lane);
     if (row < G.m) {
       float v = sum[i];
-      if (with_bias) v += G.bias[(int64_t)bi * G.bias_bs + col];
+      if (with_bias) v += bv;
       if (rb) v += rb[(size_t)row * G.ldr + col];
       if (G.c_bf16)
         cbh[(size_t)row * G.ldc + col] = (__bf16)v;
@@ -309,14 +322,14 @@ __device__ __forceinline__ void gemm_tile_ks(const e2v2_gemm_args& G, int tile, 
 
 template <int kP, bool kAB, int kD>
 __global__ __launch_bounds__(kKsThreads, 2) void k_gemm_ks(e2v2_gemm_args G) {
-  __shared__ float red[kKsW * 16 * kKsR * kKsJ * 64];
+  __shared__ float red[ks_red(kP)];
   const int n_tiles = ks_tiles(G), tile = xcd_row(blockIdx.x, n_tiles);
   if (tile >= n_tiles) return;
   gemm_tile_ks<kP, kAB, false, kD>(G, tile, red, GateOp{});
 }
 template <int kP, int kD>
 __global__ __launch_bounds__(kKsThreads, 2) void k_gemm_ks_gate(e2v2_gemm_args G, GateOp gt) {
-  __shared__ float red[kKsW * 16 * kKsR * kKsJ * 64];
+  __shared__ float red[ks_red(kP)];
   const int n_tiles = ks_tiles(G), tile = xcd_row(blockIdx.x, n_tiles);
   if (tile >= n_tiles) return;
   gemm_tile_ks<kP, false, true, kD>(G, tile, red, gt);
@@ -392,7 +405,7 @@ __global__ __launch_bounds__(kGT, 3) void k_gemm_s3_grp_p1(GemmGroups P) {
 
 template <int kP, bool kAB, int kD>
 __global__ __launch_bounds__(kKsThreads, 2) void k_gemm_ks_grp(GemmGroups P) {
-  __shared__ float red[kKsW * 16 * kKsR * kKsJ * 64];
+  __shared__ float red[ks_red(kP)];
   const int b = blockIdx.x;
 #pragma unroll
   for (int gi = 0; gi < kGGroups; ++gi) {
@@ -495,17 +508,16 @@ __global__ __launch_bounds__(kGT, 2) void k_qk_s3_fwd(const float* __restrict__ 
   }
 }
 
-// The same for few rows, K split over the wavefronts (gemm_ks.h; c = 256: four stages per wavefront): a
-// workgroup takes 32 rows x 32 pairs (their a- and b-columns) of one degree.  The weight fragments of the
-// wavefront's stages stay in registers over the degree's m-rows, the next m-row's A fragments load while the
+// The same for few rows and three pieces, K split over the wavefronts (gemm_ks.h; c = 256: four stages per
+// wavefront): a workgroup takes 32 rows x 32 pairs (their a- and b-columns) of one degree.  The weight fragments of
+// the wavefront's stages stay in registers over the degree's m-rows, the next m-row's A fragments load while the
 // current one multiplies, and the partial sums of an m-row meet in one of two LDS buffers (one barrier per
 // m-row), where wavefront w finishes rows 8 w .. 8 w + 7 of both column tiles: y, and a b into the pair sums.
-template <int kP, bool kYB>
 __global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_fwd(const float* __restrict__ x, const void* __restrict__ wp,
-                                                             const float* __restrict__ bias, void* __restrict__ y,
+                                                             const float* __restrict__ bias, float* __restrict__ y,
                                                              float* __restrict__ hq, float* __restrict__ hk, int n,
                                                              int hid) {
-  constexpr int c = 256, nks = c / kGK, kSt = nks / kKsW, kN = 32;
+  constexpr int kP = 3, c = 256, nks = c / kGK, kSt = nks / kKsW, kN = 32;
   __shared__ float red[2][kKsW * kN * 64];
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5;
   const int n_mt = (n + 31) / 32, n_ps = 2 * hid / 32, tiles = n_mt * n_ps;
@@ -551,17 +563,12 @@ __global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_fwd(const float* __rest
     ks_flat(acc, part);
     // wavefront w finishes registers 4 w .. 4 w + 3 of both column tiles
     ks_reduce<kN, kKsW>(red[m & 1], part, wv, lane, [](int w, int i) { return 16 * (i / 4) + 4 * w + i % 4; }, sum);
-    float* ym = static_cast<float*>(y) + (kYB ? 0 : (size_t)m * n * O);
-    __bf16* ymb = static_cast<__bf16*>(y) + (kYB ? (size_t)m * n * O : 0);
+    float* ym = y + (size_t)m * n * O;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int ab = i / 4, row = row0 + acc_row(4 * wv + i % 4, lane);
       if (m == 0 && bias) sum[i] += bias[128 * (ps / 2) + 64 * ab + 32 * (ps % 2) + (lane & 31)];
-      if (row < n) {
-        const size_t o = (size_t)row * O + pair_pos(p0, ab);
-        if constexpr (kYB) ymb[o] = (__bf16)sum[i];
-        else ym[o] = sum[i];
-      }
+      if (row < n) ym[(size_t)row * O + pair_pos(p0, ab)] = sum[i];
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) sp[i] = fmaf(sum[i], sum[4 + i], sp[i]);
@@ -671,14 +678,14 @@ __global__ __launch_bounds__(kGT, 2) void k_qk_s3_bwd(const void* __restrict__ y
   }
 }
 
-// The same for few rows: a 32 x 64 tile of one m-row, K (the pair columns, then the value projection's) split
-// over the wavefronts (gemm_ks.h).  A lane reads its row's partner values of y and the eight g values itself.
-template <int kP, bool kYB, int kD>
-__global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_bwd(const void* __restrict__ y, const float* __restrict__ ghq,
-                                                          const float* __restrict__ ghk, const void* __restrict__ wp,
-                                                          const float* __restrict__ gv, float* __restrict__ gx, int n,
-                                                          int hid, int c, int cv) {
-  constexpr int kW = kKsW, kN = 16 * kKsJ;
+// The same for few rows and three pieces: a 32 x 64 tile of one m-row, K (the pair columns, then the value
+// projection's) split over the wavefronts (gemm_ks.h).  A lane reads its row's partner values of y and the eight g
+// values itself.
+__global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_bwd(const float* __restrict__ y, const float* __restrict__ ghq,
+                                                             const float* __restrict__ ghk,
+                                                             const void* __restrict__ wp, const float* __restrict__ gv,
+                                                             float* __restrict__ gx, int n, int hid, int c, int cv) {
+  constexpr int kP = 3, kD = kKsD3, kW = kKsW, kN = 16 * kKsJ;
   __shared__ float red[kW * kN * 64];
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5;
   const int n_mt = (n + 31) / 32, n_ct = c / (32 * kKsJ), tiles = 9 * n_mt * n_ct;
@@ -687,12 +694,10 @@ __global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_bwd(const void* __restr
   const int ct = tile % n_ct, mt = (tile / n_ct) % n_mt, m = tile / (n_ct * n_mt);
   const int l = m == 0 ? 0 : (m < 4 ? 1 : 2);
   const int O = 4 * hid, row0 = mt * 32, nk1 = O / kGK, nks_w = nk1 + cv / kGK, r = lane & 31;
-  const __amdgpu_buffer_rsrc_t yr =
-      kYB ? rows_rsrc_bf(static_cast<const __bf16*>(y) + (size_t)m * n * O, row0, n, O)
-          : rows_rsrc(static_cast<const float*>(y) + (size_t)m * n * O, row0, n, O);
+  const __amdgpu_buffer_rsrc_t yr = rows_rsrc(y + (size_t)m * n * O, row0, n, O);
   const __amdgpu_buffer_rsrc_t qr = rows_rsrc(ghq, row0, n, 3 * hid), kr = rows_rsrc(ghk, row0, n, 3 * hid);
   const __amdgpu_buffer_rsrc_t br = b_rsrc<kP>(wp, l, c / kGN, ct * 32 * kKsJ / kGN, nks_w);
-  const uint32_t yoff = (uint32_t)(r * O + 8 * (1 - h)) * (kYB ? 2u : 4u);      // the partner half of the stage
+  const uint32_t yoff = (uint32_t)(r * O + 8 * (1 - h)) * 4u;      // the partner half of the stage
   const uint32_t voff = (uint32_t)(r * cv + 8 * h) * 4u, goff = (uint32_t)(r * 3 * hid + l * hid) * 4u;
   uint32_t boff[kKsJ];
 #pragma unroll
@@ -710,28 +715,12 @@ __global__ __launch_bounds__(kKsThreads, 2) void k_qk_ks_bwd(const void* __restr
   ks_loop<kP, 1, kKsJ, kD, Raw>(
       br, boff, ks0, ks0 + own,
       [&](int ks, int, Raw& a) {
-        if constexpr (kYB) {
-          a.x0 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 2u));
-        } else {
-          a.x0 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 4u));
-          a.x1 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 4u) + 16u);
-        }
+        a.x0 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 4u));
+        a.x1 = ks_load4(yr, yoff + (uint32_t)ks * (kGK * 4u) + 16u);
         a.g0 = ks_load4(gr, goff2 + (uint32_t)ks * 32u);
         a.g1 = ks_load4(gr, goff2 + (uint32_t)ks * 32u + 16u);
       },
-      [&](int, int, const Raw& a, bf16x8 (&p)[kP]) {
-        floatx4 x0 = a.x0, x1 = a.x1;
-        if constexpr (kYB) {
-          const bf16x8 yb = __builtin_bit_cast(bf16x8, a.x0);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            x0[u] = (float)yb[u];
-            x1[u] = (float)yb[4 + u];
-          }
-        }
-        split_pieces<kP>(x0 * a.g0, x1 * a.g1, p);
-      },
-      acc);
+      [&](int, int, const Raw& a, bf16x8 (&p)[kP]) { split_pieces<kP>(a.x0 * a.g0, a.x1 * a.g1, p); }, acc);
   if (gv) {
     struct RawV {
       floatx4 x0, x1;
@@ -840,23 +829,29 @@ int check_gemm_args(const e2v2_gemm_args& G) {
 }
 int host_tiles(const e2v2_gemm_args& G) { return G.batch * ((G.m + kGM - 1) / kGM) * (G.n / kGN); }
 
-// Which matrices take the K-split tiles (gemm_ks.h): few rows, decided by the rows alone so that a GEMM is
-// summed in the same order whether it runs alone, as a batch member or in a group.  Measured (us per call,
-// 128 x 128 tiles against K-split, operands not in L2):
+// Which matrices take the few-row tiles (gemm_ks.h), decided by the rows alone so that a GEMM is summed in the same
+// order whether it runs alone, as a batch member or in a group.  Measured (us per call, 128 x 128 tiles against
+// few-row tiles, operands not in L2):
 //   three pieces, 9 batches, K 256 -> 256:  m 24: 19.0 / 5.9, 648: 24.3 / 11.1, 1500: 26.0 / 19.8,
 //                                           2500: 31.9 / 30.0, 3318: 33.0 / 34.7, 10000: 86.8 / 110
 //   three pieces, 2 batches, K 1536 -> 512: m 24: 61.4 / 14.7, 648: 78.7 / 28.6, 2500: 81.2 / 66.8, 3318: 82.4 / 88.6
-//   one piece, fp32 A, 9 x 256 -> 256:      m 24: 15.2 / 4.8, 1500: 22.1 / 15.5, 2500: 24.0 / 23.6, 3318: 23.5 / 25.9
-//   one piece, bf16 A, 9 x 256 -> 256:      m 24: 14.2 / 4.4, 2500: 20.9 / 15.8, 3318: 21.6 / 18.9, 5000: 23.8 / 26.1
-// Above that the K-split form's fourfold operand traffic per product costs more than the stages it saves.
-constexpr int kKsRows = 2560, kKsRowsBf16 = 3584;
-bool ks_gemm(const e2v2_gemm_args& G) { return G.m <= (G.a_bf16 ? kKsRowsBf16 : kKsRows); }
-// The Q/K projection (three pieces, forward and backward): n 24: 60.2 / 11.8 and 106.6 / 22.8, 648: 79.5 / 57.3 and
-// 122 / 86, 1000: 90.1 / 84.5 and 134 / 132, 1500: 113 / 116 and 136 / 184 (one piece alike: 24: 35.4 / 8.0 and
-// 58.6 / 14.7, 1000: 58.5 / 55.4 and 97.4 / 85.7, 1500: 64.8 / 76.4 and 99.6 / 119).
+// Above that the K-split form's fourfold operand traffic per product costs more than the stages it saves.  (At that
+// switch an fp32 row's last bits change with the rows that share its call.)  One piece keeps the order of the sum, so
+// a wavefront walks all of K and the switch lies lower:
+//   fp32 A, 9 x 256 -> 256: m 24: 13.4 / 6.5, 648: 18.1 / 12.4, 1000: 18.6 / 16.9, 1500: 19.4 / 21.5
+//   fp32 A, 2 x 1536 -> 512: m 24: 29.9 / 22.7, 1000: 41.0 / 27.9, 1500: 44.3 / 51.3
+//   gated, 9 x 256 -> 256:  m 24: 18.3 / 10.8, 648: 26.5 / 21.3, 1000: 27.1 / 29.2
+//   bf16 A, 9 x 256 -> 256: m 24: 12.8 / 6.0, 1500: 18.2 / 15.8, 2048: 20.3 / 18.6, 2500: 21.8 / 22.1
+//   bf16 A, 5 x 2560 -> 256: m 24: 37.8 / 22.4, 1500: 74.3 / 54.4, 2048: 78.0 / 83.7
+constexpr int kKsRows = 2560, kFewRows = 1024, kFewRowsGated = 768, kFewRowsBf16 = 1536;
+bool ks_gemm(const e2v2_gemm_args& G, bool gated = false) {
+  return G.m <= (G.pieces == 3 ? kKsRows : gated ? kFewRowsGated : G.a_bf16 ? kFewRowsBf16 : kFewRows);
+}
+// The Q/K projection with three pieces (forward and backward): n 24: 60.2 / 11.8 and 106.6 / 22.8, 648: 79.5 / 57.3
+// and 122 / 86, 1000: 90.1 / 84.5 and 134 / 132, 1500: 113 / 116 and 136 / 184.  With one piece the 128 x 128 tiles
+// at every size (28.5 and 51.7 us at 24 rows; few-row tiles with K in one order 23.1 and 42.6, 42.4 and 104.5 against
+// 38.3 and 72.0 at 648).
 constexpr int kKsQkRows = 1024;
-// Ring depths: with three pieces two stages in flight leave four workgroups per CU; one piece takes four.
-constexpr int kKsD3 = 2, kKsD1 = 4;
 }  // namespace
 }  // namespace e2v2
 
@@ -909,7 +904,7 @@ E2V2_API int e2v2_gemm_s3_gated(const e2v2_gemm_args* g, const float* s, int64_t
   E2V2_REQUIRE((uint64_t)(G.m + kGM) * (uint64_t)ld_s * 4u < (1ull << 31), "gemm_s3_gated: logits too large (m=%d)",
                G.m);
   if (G.m == 0) return 0;
-  if (ks_gemm(G)) {
+  if (ks_gemm(G, true)) {
     const dim3 grid(xcd_grid(ks_tiles(G)));
     if (G.pieces == 3)
       hipLaunchKernelGGL((k_gemm_ks_gate<3, kKsD3>), grid, dim3(kKsThreads), 0, st, G, GateOp{s, ld_s, k1, k2});
@@ -985,14 +980,9 @@ E2V2_API int e2v2_qk_proj_fwd_s3(const float* x, const void* wp, const float* bi
   E2V2_REQUIRE(n >= 0 && (uint64_t)(n + kGM) * (uint64_t)c * 4u < (1ull << 31) &&
                    (uint64_t)(n + kGM) * 4u * hid < (1ull << 32), "qk_proj_fwd_s3: n=%d too large", n);
   if (n == 0) return 0;
-  if (n <= kKsQkRows && c == 256) {
-    const dim3 grid(3 * xcd_grid(((n + 31) / 32) * (2 * hid / 32)));
-    if (pieces == 3)
-      hipLaunchKernelGGL((k_qk_ks_fwd<3, false>), grid, dim3(kKsThreads), 0, s, x, wp, bias, y, hq, hk, n, hid);
-    else if (y_bf16)
-      hipLaunchKernelGGL((k_qk_ks_fwd<1, true>), grid, dim3(kKsThreads), 0, s, x, wp, bias, y, hq, hk, n, hid);
-    else
-      hipLaunchKernelGGL((k_qk_ks_fwd<1, false>), grid, dim3(kKsThreads), 0, s, x, wp, bias, y, hq, hk, n, hid);
+  if (n <= kKsQkRows && pieces == 3 && c == 256) {
+    hipLaunchKernelGGL(k_qk_ks_fwd, dim3(3 * xcd_grid(((n + 31) / 32) * (2 * hid / 32))), dim3(kKsThreads), 0, s, x, wp,
+                       bias, static_cast<float*>(y), hq, hk, n, hid);
     E2V2_LAUNCHED("k_qk_ks_fwd");
     return 0;
   }
@@ -1026,14 +1016,9 @@ E2V2_API int e2v2_qk_proj_bwd_s3(const void* y, const float* ghq, const float* g
   E2V2_REQUIRE(n >= 0 && (uint64_t)(n + kGM) * 4u * hid * 4u < (1ull << 31) &&
                    (uint64_t)(n + kGM) * (uint64_t)cv * 4u < (1ull << 31), "qk_proj_bwd_s3: n=%d too large", n);
   if (n == 0) return 0;
-  if (n <= kKsQkRows) {
-    const dim3 grid(xcd_grid(9 * ((n + 31) / 32) * (c / (32 * kKsJ)))), blk(kKsThreads);
-    if (pieces == 3)
-      hipLaunchKernelGGL((k_qk_ks_bwd<3, false, 2>), grid, blk, 0, s, y, ghq, ghk, wp, gv, gx, n, hid, c, cv);
-    else if (y_bf16)
-      hipLaunchKernelGGL((k_qk_ks_bwd<1, true, 2>), grid, blk, 0, s, y, ghq, ghk, wp, gv, gx, n, hid, c, cv);
-    else
-      hipLaunchKernelGGL((k_qk_ks_bwd<1, false, 2>), grid, blk, 0, s, y, ghq, ghk, wp, gv, gx, n, hid, c, cv);
+  if (n <= kKsQkRows && pieces == 3) {
+    hipLaunchKernelGGL(k_qk_ks_bwd, dim3(xcd_grid(9 * ((n + 31) / 32) * (c / (32 * kKsJ)))), dim3(kKsThreads), 0, s,
+                       static_cast<const float*>(y), ghq, ghk, wp, gv, gx, n, hid, c, cv);
     E2V2_LAUNCHED("k_qk_ks_bwd");
     return 0;
   }

@@ -1,4 +1,5 @@
-// K-split tiles of the split-bf16 GEMMs for matrices of few rows (gemm.hip).
+// Tiles of the split-bf16 GEMMs for matrices of few rows (gemm.hip): K split over the wavefronts for three operand
+// pieces, in one order for one piece.
 //
 // A 128 x 128 tile of gemm_core.h walks K in stages of 16 one after another, a barrier and the latency of its
 // two-stages-ahead loads per stage: about 2 us a stage when the operands come from the Infinity Cache, 33 us
@@ -9,7 +10,8 @@
 // loop; the four partial tiles meet once in LDS, where wavefront w adds a quarter of the tile's registers in
 // wavefront order.  The packed weight is read as it lies (a 32-column subtile of a piece is 1 KB contiguous).
 // The products, their pieces and the order inside a wavefront are those of kloop; the sum over K is the sum
-// of four shorter ones in fixed order.
+// of four shorter ones in fixed order.  With one piece the wavefronts take a column subtile each and all of K, so
+// that the sum is kloop's bit by bit.
 #pragma once
 #include "gemm_core.h"
 

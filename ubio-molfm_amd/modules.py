@@ -1931,7 +1931,7 @@ class EdgeDegreeEmbeddingNetwork_higherorder(nn.Module):
         # the edge spherical harmonics ("e3nn sph") are formed inside the degree kernels
         with record_function("e3nn sph"):
             return DegreeEmbedFn.apply(ctx.dvec, ctx.dist, ctx.nl, ctx.atom_type, table,
-                                       float(self.avg_aggregate_num), ctx.rc)
+                                       float(self.avg_aggregate_num), ctx.rc, ctx.bf16)
 
 
 class E2former(nn.Module):

@@ -282,12 +282,15 @@ class DegreeEmbedFn(torch.autograd.Function):
     The backward runs the transposed GEMM (grad_h = grad_x0 W3_l) and the bias
     column's grad_s = grad_x0 . b3_l before the edge kernel.  A "deg" table (the
     profiles' outputs) runs e2v2_deg_fwd / e2v2_deg_bwd directly.  Nothing per edge
-    is saved."""
+    is saved.  one_order (the bf16 mode): a node's sums keep their order whatever the
+    number of nodes (``gemm.gemm``'s padded_rows), as the layers that round them to
+    bf16 do."""
 
     WIDX = (0, 1, 1, 1, 2, 2, 2, 2, 2)   # profile of each m-row
 
     @staticmethod
-    def forward(ctx, dvec, dist, nl: NeighborList, atom_type, table: RadialTable, avg: float, rc: float):
+    def forward(ctx, dvec, dist, nl: NeighborList, atom_type, table: RadialTable, avg: float, rc: float,
+                one_order: bool = False):
         _need_cuda(dvec, dist)
         dev = dvec.device
         dargs = deg_args(nl, atom_type, table, avg, rc)
@@ -297,11 +300,11 @@ class DegreeEmbedFn(torch.autograd.Function):
             hs = torch.empty(9, N, 144, dtype=torch.float32, device=dev)
             _lib.call("e2v2_deg_hidden_fwd", _lib.C.byref(dargs), _p(hs), _stream(hs))
             if N:
-                gemm.gemm(hs, table.w3_pack, x0, DegreeEmbedFn.WIDX)
+                gemm.gemm(hs, table.w3_pack, x0, DegreeEmbedFn.WIDX, padded_rows=one_order)
             del hs
         else:
             _lib.call("e2v2_deg_fwd", _lib.C.byref(dargs), _p(x0), _stream(x0))
-        ctx.nl, ctx.atom_type, ctx.table, ctx.avg, ctx.rc = nl, atom_type, table, avg, rc
+        ctx.nl, ctx.atom_type, ctx.table, ctx.avg, ctx.rc, ctx.one_order = nl, atom_type, table, avg, rc, one_order
         return x0
 
     @staticmethod
@@ -320,7 +323,7 @@ class DegreeEmbedFn(torch.autograd.Function):
             gh = torch.empty(9, N, 128, dtype=torch.float32, device=dev)
             gs = torch.empty(9, max(N, 1), dtype=torch.float32, device=dev)
             if N:
-                gemm.gemm(gx0, table.w3t_pack, gh, DegreeEmbedFn.WIDX)
+                gemm.gemm(gx0, table.w3t_pack, gh, DegreeEmbedFn.WIDX, padded_rows=ctx.one_order)
             _lib.call("e2v2_deg_bias_grad", _p(gx0), _p(table.b3), _lib.i32(N), _p(gs), _stream(gx0))
             _lib.call("e2v2_deg_hidden_bwd", _lib.C.byref(dargs), _p(gh), _p(gs), _p(ddv), _p(dd), _p(ws),
                       _lib.C.c_size_t(ws.numel()), _stream(gx0))
@@ -329,7 +332,7 @@ class DegreeEmbedFn(torch.autograd.Function):
             _lib.call("e2v2_deg_bwd", _lib.C.byref(dargs), _p(gx0), _p(ddv), _p(dd), _p(ws),
                       _lib.C.c_size_t(ws.numel()), _stream(gx0))
         del ws
-        return ddv[:E], dd[:E], None, None, None, None, None
+        return ddv[:E], dd[:E], None, None, None, None, None, None
 
 
 def deg_args(nl: NeighborList, atom_type: torch.Tensor, table: RadialTable, avg: float, rc: float):
