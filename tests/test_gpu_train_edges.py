@@ -118,6 +118,31 @@ def test_attention_weights(pkg, cuda, n, separate):
                  [torch.cat([gate, ih], 1), qk, p], g, cuda)
 
 
+@pytest.mark.parametrize("through", ["function", "dispatch"])
+def test_attention_weights_of_strided_operands(pkg, cuda, through):
+    """Operands that are halves of wider tensors (QKdotS_alpha's inputhead) or transposed: their gradients of both
+    orders reach the tensors they are views of."""
+    from ubio_molfm_amd import second_order as so
+    n = 61
+    e, row, col, g = _edges(n, 71, cuda)
+    E = e.E
+    ins = [torch.randn(*s, generator=g, dtype=torch.float64).float().double() for s in ((E, 2 * H), (H, E), (2, E, H))]
+    p = torch.rand(E, 2, generator=g, dtype=torch.float64).float().double()
+
+    def views(wide, gate, both, pp):
+        return wide.tanh().split(H, 1)[0], gate.tanh().t(), both.tanh()[1], pp.sqrt()[:, 1]
+
+    def fn(*t):
+        i, ga, q, pp = views(*t)
+        return so._AttnWeightsFn.apply(i, ga, q, pp, e) if through == "function" else \
+            so.attention_weights(i, ga, q, pp, e, "softmax")
+
+    def ref(*t):
+        i, ga, q, pp = views(*t)
+        return ref_alpha(ga, i, q, pp, row, n)
+    _compare(fn, ref, [*ins, p + 0.05], g, cuda)
+
+
 @pytest.mark.parametrize("value", [float("-inf"), float("inf"), float("nan")])
 @pytest.mark.parametrize("where", ["first", "last", "one_group", "all"])
 def test_attention_weights_of_logits_that_are_not_finite(pkg, cuda, value, where):
@@ -173,3 +198,25 @@ def test_third_order(pkg, cuda):
                       (third(lambda t: so._AttnWeightsFn.apply(dev[2], None, t, dev[3], e), qk.to(cuda, torch.float32)),
                        third(lambda t: ref_alpha(eg[:, :H], eg[:, H:], t, p, row, n), qk))):
         assert float((got.double().cpu() - want).norm() / want.norm()) < 10 * TOL
+
+
+def test_third_order_of_a_strided_gradient(pkg, cuda):
+    """The same with gradients that reach the functions as transposed tensors: the copies that the kernels read
+    belong to no graph."""
+    from ubio_molfm_amd import second_order as so
+    e, row, col, g = _edges(5, 4, cuda)
+    E, n = e.E, e.N
+    e.qi = row.to(cuda)
+    eg, qk, p = (0.5 * torch.randn(*s, generator=g, dtype=torch.float64) for s in ((E, 2 * H), (E, H), (E,)))
+    p = p.abs() + 0.1
+
+    def third(fn, x):
+        x = x.clone().requires_grad_(True)
+        y = fn(x).t().clone(memory_format=torch.contiguous_format).sin()      # (its gradient comes back transposed)
+        d, = torch.autograd.grad(y.sum(), x, create_graph=True)
+        d2, = torch.autograd.grad(d.pow(2).sum(), x, create_graph=True)
+        return torch.autograd.grad(d2.pow(2).sum(), x)[0]
+    dev = [t.to(cuda, torch.float32) for t in (eg, p, qk)]
+    got = third(lambda t: so._AttnWeightsFn.apply(dev[0], None, t, dev[1], e), dev[2])
+    want = third(lambda t: ref_alpha(eg[:, :H], eg[:, H:], t, p, row, n), qk)
+    assert float((got.double().cpu() - want).norm() / want.norm()) < 10 * TOL

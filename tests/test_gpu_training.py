@@ -177,6 +177,15 @@ def test_training_second_order_qkdots_softplus(pkg, cuda):
           tp_type="QKdotS_alpha+softplus", attn_type="so2-first-order+zero-order")
 
 
+def test_training_second_order_qkdots_softmax(pkg, cuda):
+    """QKdotS_alpha with the softmax: its inputhead is a half of fc_easy's columns."""
+    from ubio_molfm_amd import systems
+    names = PARAMS + ["decoder.decoder.blocks.1.ga.direction_linear.0.weight",
+                      "decoder.decoder.blocks.3.ga.fc_easy.net.6.weight",
+                      "decoder.decoder.blocks.2.ga.source_embedding.weight"]
+    _case(cuda, systems.small_water(6, 5.6, seed=25), 35, "qkdots-softmax", names, tp_type="QKdotS_alpha")
+
+
 @pytest.mark.parametrize("w", [64, 128, 192, 512])
 def test_ln_silu_second_order(pkg, cuda, w):
     """ln_silu (the fused LayerNorm + SiLU of the radial nets on the training

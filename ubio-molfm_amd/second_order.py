@@ -681,6 +681,19 @@ class EdgeInput:
         return run_seq(net[1:], h)
 
 
+def _dense(*ts):
+    """The operands as the kernels read them: contiguous, on 16-byte boundaries.  For the call only: what is saved for
+    a backward is the operand itself, since a copy made inside a Function has no history and would end the graph of
+    the next order there."""
+    out = []
+    for t in ts:
+        if t is not None:
+            t = t.contiguous()
+            t = t.clone() if t.data_ptr() % 16 else t
+        out.append(t)
+    return out
+
+
 class _AddGathersFn(torch.autograd.Function):
     """y + xq[qi] + xk[nj] in one pass (e2v2_add_gather2); linear, so its gradient (the identity and the two
     segment sums) and theirs are this function and sums again."""
@@ -725,14 +738,14 @@ class _AttnWeightsFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, eg, gate, qk, p, edges):
-        eg, qk, p = eg.contiguous(), qk.contiguous(), p.contiguous()
-        gate = None if gate is None else gate.contiguous()
+        ins = (eg, gate, qk, p)
+        eg, gate, qk, p = _dense(*ins)
         N, E, H = edges.N, edges.E, qk.shape[1]
         alpha = torch.empty_like(qk)
         m, s, ties = (qk.new_empty(N, H) for _ in range(3))
         _lib.call("e2v2_attn_weights_fwd", *_aw_args(edges, eg, gate, qk, p), _p(alpha), _p(m), _p(s), _p(ties),
                   sparse_ops._stream(qk.device))
-        ctx.save_for_backward(eg, gate, qk, p, m, s, ties)
+        ctx.save_for_backward(*ins, m, s, ties)
         ctx.edges = edges
         return alpha
 
@@ -758,12 +771,13 @@ class _AttnWeightsGradFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, g, eg, gate, qk, p, m, s, ties, edges):
-        g = g.contiguous()
+        ins = (g, eg, gate, qk, p)
+        g, eg, gate, qk, p = _dense(*ins)
         deg, dqk, dp = torch.empty_like(eg), torch.empty_like(qk), torch.empty_like(p)
         dgate = None if gate is None else torch.empty_like(gate)
         _lib.call("e2v2_attn_weights_bwd", *_aw_args(edges, eg, gate, qk, p), _p(m), _p(s), _p(ties), _p(g),
                   *_aw_pair(deg, dgate), _p(dqk), _p(dp), sparse_ops._stream(g.device))
-        ctx.save_for_backward(g, eg, gate, qk, p, m, s, ties)
+        ctx.save_for_backward(*ins, m, s, ties)
         ctx.edges = edges
         ctx.set_materialize_grads(False)
         return deg, dgate, dqk, dp
@@ -783,7 +797,7 @@ class _AttnWeightsGradFn(torch.autograd.Function):
             f = iter(torch.autograd.grad([x for x, _ in pick], [t for t, r in zip(args, diff) if r],
                                          [c for _, c in pick], create_graph=True, allow_unused=True))
             return (*(next(f) if r else None for r in diff), None, None, None, None)
-        ceg, cgate, cqk, cp = (None if t is None else t.contiguous() for t in (ceg, cgate, cqk, cp))
+        g, eg, gate, qk, p, ceg, cgate, cqk, cp = _dense(g, eg, gate, qk, p, ceg, cgate, cqk, cp)
         fg, feg, fqk, fp = torch.empty_like(g), torch.empty_like(eg), torch.empty_like(qk), torch.empty_like(p)
         fgate = None if gate is None else torch.empty_like(gate)
         _lib.call("e2v2_attn_weights_bwd2", *_aw_args(ctx.edges, eg, gate, qk, p), _p(m), _p(s), _p(ties), _p(g),
@@ -901,7 +915,8 @@ def attention_weights(eg, gate, qk, p, edges: TrainEdges, form: str) -> torch.Te
     H = qk.shape[1]
     if (form == "softmax" and H == 128 and qk.is_cuda and all(t.dtype == torch.float32 for t in (eg, qk, p))
             and (gate is None or gate.dtype == torch.float32)):
-        return _AttnWeightsFn.apply(eg, gate, qk, p, edges)
+        # (QKdotS_alpha's inputhead is a half of a wider tensor's columns: dense here, so that no pass copies it again)
+        return _AttnWeightsFn.apply(eg.contiguous(), gate, qk, p, edges)
     if form == "softmax":
         return _softmax_weights(eg, gate, qk, p, edges)
     gate, ih = eg.split([H, eg.shape[1] - H], dim=1) if gate is None else (gate, eg)
