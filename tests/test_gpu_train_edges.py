@@ -220,3 +220,23 @@ def test_third_order_of_a_strided_gradient(pkg, cuda):
     got = third(lambda t: so._AttnWeightsFn.apply(dev[0], None, t, dev[1], e), dev[2])
     want = third(lambda t: ref_alpha(eg[:, :H], eg[:, H:], t, p, row, n), qk)
     assert float((got.double().cpu() - want).norm() / want.norm()) < 10 * TOL
+
+
+def test_value_aggregation_of_strided_operands_to_third_order(pkg, cuda):
+    from ubio_molfm_amd import second_order as so
+    e, row, col, g = _edges(5, 6, cuda)
+    E, n = e.E, e.N
+    ins = [0.5 * torch.randn(*s, generator=g, dtype=torch.float64) for s in ((H, E), (E, 4), (n, 9, C))]
+
+    def chain(fn, ins):
+        x = [t.clone().requires_grad_(True) for t in ins]
+        y = fn(x[0].tanh().t(), x[1].tanh()[:, 1:], x[2].tanh().permute(1, 0, 2))
+        z = y.transpose(-1, -2).clone(memory_format=torch.contiguous_format).sin()
+        d1 = torch.autograd.grad(z.sum(), x, create_graph=True)
+        d2 = torch.autograd.grad(sum(t.pow(2).sum() for t in d1), x, create_graph=True)
+        return [t.detach() for t in (y, *d1, *d2, *torch.autograd.grad(sum(t.pow(2).sum() for t in d2), x))]
+    got = chain(lambda w, u, v: so._So2AggFn.apply(w, u, v, e), [t.to(cuda, torch.float32) for t in ins])
+    for i, (a, b) in enumerate(zip(got, chain(lambda w, u, v: ref_aggregation(w, u, v, row, col), ins))):
+        rel = float((a.double().cpu() - b).norm() / b.norm())
+        print(i, f"{rel:.2e}", flush=True)
+        assert rel < 10 * TOL

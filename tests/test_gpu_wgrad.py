@@ -110,3 +110,41 @@ def test_so3_linear_to_third_order(pkg, cuda, n):
         print(n, i, f"{rel:.2e}", flush=True)
         # relative error of a sum of at most 9 n x 128 products per order, orders chained three deep
         assert rel < 1e-5
+
+
+@pytest.mark.parametrize("name", ["m_contraction", "m_expansion", "weight_gradient"])
+def test_third_order_of_strided_operands(pkg, cuda, name):
+    """Operands that are views, and incoming gradients that are transposed: the copies that the kernels read belong
+    to no graph.  Bound as above."""
+    from ubio_molfm_amd import second_order as so
+    g = torch.Generator().manual_seed(7)
+    n, w = 13, 64
+    shapes = {"m_contraction": ((n, 9, w), (n, 9, w)), "m_expansion": ((3 * w, n), (n, 9, w)),
+              "weight_gradient": ((n, 9, w), (n, 9, w))}[name]
+    ins = [0.3 * torch.randn(s, generator=g) for s in shapes]
+
+    def of(t):
+        return t.tanh().t() if t.dim() == 2 else t.tanh().permute(1, 0, 2)
+
+    def compose(a, b):
+        if name == "m_contraction":
+            return torch.cat([p.sum(0) for p in (a * b).split([1, 3, 5])], dim=-1)
+        if name == "m_expansion":
+            return torch.cat([a.view(n, 3, w)[:, l].unsqueeze(0) * b[l * l:(l + 1) ** 2] for l in range(3)])
+        return torch.stack([(a[p:q].reshape(-1, w).t().contiguous() @ b[p:q].reshape(-1, w).contiguous())
+                            for p, q in ((0, 1), (1, 4), (4, 9))])
+    fn = {"m_contraction": so._MDotFn, "m_expansion": so._MExpandFn, "weight_gradient": so._DegreeWGradFn}[name].apply
+
+    def chain(f, ins):
+        x = [t.clone().requires_grad_(True) for t in ins]
+        y = f(*map(of, x))
+        z = y.transpose(-1, -2).clone(memory_format=torch.contiguous_format).sin()    # (its gradient: transposed)
+        d1 = torch.autograd.grad(z.sum(), x, create_graph=True)
+        d2 = torch.autograd.grad(sum(t.pow(2).sum() for t in d1), x, create_graph=True)
+        return [t.detach() for t in (y, *d1, *d2, *torch.autograd.grad(sum(t.pow(2).sum() for t in d2), x))]
+
+    got = chain(fn, [t.to(cuda) for t in ins])
+    for i, (a, b) in enumerate(zip(got, chain(compose, [t.double() for t in ins]))):
+        rel = float((a.double().cpu() - b).norm() / b.norm())
+        print(name, i, f"{rel:.2e}", flush=True)
+        assert rel < 1e-5

@@ -272,6 +272,19 @@ def _cartesian(device) -> torch.Tensor:
 _DEGREE_ROWS = (0, 1, 4, 9)      # bounds of the m-rows of each degree
 
 
+def _dense(*ts):
+    """The operands as the kernels read them: contiguous, on 16-byte boundaries.  For the call only: what is saved for
+    a backward is the operand itself, since a copy made inside a Function has no history and would end the graph of
+    the next order there."""
+    out = []
+    for t in ts:
+        if t is not None:
+            t = t.contiguous()
+            t = t.clone() if t.data_ptr() % 16 else t
+        out.append(t)
+    return out
+
+
 class _DegreeMmFn(torch.autograd.Function):
     """y [9, N, O] with y[m] = x[m] W_l(m)^T, W [3, O, K] (``t``: x[m] W_l(m), W [3, K, O]), the bias added to row 0;
     We is W with its rows expanded to the m-rows.  Gradients of any order: the input gradient is this function with
@@ -304,8 +317,8 @@ class _DegreeWGradFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, a, b):
-        a, b = a.contiguous(), b.contiguous()
         ctx.save_for_backward(a, b)
+        a, b = _dense(a, b)
         M, n, m = a.shape
         k = b.shape[2]
         chunks = int(_lib.load().e2v2_wgrad_chunks(n, M, m, k))
@@ -355,8 +368,8 @@ class _MDotFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, a, b):
-        a, b = a.contiguous(), b.contiguous()
         ctx.save_for_backward(a, b)
+        a, b = _dense(a, b)
         h = a.new_empty(a.shape[1], 3 * a.shape[2])
         _lib.call("e2v2_mdot", _p(a), _p(b), _lib.i32(a.shape[1]), _lib.i32(a.shape[2]), _p(h),
                   sparse_ops._stream(a.device))
@@ -374,8 +387,8 @@ class _MExpandFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, h, b):
-        h, b = h.contiguous(), b.contiguous()
         ctx.save_for_backward(h, b)
+        h, b = _dense(h, b)
         y = torch.empty_like(b)
         _lib.call("e2v2_mexpand", _p(h), _p(b), _lib.i32(b.shape[1]), _lib.i32(b.shape[2]), _p(y),
                   sparse_ops._stream(b.device))
@@ -681,19 +694,6 @@ class EdgeInput:
         return run_seq(net[1:], h)
 
 
-def _dense(*ts):
-    """The operands as the kernels read them: contiguous, on 16-byte boundaries.  For the call only: what is saved for
-    a backward is the operand itself, since a copy made inside a Function has no history and would end the graph of
-    the next order there."""
-    out = []
-    for t in ts:
-        if t is not None:
-            t = t.contiguous()
-            t = t.clone() if t.data_ptr() % 16 else t
-        out.append(t)
-    return out
-
-
 class _AddGathersFn(torch.autograd.Function):
     """y + xq[qi] + xk[nj] in one pass (e2v2_add_gather2); linear, so its gradient (the identity and the two
     segment sums) and theirs are this function and sums again."""
@@ -701,8 +701,7 @@ class _AddGathersFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, y, xq, xk, edges):
         ctx.edges = edges
-        y = None if y is None else y.contiguous()
-        xq, xk = xq.contiguous(), xk.contiguous()
+        y, xq, xk = _dense(y, xq, xk)
         out = xq.new_empty(edges.E, xq.shape[1])
         _lib.call("e2v2_add_gather2", _p(y), _p(xq), _p(edges.row32), _p(xk), _p(edges.col32), _lib.i64(edges.E),
                   _lib.i32(xq.shape[1]), _p(out), sparse_ops._stream(xq.device))
@@ -813,9 +812,9 @@ class _So2AggFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, w, u, v, edges):
-        w, u, v = w.contiguous(), u.contiguous(), v.contiguous()
         ctx.save_for_backward(w, u, v)
         ctx.edges = edges
+        w, u, v = _dense(w, u, v)
         return _so2_agg(edges, v, ((w, u),))
 
     @staticmethod
@@ -854,10 +853,10 @@ class _So2AggGradFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, g, w, u, v, edges):
-        g = g.contiguous()
         ctx.save_for_backward(g, w, u, v)
         ctx.edges = edges
         ctx.set_materialize_grads(False)
+        g, w, u, v = _dense(g, w, u, v)
         dw, du = _so2_dw(edges, g, w, u, v)
         return dw, du, _so2_dv(edges, g, ((w, u),))
 
@@ -871,7 +870,7 @@ class _So2AggGradFn(torch.autograd.Function):
             dg = sum(_So2AggFn.apply(*t, e) for t in parts)
             (_, du1, dv1), (dw2, _, dv2), (dw3, du3, _) = (_So2AggGradFn.apply(g, *t, e) for t in parts)
             return dg, dw2 + dw3, du1 + du3, dv1 + dv2, None
-        qw, qu, qv = (None if t is None else t.contiguous() for t in (qw, qu, qv))
+        g, w, u, v, qw, qu, qv = _dense(g, w, u, v, qw, qu, qv)
         terms = ([(qw, u)] if qw is not None else []) + ([(w, qu)] if qu is not None else [])
         t2 = terms or [(None, None)]
         dg = _so2_agg(e, v, t2, (w, u, qv) if qv is not None else (None, None, None))
