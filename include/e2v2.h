@@ -464,13 +464,15 @@ typedef struct e2v2_attn_args {
 #define E2V2_SO2_LD(t) ((t) == 0 ? 256 : (t) < 10 ? 768 : 512)
 #define E2V2_SO2_COL(t) ((t) == 0 ? 0 : (t) < 10 ? 256 * (((t) - 1) / 3) : 256 * (((t) - 10) / 5))
 int e2v2_attn_fwd(const e2v2_attn_args* args, void* out, float* mrow, float* srow, int32_t* cnt, hipStream_t s);
-/* Bytes of device workspace e2v2_attn_bwd needs for n_edges edges (per-edge weights handed from the row
-   pass to the column pass and per-slice partial edge gradients, alive during the call only): 384 per edge, or
-   1,152 for at most 98,304 edges, whose four head groups run at once. */
+/* Bytes of device workspace to give e2v2_attn_bwd for n_edges edges (per-edge weights handed from the row
+   pass to the column pass and per-slice partial edge gradients, alive during the call only): 1,152 per edge for
+   at most 98,304 edges, whose four head groups then run at once, else 384.  384 per edge are enough for any
+   call (the head groups run in turn, with bitwise the same results), so a workspace sized for a longer list
+   serves a shorter one. */
 size_t e2v2_attn_bwd_workspace(int64_t n_edges);
 /* grad_out, out (l3-grouped as above; float, or bf16 if act_bf16) -> ddvec [E,3], ddist [E] (including the radial
    profile's distance derivative, from the table), dq, dk [N,H,D], dv [9][N][C] (all float, dv in slice
-   order); workspace: e2v2_attn_bwd_workspace(E) bytes, 16-byte aligned */
+   order); workspace: e2v2_attn_bwd_workspace(E) bytes, at least 384 E, 16-byte aligned */
 int e2v2_attn_bwd(const e2v2_attn_args* args, const void* grad_out, const void* out, const float* mrow,
                   const float* srow, const int32_t* cnt, float* ddvec, float* ddist, float* dq, float* dk, float* dv,
                   void* workspace, size_t workspace_bytes, hipStream_t s);

@@ -961,22 +961,22 @@ E2V2_API int e2v2_attn_fwd(const e2v2_attn_args* args, void* out, float* mrow, f
   });
 }
 
-// Up to this many edges the backward runs its four head groups in one row launch and one column launch, each
-// group with its own w / dqk pair: a group of a small system alone leaves most of the GPU idle (row + column
-// passes of a layer: 24 atoms 4 x (17.8 + 26.5) = 177 us, merged 47; 648 atoms, 59 k edges, 4 x (29.2 + 47.5) =
-// 307 us, merged 177).  Above it a group fills the GPU by itself (1,501 atoms, 128 k edges: 3,002 wavefronts of
-// the row pass at two per SIMD) and the pairs of four groups would be the largest per-edge allocation (1.2 KB per
-// edge instead of 384 B).
+// Up to this many edges, and where the workspace holds four w / dqk pairs, the backward runs its four head groups in
+// one row launch and one column launch, each group with its own pair: one group's launches leave part of the GPU idle
+// and their last round of workgroups four times over.  Row, column and sum passes of a layer, in turn / merged (us):
+// 24 atoms, 2 k edges 174 / 47; 648, 59 k 302 / 163; 900, 82 k 335 / 203; and beyond the line 1,401, 130 k 443 / 304;
+// 2,190, 205 k 652 / 465; 3,300, 304 k 810 / 696; 6,600, 608 k 1,572 / 1,518; 10,000, 924 k 2,290 / 2,287.  The line
+// is one of memory, not of time: four pairs are 1,152 bytes per edge (113 MB here) in place of 384, more than any other
+// per-edge array.  The sums and their order are the same.
 constexpr int64_t kMergeEdges = 98304;
-static int bwd_pairs(int64_t n_edges) { return n_edges <= kMergeEdges ? kGroups : 1; }
 // workspace of e2v2_attn_bwd: w [E][32] and dL/dqk [E][32] of one head group (of each, when merged), handed from
 // the row pass to the column pass, and the slice partials of dL/d dvec, dL/dd [8][E][4]
-static size_t bwd_ws_floats(int64_t n_edges) {
-  return (size_t)n_edges * (2 * kGroupHeads * bwd_pairs(n_edges) + 4 * kSl);
+static size_t bwd_ws_bytes(int64_t n_edges, int pairs) {
+  return n_edges > 0 ? (size_t)n_edges * (2 * kGroupHeads * pairs + 4 * kSl) * sizeof(float) : 0;
 }
 
 E2V2_API size_t e2v2_attn_bwd_workspace(int64_t n_edges) {
-  return n_edges > 0 ? bwd_ws_floats(n_edges) * sizeof(float) : 0;
+  return bwd_ws_bytes(n_edges, n_edges <= kMergeEdges ? kGroups : 1);
 }
 
 // The four head groups in turn (or merged): the row pass of the group's two slices, then its column pass (clusters
@@ -984,10 +984,9 @@ E2V2_API size_t e2v2_attn_bwd_workspace(int64_t n_edges) {
 template <typename TS, int kMode>
 static int attn_bwd_launch(const e2v2_attn_args& A, const TS* G, const TS* O, const float* mrow, const float* srow,
                            const int32_t* cnt, float* ddvec, float* ddist, float* dq, float* dk, float* dv,
-                           float* ws, hipStream_t s) {
+                           float* ws, bool all, hipStream_t s) {
   const int64_t E = A.n_edges;
-  const int np = bwd_pairs(E);
-  const bool all = np == kGroups;
+  const int np = all ? kGroups : 1;
   float* w_g = ws;
   float* dqk_g = ws + (size_t)E * kGroupHeads * np;
   float* part = ws + (size_t)E * 2 * kGroupHeads * np;
@@ -1021,10 +1020,11 @@ E2V2_API int e2v2_attn_bwd(const e2v2_attn_args* args, const void* grad_out, con
                "attn_bwd: column clusters need span 4 and all three slot arrays (span %d)", A.col_span);
   if (A.n_rows == 0) return 0;
   if (int rc = check_table(A, "attn_bwd")) return rc;
-  const size_t need = e2v2_attn_bwd_workspace(A.n_edges);
+  const size_t need = bwd_ws_bytes(A.n_edges, 1);
   E2V2_REQUIRE(workspace_bytes >= need && (need == 0 || workspace) &&
                    reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
                "attn_bwd: workspace of %zu bytes (16-byte aligned) needed, got %zu", need, workspace_bytes);
+  const bool all = A.n_edges <= kMergeEdges && workspace_bytes >= bwd_ws_bytes(A.n_edges, kGroups);
   float* ws = static_cast<float*>(workspace);
   const auto* Gb = static_cast<const __bf16*>(grad_out);
   const auto* Ob = static_cast<const __bf16*>(out);
@@ -1033,7 +1033,7 @@ E2V2_API int e2v2_attn_bwd(const e2v2_attn_args* args, const void* grad_out, con
   E2V2_REQUIRE(!A.ext_gate || A.ext_dgate, "attn_bwd: the external gate needs ext_dgate for its gradient");
   return with_mode(kernel_mode(A), [&](auto md) -> int {
     constexpr int kM = decltype(md)::value;
-    if (A.act_bf16) return attn_bwd_launch<__bf16, kM>(A, Gb, Ob, mrow, srow, cnt, ddvec, ddist, dq, dk, dv, ws, s);
-    return attn_bwd_launch<float, kM>(A, Gf, Of, mrow, srow, cnt, ddvec, ddist, dq, dk, dv, ws, s);
+    if (A.act_bf16) return attn_bwd_launch<__bf16, kM>(A, Gb, Ob, mrow, srow, cnt, ddvec, ddist, dq, dk, dv, ws, all, s);
+    return attn_bwd_launch<float, kM>(A, Gf, Of, mrow, srow, cnt, ddvec, ddist, dq, dk, dv, ws, all, s);
   });
 }
