@@ -87,3 +87,19 @@ def test_layer_copies_and_pickles_with_its_module(pkg, cuda):
     with torch.no_grad():
         twin.slinear_2.weight.mul_(2.0)
     assert torch.equal(ffn(x), y) and torch.equal(back(x), y) and not torch.equal(twin(x), y)
+
+
+@pytest.mark.parametrize("rows", [8192, 0], ids=["layer_call", "single_calls"])
+def test_ffn_gradient_is_not_differentiated_again_silently(pkg, cuda, monkeypatch, rows):
+    """The fused blocks leave no graph of their gradient: with create_graph=True they raise, as the fused attention
+    does, where a second differentiation would have lost their terms."""
+    from ubio_molfm_amd import modules
+    monkeypatch.setattr(modules, "LAYER_ROWS", rows)
+    m = _model(cuda, {})
+    ffn = next(x for x in m.modules() if type(x).__name__ == "FeedForwardNetwork_s3")
+    x = torch.randn(9, 5, 256, device=cuda, requires_grad=True)
+    g = torch.randn(9, 5, 256, device=cuda)
+    for res, bf16 in ((None, False), (x, False), (None, True)):
+        torch.autograd.grad(ffn(x, res=res, bf16=bf16), x, g)
+        with pytest.raises(NotImplementedError, match="first-order"):
+            torch.autograd.grad(ffn(x, res=res, bf16=bf16), x, g, create_graph=True)

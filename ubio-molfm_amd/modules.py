@@ -1087,6 +1087,7 @@ class FFNS3Fn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gout):
+        _no_double_backward()
         sc, h = ctx.saved_tensors
         gout = gout.contiguous()
         gy = torch.empty_like(h)
@@ -1133,6 +1134,7 @@ class FFNLayerFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gout):
+        _no_double_backward()
         sc, h = ctx.saved_tensors
         gout = gout.contiguous()
         N, dev = h.shape[1], h.device
