@@ -240,3 +240,22 @@ def test_value_aggregation_of_strided_operands_to_third_order(pkg, cuda):
         rel = float((a.double().cpu() - b).norm() / b.norm())
         print(i, f"{rel:.2e}", flush=True)
         assert rel < 10 * TOL
+
+
+def test_value_aggregation_rule(pkg, cuda, monkeypatch):
+    """fp32 at the kernels' sizes takes them; half precision and 64 heads the composition, with the same values."""
+    from ubio_molfm_amd import second_order as so
+    n = 61
+    e, row, col, g = _edges(n, 31, cuda)
+    e.qi = row.to(cuda)
+    calls = []
+    real = so._lib.call
+    monkeypatch.setattr(so._lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    u = torch.randn(e.E, 3, generator=g)
+    for heads, dtype in ((128, torch.float32), (64, torch.float32), (128, torch.bfloat16)):
+        w, v = (torch.randn(*s, generator=g).to(dtype) for s in ((e.E, heads), (9, n, C)))
+        calls.clear()
+        got = so.value_aggregation(w.to(cuda), u.to(cuda, dtype), v.to(cuda), e)
+        assert ("e2v2_so2_agg" in calls) == (heads == 128 and dtype == torch.float32)
+        ref = ref_aggregation(w.double().repeat(1, 128 // heads), u.to(dtype).double(), v.double(), row, col)
+        assert float((got.double().cpu() - ref).norm() / ref.norm()) < (TOL if dtype == torch.float32 else 1e-2)

@@ -5,6 +5,7 @@ first differentiation with create_graph=True, and the second differentiation to
 the inputs and parameters, including a first differentiation that skips the
 weight gradient), the split-K product with rows left over, and run_seq over a
 RadialProfile net (on the CPU every LayerNorm + SiLU pair runs as the modules)."""
+import pytest
 import torch
 
 from ubio_molfm_amd import modules
@@ -50,3 +51,35 @@ def test_run_seq_matches_radial_profile_on_cpu():
     h = torch.randn(300, 64, dtype=torch.float64)
     assert not so.ln_silu_fusable(prof.net[1], h)
     assert torch.equal(so.run_seq(prof.net[1:], h), prof.net[1:](h))
+
+
+class _HostEdges:
+    """The value aggregation of an edge list in plain PyTorch."""
+
+    def __init__(self, row, col, n):
+        self.row, self.col, self.N, self.E = row, col, n, row.numel()
+
+    def v_agg(self, value, alpha):
+        out = torch.zeros(self.N, *value.shape[1:], dtype=value.dtype)
+        return out.index_add(0, self.row, value[self.col] * alpha.unsqueeze(1).to(value.dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,channels,heads", [(9, 256, 128), (9, 128, 128), (9, 256, 64), (4, 256, 128)])
+def test_value_aggregation_of_other_types_and_sizes(monkeypatch, dtype, rows, channels, heads):
+    """The fused kernels take raw pointers and fixed sizes: operands of another type, size or device never reach
+    them and run the composition."""
+    def never(*a):
+        raise AssertionError("the kernel was called")
+    monkeypatch.setattr(so._lib, "call", never)
+    g = torch.Generator().manual_seed(5)
+    n, E = 7, 30
+    row, col = torch.randint(0, n, (2, E), generator=g)
+    w, u, v = (torch.randn(*s, generator=g).to(dtype) for s in ((E, heads), (E, 3), (rows, n, channels)))
+    got = so.value_aggregation(w, u, v, _HostEdges(row, col, n))
+    assert got.shape == (3, rows, n, channels) and got.dtype == dtype
+    t = w.double().repeat(1, channels // heads).unsqueeze(0) * v.double()[:, col]
+    ref = torch.stack([torch.zeros(rows, n, channels, dtype=torch.float64).index_add(1, row, t * u.double()[:, k:k + 1])
+                       for k in range(3)])
+    # up to 30 terms of three factors, each product and sum rounded once in the type
+    assert _rel(got.double(), ref) < 40 * torch.finfo(dtype).eps

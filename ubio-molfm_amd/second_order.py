@@ -879,6 +879,19 @@ class _So2AggGradFn(torch.autograd.Function):
         return dg, dw, du, dv, None
 
 
+def value_aggregation(w, u, v, edges) -> torch.Tensor:
+    """a[k, r, i, c] = sum over the edges of row i of w[e, c mod H] u[e, k] v[r, col_e, c], [3, R, N, C], for w [E, H],
+    u [E, 3], v [R, N, C]: _So2AggFn at the sizes its kernels are built for (fp32 on the GPU, nine rows of 256
+    channels, 128 heads); other inputs three value aggregations."""
+    if (v.is_cuda and all(t.dtype == torch.float32 for t in (w, u, v)) and v.dim() == 3 and w.dim() == u.dim() == 2
+            and (v.shape[0], v.shape[2], w.shape[1], u.shape[1]) == (9, 256, 128, 3) and v.shape[1] == edges.N
+            and w.shape[0] == u.shape[0] == edges.E):
+        return _So2AggFn.apply(w, u, v, edges)
+    R, N, C = v.shape
+    vh = v.permute(1, 0, 2).reshape(N, -1, w.shape[1])                       # channel c -> head c mod H
+    return torch.stack([edges.v_agg(vh, w * u[:, k:k + 1]).reshape(N, R, C).permute(1, 0, 2) for k in range(3)])
+
+
 class _RowMaxFn(torch.autograd.Function):
     """m[i, h] = max over the edges of row i of logit[e, h] (scatter_reduce amax from
     -inf, e2former.py:335-347), with scatter_reduce's gradient -- g[i, h] split evenly
@@ -999,7 +1012,7 @@ def attention(ga, x: torch.Tensor, edges: TrainEdges, rbf: torch.Tensor) -> torc
         vh = v.permute(1, 0, 2).reshape(N, -1, H)                            # channel c -> head c mod H
         agg = edges.v_agg(vh, alpha).reshape(N, -1, C).permute(1, 0, 2)      # [9, N, C]
         return so3_linear(ga.proj_zero, agg)
-    a = _So2AggFn.apply(alpha, edges.unit_vectors(), v, edges)                # [3, 9, N, C], alpha / d * dvec_k
+    a = value_aggregation(alpha, edges.unit_vectors(), v, edges)              # [3, 9, N, C], alpha / d * dvec_k
     so2 = torch.mm(_cartesian(x.device), a.view(27, N * C)).view(-1, N, C)
     return so3_linear(ga.proj_first, so2_forward_linear(ga.first_order_tp.so2_tp, so2))
 
