@@ -259,3 +259,25 @@ def test_value_aggregation_rule(pkg, cuda, monkeypatch):
         assert ("e2v2_so2_agg" in calls) == (heads == 128 and dtype == torch.float32)
         ref = ref_aggregation(w.double().repeat(1, 128 // heads), u.to(dtype).double(), v.double(), row, col)
         assert float((got.double().cpu() - ref).norm() / ref.norm()) < (TOL if dtype == torch.float32 else 1e-2)
+
+
+def test_other_shapes_do_not_reach_the_kernels(pkg, cuda, monkeypatch):
+    """Operands that the list's sizes do not fit are refused by the composition's own checks."""
+    from ubio_molfm_amd import second_order as so
+    e, row, _, g = _edges(5, 33, cuda)
+    e.qi = row.to(cuda)
+    E, n = e.E, e.N
+
+    def never(name, *a):
+        assert not name.startswith(("e2v2_attn_weights", "e2v2_add_gather2")), name
+        return real(name, *a)
+    real = so._lib.call
+    monkeypatch.setattr(so._lib, "call", never)
+    qk, p = torch.randn(E, H, device=cuda), torch.rand(E, device=cuda)
+    for eg, gate in ((torch.randn(E, 192, device=cuda), None), (torch.randn(E, H, device=cuda), None),
+                     (torch.randn(E, 192, device=cuda), qk)):
+        with pytest.raises(RuntimeError):
+            so.attention_weights(eg, gate, qk, p, e, "softmax")
+    for xq in (torch.randn(n, 64, device=cuda), torch.randn(n - 1, H, device=cuda)):
+        with pytest.raises((RuntimeError, ValueError)):
+            e.add_gathers(qk, xq, xq)

@@ -645,7 +645,8 @@ class TrainEdges:
 
     def add_gathers(self, y: torch.Tensor, xq: torch.Tensor, xk: torch.Tensor) -> torch.Tensor:
         """y + xq[qi] + xk[nj], y [E, F], xq and xk [N, F]."""
-        if y.dtype == xq.dtype == xk.dtype == torch.float32 and y.shape[1] % 4 == 0 and y.shape[1] <= 1024:
+        if (y.dtype == xq.dtype == xk.dtype == torch.float32 and y.shape[1] % 4 == 0 and y.shape[1] <= 1024
+                and y.shape[0] == self.E and xq.shape == xk.shape == (self.N, y.shape[1])):
             return _AddGathersFn.apply(y, xq, xk, self)
         return y + self.gather_q(xq) + self.gather_k(xk)
 
@@ -924,9 +925,10 @@ def attention_weights(eg, gate, qk, p, edges: TrainEdges, form: str) -> torch.Te
     and inputhead side by side; with ``gate`` given, eg [E, H] is the inputhead.
     fp32 on the GPU with 128 heads takes the softmax through _AttnWeightsFn;
     other inputs the composition."""
-    H = qk.shape[1]
+    H, E = qk.shape[1], edges.E
     if (form == "softmax" and H == 128 and qk.is_cuda and all(t.dtype == torch.float32 for t in (eg, qk, p))
-            and (gate is None or gate.dtype == torch.float32)):
+            and (gate is None or (gate.dtype == torch.float32 and gate.shape == qk.shape))
+            and eg.shape == (E, 256 if gate is None else 128) and qk.shape[0] == E and p.shape == (E,)):
         # (QKdotS_alpha's inputhead is a half of a wider tensor's columns: dense here, so that no pass copies it again)
         return _AttnWeightsFn.apply(eg.contiguous(), gate, qk, p, edges)
     if form == "softmax":
