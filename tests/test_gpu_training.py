@@ -365,3 +365,47 @@ def test_eval_mode_keeps_the_fused_path(pkg, cuda):
     e, _ = m.energy_flat(p, Z, s["graph_ptr"], s["cell"], s["pbc"])
     with pytest.raises(NotImplementedError):
         torch.autograd.grad(e.sum(), p, create_graph=True)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_training_embedding_that_is_not_finite_stays_with_its_element(pkg, cuda, value):
+    """A batch of two molecules, the carbon embedding rows infinite or NaN: the molecule without carbon has the energy
+    and forces it has alone beside finite rows."""
+    m, _ = _pair(cuda, 41)
+    rng = np.random.default_rng(3)
+    n = 9
+    pos = torch.as_tensor(np.concatenate([rng.random((n, 3)) * 4, rng.random((n, 3)) * 4]), dtype=torch.float32,
+                          device=cuda)
+    Z = torch.as_tensor([6, 1, 1, 6, 8, 1, 1, 8, 6] + [8, 1, 1, 8, 1, 1, 7, 1, 1], device=cuda)
+    call = (pos, Z, np.array([0, n, 2 * n]), np.zeros((2, 3, 3)), np.zeros((2, 3), bool))
+    e0, f0, _ = m.energy_forces_flat(*call)
+    with torch.no_grad():
+        for name, p in m.named_parameters():
+            if name.endswith(("source_embedding.weight", "target_embedding.weight")):
+                p[6] = value
+    e, f, _ = m.energy_forces_flat(*call)
+    assert not bool(e[0].isfinite()) and bool(f0.isfinite().all())
+    assert torch.equal(e[1], e0[1]) and torch.equal(f[n:], f0[n:])
+
+
+def test_training_rows_of_types(pkg, cuda):
+    """TrainEdges.type_rows: the row of each atom's type, its gradient the sum over the type's atoms (any order), types
+    without an atom among them.  Sums of up to 700 terms: 2-norm 1e-6 of float64's."""
+    from ubio_molfm_amd import second_order as so
+    g = torch.Generator().manual_seed(1)
+    n, T, F = 700, 5, 128
+    a = torch.randint(0, T - 1, (n,), generator=g)
+    a[a == 2] = 3
+    e = so.TrainEdges.__new__(so.TrainEdges)
+    e.N, e.atom_type, e.type_z, e._types = n, a.to(cuda), torch.arange(T, device=cuda), None
+    x, r = torch.randn(T, F, generator=g), torch.randn(n, F, generator=g)
+
+    def chain(f, x, r):
+        x = x.clone().requires_grad_(True)
+        y = f(x)
+        d, = torch.autograd.grad((y.pow(3) * r).sum(), x, create_graph=True)
+        return [t.detach() for t in (y, d, torch.autograd.grad(d.pow(2).sum(), x)[0])]
+    got = chain(e.type_rows, x.to(cuda), r.to(cuda))
+    for p, q in zip(got, chain(lambda t: t[a], x.double(), r.double())):
+        assert _rel(p, q) < 1e-6
+    assert torch.equal(got[0].cpu(), x[a]) and not bool(got[1][2].any())

@@ -578,7 +578,7 @@ class TrainEdges:
         self.dist = self.dvec.norm(dim=-1)
         self._unit = self._env = None
         self.type_z, self.atom_type = ctx.type_z.long(), ctx.atom_type.long()
-        self._hot = None
+        self._types = None
         self.offset, self.coeff = ctx.rbf_offset, float(ctx.rbf_coeff)
         self.env_kind, self.env_lo = ctx.env_kind, ctx.env_lo
         eid = torch.arange(E, dtype=torch.int32, device=pos.device)
@@ -592,14 +592,16 @@ class TrainEdges:
         t = (self.nl.row_ptr, self.col32, self.row32, self.nl.key_ptr, self.md[5])
         return C.byref(_lib.TrainEdges(self.N, self.E, *[x.data_ptr() if x.numel() else None for x in t]))
 
-    def type_rows(self, dtype) -> torch.Tensor:
-        """[N, T] selecting each atom's type: a product with it expands per-type rows to the atoms, and its
-        transpose sums their gradients (an embedding's gradient walks the atoms of a type one by one: 110 us a
-        profile for 1500 atoms), formed once for all layers."""
-        if self._hot is None or self._hot.dtype != dtype:
-            types = torch.arange(self.type_z.numel(), device=self.type_z.device)
-            self._hot = (self.atom_type[:self.N].view(-1, 1) == types).to(dtype)
-        return self._hot
+    def type_rows(self, x: torch.Tensor) -> torch.Tensor:
+        """x [T, F] -> the row of each atom's type [N, F], its gradient summed by the atoms of each type (segments formed
+        once for all layers; an embedding's own gradient walks the atoms of a type one by one: 110 us a profile for 1500
+        atoms).  A row gather, so that a row that is not finite stays with its type's atoms."""
+        if self._types is None:
+            types, order = torch.sort(self.atom_type[:self.N], stable=True)
+            bounds = torch.arange(self.type_z.numel() + 1, device=types.device, dtype=types.dtype)
+            self._types = (self.atom_type[:self.N].int(), torch.searchsorted(types, bounds, out_int32=True), order.int())
+        index, ptr, atoms = self._types
+        return sparse_ops.sparse_gather_edge_index(x, index, self.type_z.numel(), (ptr, atoms))
 
     def unit_vectors(self) -> torch.Tensor:
         """dvec / max(dist, 1e-6) [E, 3], formed once for all layers."""
@@ -688,9 +690,8 @@ class EdgeInput:
         K, ne = self.rbf.shape[1], self.tgt.weight.shape[1]
         W = lin1.weight
         e = self.edges
-        hot = e.type_rows(W.dtype)                               # per type, then per atom [N, hidden]
-        ht = hot @ (self.tgt(e.type_z) @ W[:, K:K + ne].t())
-        hs = hot @ (self.src(e.type_z) @ W[:, K + ne:K + 2 * ne].t())
+        ht = e.type_rows(self.tgt(e.type_z) @ W[:, K:K + ne].t())      # per type, then per atom [N, hidden]
+        hs = e.type_rows(self.src(e.type_z) @ W[:, K + ne:K + 2 * ne].t())
         h = e.add_gathers(_EdgeLinearFn.apply(self.rbf, W[:, :K], lin1.bias), ht, hs)
         return run_seq(net[1:], h)
 
