@@ -191,8 +191,8 @@ int e2v2_pair_emit(const e2v2_pair_plan* plan, const int32_t* row_ptr, int64_t n
 /* The segment layout of the reference's Triton kernels: slot p of row r (row_ptr[r] <= p <
    row_ptr[r+1]) carries edge alpha_index[p] and partner row col_index[p].  Slots whose partner row is
    outside [0, n_cols) or whose edge is outside [0, n_edges) are skipped; row bounds are clamped to
-   [0, n_slots].  Rows are summed in slot order by one workgroup each (deterministic).  Operands are
-   fp32 with element strides: a logical [rows, H, D] operand A has A[r, h, d] at r s[0] + h s[1] + d s[2]. */
+   [0, n_slots].  Rows are summed by one workgroup each in an order fixed by the sizes (deterministic).  Operands
+   are fp32 with element strides: a logical [rows, H, D] operand A has A[r, h, d] at r s[0] + h s[1] + d s[2]. */
 typedef struct e2v2_segments {
   const int32_t* row_ptr;           /* [n_rows + 1]                                                     */
   const int32_t* col_index;         /* [n_slots] (may be NULL where no partner operand is read)          */
@@ -629,8 +629,8 @@ typedef struct {
   int c_bf16;           /* 1: c is written as bf16 (rounded once from the fp32 result) */
 } e2v2_gemm_args;
 int e2v2_gemm_s3(const e2v2_gemm_args* args, hipStream_t s);
-/* e2v2_gemm_s3 with every row summed in the same order whatever the number of rows m (e2v2_gemm_s3 takes other
- * tiles, which split the sum over k, for matrices of few rows): for operands whose row count is a capacity, so
+/* e2v2_gemm_s3 with every row summed in the same order whatever the number of rows m (with three pieces
+ * e2v2_gemm_s3 splits the sum over k for matrices of few rows; with one piece its order is this one's): for operands whose row count is a capacity, so
  * that padding rows change no value. */
 int e2v2_gemm_s3_padded(const e2v2_gemm_args* args, hipStream_t s);
 /* Up to four independent GEMMs (each as e2v2_gemm_s3, with its own shapes, operands and packed weight) in one

@@ -1,6 +1,7 @@
-"""The K-split tiles of the split GEMMs (matrices of few rows) at their edges: row counts around the 32-row
-tile and around the switch to the 128 x 128 tiles, K from one 16-k stage (three of the four wavefronts idle)
-over stage counts that do not divide by four, every operand form; and the Q/K projection likewise.
+"""The few-row tiles of the split GEMMs at their edges: row counts around the 32-row tile and around the switch to
+the 128 x 128 tiles, K from one 16-k stage (three of the four wavefronts that split it idle) over stage counts
+that do not divide by four, every operand form; and the Q/K projection likewise.  The one-piece forms, which do
+not split K, bitwise between few and many rows.
 
 Error over the GEMM's own scale sum_k |a| |b|, as in test_gpu_gemm.py: at most 8 units of 2^-24 times
 max(sqrt(k), 4) (the sums are of at least six fp32-rounded terms per 16 k); one-piece (bf16) operands against
@@ -117,7 +118,8 @@ def _same_rows(few, many, at, m):
     assert torch.equal(few, many[..., at:at + m, :])
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 128, 16), (33, 256, 144), (700, 512, 256), (2500, 256, 512)])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 16), (33, 256, 144), (700, 512, 256), (2500, 256, 512),
+                                   (768, 128, 48), (1024, 128, 48), (1536, 128, 48)])
 @pytest.mark.parametrize("form", ["fp32 A", "bf16 A", "gated"])
 def test_one_piece_rows_do_not_depend_on_the_call(pkg, cuda, m, n, k, form):
     """bf16 mode: a row's result is bitwise the same among few rows as among many, alone and in a group (a sum in

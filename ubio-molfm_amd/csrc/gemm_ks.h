@@ -57,8 +57,7 @@ __device__ __forceinline__ void ks_mfma(const bf16x8 (&a)[kP], const bf16x8 (&b)
 // acc[i][j] += the sum over stages [ks0, ks1) of the row tile i (32 rows) times the column subtile j.  Raw: one row
 // tile's A registers of a stage, loaded by load_a(ks, i, raw) and turned into pieces by split(ks, i, raw, a).
 // boff[j]: the lane's byte offset of subtile j in a piece of stage 0.  A ring of kD stages' registers, each
-// slot refilled as soon as it is consumed; loads past ks1 stay inside the buffers (bound by their resources)
-// and are never used.
+// slot refilled as soon as it is consumed; no load past ks1 is issued.
 template <int kP, int kR, int kJ, int kD, typename Raw, typename LoadA, typename Split>
 __device__ __forceinline__ void ks_loop(__amdgpu_buffer_rsrc_t br, const uint32_t (&boff)[kJ], int ks0, int ks1,
                                         LoadA&& load_a_, Split&& split, floatx16 (&acc)[kR][kJ]) {
